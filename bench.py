@@ -6,10 +6,10 @@ same run on the same resident particles:
   fp32     plain FP32 cross terms (the parity path)
   fp16x3   split-precision cross terms (FP16 hi+lo on MFMA, FP32 accumulate, FP64 normalisation)
   fp16x2   the dense coarse cross term with 2 MFMA products (FP16 hi+lo images x FP16 hi
-           references); the fine pass and every other cross term as fp16x3. Global split-precision
-           searches take the pruned coarse pass by default: a one-product bounds GEMM over the
-           low-frequency prefix of the coarse pixels, then the full GEMM only on tiles not beyond
-           the negligible-weight cut (identical outputs)
+           references); the fine pass and every other cross term as fp16x3
+           (Global searches of every precision take the pruned coarse pass by default: an INT8
+           bounds GEMM over the low-frequency coarse pixels, then the full GEMM only on tiles not
+           beyond the negligible-weight cut, with identical outputs.)
   fp16x2+exhaustive  the same with the coarse GEMM over every tile (coarse_exhaustive 1)
   fp16x2+graph  the same, each batch's launches after its preprocessing captured once per batch
            size as a hipGraph and replayed (reported beside the eager paths)
@@ -705,18 +705,18 @@ def main():
         # actually did is reported beside it
         f_kept = 1.0 - st.coarse_tiles_pruned / st.coarse_tiles_checked
         exec_pairs = (st.coarse_bound_flop + flop_total * f_kept) / launches
-        exec_products = (st.coarse_bound_flop * 1 + flop_total * f_kept * nprod) / launches
+        # matrix-core time of the executed work at the dense peaks (INT8 bounds: 5 POP/s)
+        exec_ms = (st.coarse_bound_flop / 5000e9 + flop_total * f_kept * nprod / (peak * 1e9)) / launches
         roof.update({
-            "kernel": ("coarse diff2 cross term, pruned pass: k_gemm_x3p<f16, 1, 4> (bounds: 1 FP16 product over "
-                       "the low-frequency prefix of the coarse pixels, two K chunks per LDS stage, block minima only) "
-                       "+ k_prune_c + k_prune_seed + k_prune_plan + "
-                       f"k_gemm_x3p<LIST> ({nprod} products, persistent over the 256x256 tiles not beyond the "
-                       "negligible-weight cut)"),
+            "kernel": ("coarse diff2 cross term, pruned pass: k_prune_quant_a + k_prune_base + k_gemm_i8_bounds (INT8 "
+                       "over the low-frequency coarse pixels, block minima only) + k_prune_seed + k_prune_plan + "
+                       + ("k_gemm_tn<LIST> (FP32" if hb == "fp32" else f"k_gemm_x3<LIST> ({nprod} products") +
+                       ", persistent over the 128x128 tiles not beyond the negligible-weight cut)"),
             "achieved_convention": ("effective: the exhaustive pass's algorithmic flops per batch over the pruned "
                                     "stage's time per batch (same outputs)"),
             "tiles_pruned_fraction": 1.0 - f_kept,
             "executed_flop_per_launch": exec_pairs,
-            "executed_mfma_product_utilisation": exec_products / (avg_ms * 1e-3) / 1e12 / peak if avg_ms > 0 else 0.0,
+            "executed_mfma_utilisation": exec_ms / avg_ms if avg_ms > 0 else 0.0,
         })
         del roof["mfma_product_utilisation"]
     configure(cfg, head)

@@ -14,7 +14,7 @@ OUT_DIR = os.path.join(HERE, "lib")
 BUILD_DIR = os.path.join(HERE, "_build")
 LIB = os.path.join(OUT_DIR, "libt2x.so")
 
-SOURCES = ["t2x_device.hip", "t2x_sampling.cpp", "t2x_gemm.hip", "t2x_select.hip",
+SOURCES = ["t2x_device.hip", "t2x_sampling.cpp", "t2x_gemm.hip", "t2x_prune.hip", "t2x_select.hip",
            "t2x_estep.hip", "t2x_synth.hip", "t2x_recon.hip",
            "t2x_cnn.hip", "t2x_proposal.hip", "t2x_io.cpp"]
 

@@ -43,13 +43,9 @@ int launch_gemm_x3(int prec, int epi, const void* Ah, const void* Al, const floa
                    long long a_rows, const void* Bh, const void* Bl, const float* Bs, long long ldb, int K,
                    int Mrows_pad, int Nrows_pad, const EpiParams& ep, hipStream_t st, GemmChoice want,
                    const int* rowmap, GemmChoice* used);
-int launch_gemm_h1_bounds(const void* Ah, const float* As, long long lda, long long a_rows, const void* Bh,
-                          const float* Bs, long long ldb, int K, int Mrows_pad, int Nrows_pad, const EpiParams& ep,
-                          hipStream_t st);
-int launch_gemm_pruned(int prec, const void* Ah, const void* Al, const float* As, long long lda, long long a_rows,
-                       const void* Bh, const void* Bl, const float* Bs, long long ldb, int K, int Mrows_pad,
-                       int Nrows_pad, const EpiParams& ep, const float* lb, const float* seed, unsigned* list,
-                       long long list_cap, unsigned* count, int n_cu, hipStream_t st);
+int launch_gemm_pruned(int prec, const void* Ah, const void* Al, const float* As, long long lda, const void* Bh,
+                       const void* Bl, const float* Bs, long long ldb, int K, int Mrows_pad, int Nrows_pad,
+                       const EpiParams& ep, const unsigned* list, const unsigned* count, int n_cu, hipStream_t st);
 int launch_gemm_local_x3(int prec, const void* Sh, const void* Sl, const float* Ss, const void* Wh, const void* Wl,
                          const float* Ws, long long ld, int K, const int2* items, int n_items, int T,
                          const long long* orient_off, const int* rowu, const double* cb, const double* n1,
@@ -1938,111 +1934,6 @@ __global__ void k_gather_ccoarse(const PartScalars* __restrict__ ps, int B, doub
     if (i < B) out[i] = ps[i].C_coarse;
 }
 
-// Pruned coarse pass, the bounds pass's N1 term. The coarse diff2 over the pixels beyond the
-// low-frequency prefix (the high set h) is 1/2 sum_h minv |ctf F - X|^2 = Ch + N1h - G_h, with
-// Ch = 1/2 sum_h minv |X|^2 (C_coarse - C_low, the constant highres term cancelling), N1h =
-// 1/2 sum_h minv ctf^2 |F|^2 and G_h = sum_h minv Re(ctf F conj X); Cauchy-Schwarz bounds
-// G_h <= 2 sqrt(N1h Ch). So C_b + N1 - G_low - 2 sqrt(N1h Ch) is a lower bound of the full diff2,
-// and the bounds GEMM over the prefix gets it with N1 - 2 sqrt(N1h Ch) as its N1. The factor
-// 1 + 2^-8 covers the split operands' rounding (the FP16 reference side's 2^-11 relative) and the
-// FP32 sums. A bounds GEMM of one FP16 product per element (A hi . B hi) drops A lo . B hi (and,
-// under FP16X3, A hi . B lo): each |A lo| <= 2^-11 |A| (the rows are scaled to a maximum in
-// [0.5, 1), so normal FP16 but for negligible elements), so the dropped sum is at most
-// 2 . 2^-11 . sum |A||B| <= 2^-10 . 2 sqrt(N1 Cl), Cl = C_low - highres/2 the image energy of the
-// prefix (Cauchy-Schwarz again); eps1 = 2^-9 allows twice that, for the FP32 sums of both
-// passes. eps1 = 0 for a bounds GEMM in the full split precision. The GEMM's epilogue forms
-// N1 - c0 sqrt(N1h) - c1 sqrt(N1) where it reads N1 (N1h from its GEMM over the high set); this
-// kernel gives each particle's c0 = 2 (1 + 2^-8) sqrt(Ch) and c1 = 2 eps1 sqrt(Cl).
-__global__ void k_prune_c(const PartScalars* __restrict__ ps, int B, double eps1, double* __restrict__ c)
-{
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= B) return;
-    const double ch = fmax(ps[b].C_coarse - ps[b].C_low, 0.);
-    const double cl = fmax(ps[b].C_low - ps[b].highres_Xi2 / 2., 0.);
-    c[2 * b] = 2. * (1. + 1. / 256.) * sqrt(ch);
-    c[2 * b + 1] = 2. * eps1 * sqrt(cl);
-}
-
-// Pruned coarse pass: per particle an upper bound of its coarse minimum diff2, the full diff2 of
-// the 64 columns of the (row, block) whose low-frequency bound is smallest (where the minimum
-// most likely lies), recomputed from the split operands in FP32 (the GEMM's products and scales,
-// summed in another order), plus a margin of 1 + 1e-4 |d| for that order; +inf where the
-// particle has no scored column. It seeds the pruning test and the lazy stores' running minima.
-template <class H>
-__global__ __launch_bounds__(256) void k_prune_seed(const float* __restrict__ lb, int lb_ld, int nblk, int T,
-                                                    const H* __restrict__ Ah, const H* __restrict__ Al,
-                                                    const float* __restrict__ As, const H* __restrict__ Bh,
-                                                    const H* __restrict__ Bl, const float* __restrict__ Bs,
-                                                    long long ld, int K, const double* __restrict__ Cb,
-                                                    const float* __restrict__ N1, long long ldn,
-                                                    const double* __restrict__ prior_o, long long N,
-                                                    float* __restrict__ seed, unsigned int* __restrict__ pmin)
-{
-    __shared__ float sv[256];
-    __shared__ long long si[256];
-    __shared__ float sd[64];
-    const int b = blockIdx.x, tid = threadIdx.x;
-    float best = 3.0e38f;
-    long long bi = -1;
-    // the particle's T rows of bounds, four blocks per load (lb_ld is a multiple of 4; blocks at
-    // or beyond nblk are padding)
-    const int w4 = lb_ld / 4;
-    for (long long q4 = tid; q4 < (long long)T * w4; q4 += blockDim.x) {
-        const long long t = q4 / w4;
-        const int k = (int)(q4 - t * w4) * 4;
-        const float4 v = *reinterpret_cast<const float4*>(lb + ((long long)b * T + t) * lb_ld + k);
-        const float vv[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-        for (int e = 0; e < 4; e++)
-            if (k + e < nblk && vv[e] < best) { best = vv[e]; bi = t * nblk + k + e; }
-    }
-    sv[tid] = best;
-    si[tid] = bi;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (tid < w && sv[tid + w] < sv[tid]) { sv[tid] = sv[tid + w]; si[tid] = si[tid + w]; }
-        __syncthreads();
-    }
-    const long long q = si[0];
-    if (q < 0) {
-        if (tid == 0) { seed[b] = __builtin_inff(); pmin[b] = float_to_ordered(__builtin_inff()); }
-        return;
-    }
-    const long long r = (long long)b * T + q / nblk;
-    const int c = tid >> 2, part = tid & 3;
-    const long long n = (q % nblk) * 64 + c;
-    float acc = 0.f;
-    if (n < N) {
-        const H* ah = Ah + r * ld;
-        const H* al = Al + r * ld;
-        const H* bh = Bh + n * ld;
-        const H* bl = Bl ? Bl + n * ld : nullptr;
-        for (int k = part; k < K; k += 4) {
-            const float av = (float)ah[k] + (float)al[k];
-            const float bv = bl ? (float)bh[k] + (float)bl[k] : (float)bh[k];
-            acc += av * bv;
-        }
-    }
-    acc += __shfl_xor(acc, 1);
-    acc += __shfl_xor(acc, 2);
-    if (part == 0) {
-        float d = 3.0e38f;
-        if (n < N && prior_o[n] > 0.) {
-            const float v = acc * (As ? As[r] : 1.f) * (Bs ? Bs[n] : 1.f);
-            d = (float)(Cb[b] + (double)N1[(long long)b * ldn + n] - (double)v);
-        }
-        sd[c] = d;
-    }
-    __syncthreads();
-    if (tid == 0) {
-        float m = 3.0e38f;
-        for (int k = 0; k < 64; k++) m = fminf(m, sd[k]);
-        const float sdv = m < 3.0e38f ? m + 1.f + 1e-4f * fabsf(m) : __builtin_inff();
-        seed[b] = sdv;
-        pmin[b] = float_to_ordered(sdv);
-    }
-}
-
 // ------------------------------------------------------------------------------------------
 // Local angular searches: HealpixSampling::selectOrientationsWithNonZeroPriorProbability
 // (healpix_sampling.cpp:769-1145) for C1, without bimodal psi or multi-body terms, sigma_cutoff 3,
@@ -2770,6 +2661,23 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
         lsp.sig_psi = cfg->sigma_psi;
     }
 
+    // ---- pruned coarse pass (t2x_prune.hip): global searches without the proposal or diagnostics ----
+    // The low set: the (|frequency|-ordered) coarse pixels within 0.80 of the coarse radius, filled up
+    // to whole K steps of the INT8 GEMM.
+    int n_low = 0, K8 = 0;
+    const bool prune_force = getenv("T2X_PRUNE_FORCE") != nullptr;   // tests: every batch, whatever it prunes
+    bool prune_call = !cfg->coarse_exhaustive && !local && !use_prop && !(dbg && dbg->n_debug > 0);
+    if (prune_call) {
+        double frac = 0.80;
+        const char* env_pr = getenv("T2X_PRUNE_RADIUS");   // fraction of the coarse radius
+        if (env_pr && atof(env_pr) > 0.) frac = atof(env_pr);
+        const double rl = frac * (cc / 2.0);
+        while (n_low < tc.npix && tc.h_x[n_low] * tc.h_x[n_low] + tc.h_y[n_low] * tc.h_y[n_low] <= rl * rl) n_low++;
+        K8 = (int)std::min<long long>(round_up(2LL * n_low, 128), 16384);   // 16,384: the image side's LDS row
+        n_low = std::min(tc.npix, K8 / 2);
+        if (n_low < 16) prune_call = false;
+    }
+
     // ---- coarse projections, cached across calls ----
     const int Kc = tc.npix_pad * 2;            // GEMM K (re/im)
     const int Kn = tc.npix_pad;                // N1 GEMM K
@@ -2826,6 +2734,15 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
         }
         T2X_HIP(hipStreamSynchronize(st));
         d->coarse_key = key;
+        d->prune_key.clear();
+    }
+    if (prune_call) {
+        const std::string pkey = key + "/" + std::to_string(n_low);
+        if (pkey != d->prune_key) {
+            d->prune_key.clear();
+            T2X_TRY(prune_prepare_refs(d, O_all, O_pad, Kc, Kn, n_low, K8, st));
+            d->prune_key = pkey;
+        }
     }
     (void)hipEventRecord(d->ev[1], st);
     {
@@ -2902,23 +2819,6 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
     stt.P_coarse = tc.npix;
     stt.P_fine = tf.npix;
 
-    // ---- pruned coarse pass: the low-frequency prefix of the (|frequency|-ordered) coarse pixels ----
-    // (global searches in a split precision, without the proposal or diagnostics). The prefix holds
-    // the pixels within 0.82 of the coarse radius (two thirds of them), rounded up to 32 pixels.
-    int K_low = 0;
-    bool prune_call = !cfg->coarse_exhaustive && prec != T2X_PREC_FP32 && !local && !use_prop &&
-                      !(dbg && dbg->n_debug > 0);
-    if (prune_call) {
-        double frac = 0.82;
-        const char* env_pr = getenv("T2X_PRUNE_RADIUS");   // fraction of the coarse radius
-        if (env_pr && atof(env_pr) > 0.) frac = atof(env_pr);
-        const double rl = frac * (cc / 2.0);
-        int n_low = 0;
-        while (n_low < tc.npix && tc.h_x[n_low] * tc.h_x[n_low] + tc.h_y[n_low] * tc.h_y[n_low] <= rl * rl) n_low++;
-        K_low = (int)round_up(2LL * n_low, 64);
-        if (n_low < 16 || K_low >= Kc - 64) prune_call = false;
-    }
-
     // ---- brick backprojection: the call's work units and buffers ----
     const bool bp_bricks = !cfg->bp_direct && K <= BP_KMAX;
     long long bp_item_cap = 0;
@@ -2981,9 +2881,14 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
 
     for (int b0 = 0; b0 < n; b0 += Bmax) {
         const int B = std::min(Bmax, n - b0);
-        const bool prune_batch = prune_call;   // the pruned coarse pass for this batch
-        // its full GEMM's tiles (the 256x256 tiles of k_gemm_x3p), known here for graph replays too
-        const long long prune_ntiles = prune_batch ? (round_up((long long)B * T, 256) / 256) * (O_pad / 256) : 0;
+        // the pruned coarse pass for this batch: its ten launches and the bounds GEMM pay where the
+        // exhaustive GEMM takes longer than about 0.15 ms (110 TFLOP/s in FP32, 1,150 TFLOP/s a product)
+        const double gemm_flop = 4. * (double)T * (double)O_all * (double)tc.npix * B;
+        const double gemm_rate = prec == T2X_PREC_FP32 ? 110e12 : (prec == T2X_PREC_FP16X2 ? 575e12 : 383e12);
+        const bool prune_batch = prune_call && (prune_force || gemm_flop > 1.5e-4 * gemm_rate);
+        // its full GEMM's tiles, known here for graph replays too
+        const long long prune_ntiles =
+            prune_batch ? (round_up((long long)B * T, 256) / PRUNED_TILE) * (O_pad / PRUNED_TILE) : 0;
         const size_t NN = (size_t)N * N;
         int ev = 0;
         (void)hipEventRecord(d->ev[ev++], st);
@@ -3382,18 +3287,6 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
                                            d->coarse_B2h.ptr, d->coarse_B2l.ptr, d->coarse_B2s.as<float>(), Kn, Kn,
                                            (int)B_pad, (int)O_pad, ep, st,
                                            GemmChoice{cfg->gemm_tile, cfg->gemm_group}, nullptr, nullptr));
-                    if (prune_batch) {   // N1h: the same over the pixels beyond the low-frequency prefix
-                        T2X_TRY(d->prune_n1.ensure(sizeof(float) * B_pad * O_pad));
-                        EpiParams el = ep;
-                        el.C = d->prune_n1.as<float>();
-                        const int k0 = K_low / 2;   // a multiple of 32 elements: 64-byte aligned rows
-                        T2X_TRY(launch_gemm_x3(prec == T2X_PREC_FP16X2 ? T2X_PREC_FP16X3 : prec, EPI_STORE,
-                                               (const uint16_t*)d->A1h.ptr + k0, (const uint16_t*)d->A1l.ptr + k0,
-                                               d->A1s.as<float>(), Kn, B_pad, (const uint16_t*)d->coarse_B2h.ptr + k0,
-                                               (const uint16_t*)d->coarse_B2l.ptr + k0, d->coarse_B2s.as<float>(),
-                                               Kn, Kn - k0, (int)B_pad, (int)O_pad, el, st,
-                                               GemmChoice{cfg->gemm_tile, cfg->gemm_group}, nullptr, nullptr));
-                    }
                 }
                 if (local) {
                     const long long ne = (long long)B * O_all;
@@ -3482,59 +3375,35 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
                 k_fill_f32<<<(unsigned)((M_pad * rowmin_ld + 255) / 256), 256, 0, st>>>(d_rowmin.as<float>(), 3.0e38f,
                                                                                         M_pad * rowmin_ld);
                 if (prune_batch) {
-                    // 1. bounds: block minima of C_b + N1 - G_low - 2 sqrt(N1h Ch), the cross term over
-                    //    the first K_low columns and the rest bounded by Cauchy-Schwarz, no values stored
+                    // bounds, seeds and the list of the tiles to compute; a tile that is not keeps +inf minima
                     k_const_term<<<B, 256, 0, st>>>(d->Fimg_cur.as<float2>(), Pw, tc.d_win.as<int>(),
-                                                    tc.d_minv.as<float>(), tc.npix, d_ps, 2,
-                                                    std::min(K_low / 2, tc.npix));
-                    // one FP16 product per element unless the precision is BF16X3 (whose dropped
-                    // terms would cost 2^-7 of the bound) or the full split is asked for
-                    const char* env_fb = getenv("T2X_PRUNE_FULL_BOUNDS");
-                    const bool h1 = prec != T2X_PREC_BF16X3 && !(env_fb && atoi(env_fb) != 0);
-                    T2X_TRY(d->prune_c.ensure(sizeof(double) * 2 * B));
-                    k_prune_c<<<(unsigned)((B + 255) / 256), 256, 0, st>>>(d_ps, B, h1 ? 1. / 512. : 0.,
-                                                                           d->prune_c.as<double>());
+                                                    tc.d_minv.as<float>(), tc.npix, d_ps, 2, n_low);
                     T2X_HIP(hipGetLastError());
-                    // the bounds go into the block minima themselves: a pruned tile keeps them, a
-                    // kept tile's full GEMM overwrites them
-                    EpiParams eb = ep;
-                    eb.C = nullptr;
-                    eb.N1h = d->prune_n1.as<float>();
-                    eb.prune_c = d->prune_c.as<double>();
-                    eb.pmin = nullptr;
-                    if (h1)
-                        T2X_TRY(launch_gemm_h1_bounds(d->Ah.ptr, d->As.as<float>(), Kc, M_pad, d->coarse_Bh.ptr,
-                                                      d->coarse_Bs.as<float>(), Kc, K_low, (int)M_pad, (int)O_pad,
-                                                      eb, st));
-                    else
-                        T2X_TRY(launch_gemm_x3(prec, EPI_DIFF2, d->Ah.ptr, d->Al.ptr, d->As.as<float>(), Kc, M_pad,
-                                               d->coarse_Bh.ptr, d->coarse_Bl.ptr, d->coarse_Bs.as<float>(), Kc, K_low,
-                                               (int)M_pad, (int)O_pad, eb, st,
-                                               GemmChoice{cfg->gemm_tile, cfg->gemm_group}, nullptr, nullptr));
-                    // 2. seeds: per particle the full diff2 of its most promising block (also the lazy
-                    //    stores' starting minima)
-                    T2X_TRY(d->prune_seed.ensure(sizeof(float) * B));
-                    const int nblk = (int)((O_all + 63) / 64);
-                    if (prec == T2X_PREC_BF16X3)
-                        k_prune_seed<__bf16><<<B, 256, 0, st>>>(
-                            d_rowmin.as<float>(), rowmin_ld, nblk, (int)T, (const __bf16*)d->Ah.ptr,
-                            (const __bf16*)d->Al.ptr, d->As.as<float>(), (const __bf16*)d->coarse_Bh.ptr,
-                            (const __bf16*)d->coarse_Bl.ptr, d->coarse_Bs.as<float>(), Kc, Kc, ep.Cb, ep.N1, O_pad,
-                            ep.prior_o, O_all, d->prune_seed.as<float>(), d->pmin.as<unsigned>());
-                    else
-                        k_prune_seed<_Float16><<<B, 256, 0, st>>>(
-                            d_rowmin.as<float>(), rowmin_ld, nblk, (int)T, (const _Float16*)d->Ah.ptr,
-                            (const _Float16*)d->Al.ptr, d->As.as<float>(), (const _Float16*)d->coarse_Bh.ptr,
-                            prec == T2X_PREC_FP16X2 ? nullptr : (const _Float16*)d->coarse_Bl.ptr,
-                            d->coarse_Bs.as<float>(), Kc, Kc, ep.Cb, ep.N1, O_pad, ep.prior_o, O_all,
-                            d->prune_seed.as<float>(), d->pmin.as<unsigned>());
-                    T2X_HIP(hipGetLastError());
-                    // 3. the full pass computes the tiles with a block not beyond the cut (below)
-                    T2X_TRY(d->prune_cnt.ensure(sizeof(unsigned)));
-                    T2X_TRY(zero_async(d->prune_cnt.ptr, sizeof(unsigned), st));
-                    T2X_TRY(d->prune_list.ensure(sizeof(unsigned) * prune_ntiles));
-                }
-                if (prec == T2X_PREC_FP32) {
+                    T2X_TRY(d->prune.cnt.ensure(sizeof(unsigned) * 2));
+                    T2X_TRY(zero_async(d->prune.cnt.ptr, sizeof(unsigned) * 2, st));
+                    PruneCall pc{};
+                    pc.prec = prec;
+                    pc.B = B;
+                    pc.T = (int)T;
+                    pc.M_pad = M_pad;
+                    pc.O_all = O_all;
+                    pc.O_pad = O_pad;
+                    pc.Kn = Kn;
+                    pc.n_low = n_low;
+                    pc.K8 = K8;
+                    pc.Cb = ep.Cb;
+                    pc.force = prune_force;
+                    T2X_TRY(prune_bounds(d, pc, d_ps, tc, Pw, st));
+                    const bool f32 = prec == T2X_PREC_FP32;
+                    T2X_TRY(launch_gemm_pruned(prec, f32 ? d->A.ptr : d->Ah.ptr, d->Al.ptr, d->As.as<float>(), Kc,
+                                               f32 ? d->coarse_B.ptr : d->coarse_Bh.ptr, d->coarse_Bl.ptr,
+                                               d->coarse_Bs.as<float>(), Kc, Kc, (int)M_pad, (int)O_pad, ep,
+                                               d->prune.list.as<unsigned>(), d->prune.cnt.as<unsigned>(), d->n_cu, st));
+                    if (!f32) {   // group 0: the tile list
+                        d->stats.s.gemm_tile_used = PRUNED_TILE;
+                        d->stats.s.gemm_group_used = 0;
+                    }
+                } else if (prec == T2X_PREC_FP32) {
                     T2X_TRY(launch_gemm(EPI_DIFF2, d->A.as<float>(), Kc, d->coarse_B.as<float>(), Kc, Kc,
                                         (int)M_pad, (int)O_pad, ep, st));
                 } else {
@@ -3553,13 +3422,6 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
                                                     d->coarse_Bl.ptr, d->coarse_Bs.as<float>(), Kc, Kc,
                                                     d->prop_plist.as<int>(), d->prop_work.ptr, n_work, (int)T,
                                                     O_pad - 1, ep, st));
-                    } else if (prune_batch) {
-                        T2X_TRY(launch_gemm_pruned(prec, d->Ah.ptr, d->Al.ptr, d->As.as<float>(), Kc, M_pad,
-                                                   d->coarse_Bh.ptr, d->coarse_Bl.ptr, d->coarse_Bs.as<float>(), Kc, Kc,
-                                                   (int)M_pad, (int)O_pad, ep, d_rowmin.as<float>(),
-                                                   d->prune_seed.as<float>(), d->prune_list.as<unsigned>(),
-                                                   prune_ntiles, d->prune_cnt.as<unsigned>(), d->n_cu, st));
-                        gused = GemmChoice{258, 0};   // group 0: the tile list
                     } else
                         T2X_TRY(launch_gemm_x3(prec, EPI_DIFF2, d->Ah.ptr, d->Al.ptr, d->As.as<float>(), Kc,
                                                M_pad, d->coarse_Bh.ptr, d->coarse_Bl.ptr, d->coarse_Bs.as<float>(), Kc,
@@ -4034,7 +3896,7 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
             rb.add(hpower.data(), d->power.ptr, sizeof(double) * B * xN);
             rb.add(hps2.data(), d_ps, sizeof(PartScalars) * B);
             if (cand_path) rb.add(hflag.data(), d_radix, sizeof(int) * B);
-            if (prune_batch) rb.add(&hprune, d->prune_cnt.ptr, sizeof(unsigned));
+            if (prune_batch) rb.add(&hprune, d->prune.cnt.ptr, sizeof(unsigned));
             T2X_TRY(rb.run(d, st));
         }
         if (hplan.err_code) {
@@ -4057,9 +3919,9 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
             const double skipped = (double)prune_ntiles - (double)hprune;
             stt.coarse_tiles_pruned += skipped;
             stt.coarse_tiles_checked += (double)prune_ntiles;
-            stt.coarse_bound_flop += 4.0 * (double)T * (double)O_all * (double)(K_low / 2) * B;
-            // a pass that prunes little costs more than the exhaustive one: off for the call's rest
-            if (prune_ntiles > 0 && skipped < 0.4 * (double)prune_ntiles) prune_call = false;
+            stt.coarse_bound_flop += 4.0 * (double)T * (double)O_all * (double)n_low * B;
+            // a pass that prunes little does not pay for its bounds: off for the call's rest
+            if (!prune_force && skipped < 0.4 * (double)prune_ntiles) prune_call = false;
         }
         if (!cand_path) {
             stt.n_select_fallbacks += 1;

@@ -27,18 +27,6 @@ enum { EPI_STORE = 0, EPI_DIFF2 = 1 };
 // gets 8 rows x 8 columns of them: every A and B tile slice fetched into an XCD's L2 feeds 8
 // workgroups there, and all XCDs walk the same B columns at the same time (one HBM read of B
 // per row group, shared through the MALL). The map is a bijection for any tiles_m, tiles_n.
-// The epilogue's N1 term of particle p, column n: N1 itself, or in a bounds launch of the pruned
-// coarse pass N1 - c0 sqrt(N1h) - c1 sqrt(N1) (the Cauchy-Schwarz bound of the cross term beyond
-// the low-frequency prefix and the margin for the dropped FP16 product; c0, c1 per particle).
-__device__ __forceinline__ float n1_at(const EpiParams& ep, long long p, long long n)
-{
-    const long long q = p * ep.ldn + n;
-    const float v = ep.N1[q];
-    if (ep.N1h == nullptr) return v;
-    const double c0 = ep.prune_c[2 * p], c1 = ep.prune_c[2 * p + 1];
-    return (float)((double)v - c0 * sqrt(fmax((double)ep.N1h[q], 0.)) - c1 * sqrt(fmax((double)v, 0.)));
-}
-
 __device__ __forceinline__ void tile_coords(int pid, int tiles_m, int tiles_n, int group_m, int& tm, int& tn)
 {
     const int per_group = group_m * tiles_n;
@@ -48,41 +36,6 @@ __device__ __forceinline__ void tile_coords(int pid, int tiles_m, int tiles_n, i
     const int in_group = pid - gid * per_group;
     tm = first_m + in_group % gsize;
     tn = in_group / gsize;
-}
-
-// Pruned coarse pass, tile plan: one wave per tile of tile_rows x tile_cols (tile_cols a multiple
-// of 64). A tile stays uncomputed when every 64-column block of every valid row has its lower
-// bound lb more than the negligible-weight cut (60, plus 1 for rounding) above the row's
-// particle's seed (an upper bound of its minimum diff2); its blocks then get their bounds as
-// minima (already in place when lb is the minima buffer itself). The other tiles are appended to
-// `list` (count[0] of them), in no particular order.
-__global__ __launch_bounds__(256) void k_prune_plan(const float* lb, const float* __restrict__ seed,
-                                                    float* rowmin, int rowmin_ld, long long M, int T,
-                                                    int tile_rows, int tile_cols, int tiles_m, int tiles_n,
-                                                    unsigned* __restrict__ list, unsigned* __restrict__ count)
-{
-    const unsigned tile = blockIdx.x * 4u + (threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
-    if (tile >= (unsigned)tiles_m * (unsigned)tiles_n) return;   // uniform over the wave
-    const int nblk = tile_cols / 64;
-    const long long m0 = (long long)(tile / (unsigned)tiles_n) * tile_rows;
-    const long long blk0 = (long long)(tile % (unsigned)tiles_n) * nblk;
-    bool keep = false;
-    for (int q = lane; q < tile_rows * nblk; q += 64) {
-        const long long m = m0 + q / nblk, blk = blk0 + q % nblk;
-        if (m >= M || blk >= rowmin_ld) continue;
-        if (!(lb[m * rowmin_ld + blk] > seed[m / T] + 61.f)) keep = true;
-    }
-    if (__any(keep)) {
-        if (lane == 0) list[atomicAdd(&count[0], 1u)] = tile;
-        return;
-    }
-    if (rowmin == lb) return;
-    for (int q = lane; q < tile_rows * nblk; q += 64) {
-        const long long m = m0 + q / nblk, blk = blk0 + q % nblk;
-        if (m >= M || blk >= rowmin_ld) continue;
-        rowmin[m * rowmin_ld + blk] = lb[m * rowmin_ld + blk];
-    }
 }
 
 // Shared epilogue of the GEMM kernels for one wave's block of MI x 4 MFMA tiles (lane holds
@@ -130,7 +83,7 @@ __device__ __forceinline__ void gemm_epilogue(const floatx4 (&acc)[MI][4], long 
                 pb[r] = b;
                 cb[r] = ep.Cb[b];
 #pragma unroll
-                for (int j = 0; j < 4; j++) n1[r][j] = n1_at(ep, b, nval[j] ? ncol[j] : 0);
+                for (int j = 0; j < 4; j++) n1[r][j] = ep.N1[(long long)b * ep.ldn + (nval[j] ? ncol[j] : 0)];
             }
         }
 #pragma unroll
@@ -150,7 +103,7 @@ __device__ __forceinline__ void gemm_epilogue(const floatx4 (&acc)[MI][4], long 
                     if (mval[r] && nval[j] && scored[j]) rmin = fminf(rmin, dv[j]);
                 }
                 for (int o = 1; o < 16; o <<= 1) rmin = fminf(rmin, __shfl_xor(rmin, o));
-                bool store = ep.C != nullptr;   // null: a bounds-only launch (block minima alone)
+                bool store = true;
                 if (ep.pmin && mval[r]) {
                     // the particle's final minimum is <= est, so a block more than the cut (60,
                     // plus one for rounding) above est is negligible whatever the final minimum
@@ -171,19 +124,14 @@ __device__ __forceinline__ void gemm_epilogue(const floatx4 (&acc)[MI][4], long 
 #define GBK 16
 #define GPAD 4
 
+// One 128x128 tile of the FP32 GEMM, rows from m0, columns from n0.
 template <int EPI>
-__global__ __launch_bounds__(256) void k_gemm_tn(const float* __restrict__ A, long long lda,
-                                                 const float* __restrict__ B, long long ldb,
-                                                 int K, int tiles_m, int tiles_n, int group_m, EpiParams ep)
+__device__ __forceinline__ void gemm_tn_tile(float (&As)[GBK][GBM + GPAD], float (&Bs)[GBK][GBN + GPAD],
+                                             const float* __restrict__ A, long long lda, const float* __restrict__ B,
+                                             long long ldb, int K, long long m0, long long n0, const EpiParams& ep)
 {
-    __shared__ float As[GBK][GBM + GPAD];
-    __shared__ float Bs[GBK][GBN + GPAD];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
-
-    int tm, tn;
-    tile_coords(blockIdx.x, tiles_m, tiles_n, group_m, tm, tn);
-    const long long m0 = (long long)tm * GBM, n0 = (long long)tn * GBN;
 
     floatx4 acc[4][4];
     for (int i = 0; i < 4; i++)
@@ -234,8 +182,28 @@ __global__ __launch_bounds__(256) void k_gemm_tn(const float* __restrict__ A, lo
     gemm_epilogue<4, EPI>(acc, m0 + wm * 64, n0 + wn * 64, lane, nullptr, nullptr, ep);
 }
 
-template __global__ void k_gemm_tn<EPI_STORE>(const float*, long long, const float*, long long, int, int, int, int, EpiParams);
-template __global__ void k_gemm_tn<EPI_DIFF2>(const float*, long long, const float*, long long, int, int, int, int, EpiParams);
+// LIST (the pruned coarse pass): a persistent grid over the tiles listed in ep.tile_list
+// (*ep.tile_count of them, indices tm * tiles_n + tn).
+template <int EPI, bool LIST = false>
+__global__ __launch_bounds__(256) void k_gemm_tn(const float* __restrict__ A, long long lda,
+                                                 const float* __restrict__ B, long long ldb,
+                                                 int K, int tiles_m, int tiles_n, int group_m, EpiParams ep)
+{
+    __shared__ float As[GBK][GBM + GPAD];
+    __shared__ float Bs[GBK][GBN + GPAD];
+    if constexpr (LIST) {
+        const unsigned n = *ep.tile_count;
+        for (unsigned it = blockIdx.x; it < n; it += gridDim.x) {
+            const unsigned t = ep.tile_list[it];
+            gemm_tn_tile<EPI>(As, Bs, A, lda, B, ldb, K, (long long)(t / (unsigned)tiles_n) * GBM,
+                              (long long)(t % (unsigned)tiles_n) * GBN, ep);
+        }   // (the tile's K loop starts with a barrier: its LDS is free again)
+    } else {
+        int tm, tn;
+        tile_coords(blockIdx.x, tiles_m, tiles_n, group_m, tm, tn);
+        gemm_tn_tile<EPI>(As, Bs, A, lda, B, ldb, K, (long long)tm * GBM, (long long)tn * GBN, ep);
+    }
+}
 
 // group_m of the tile walk; T2X_GEMM_GROUP_M overrides it for tile-order sweeps
 static int gemm_group_m()
@@ -303,20 +271,19 @@ struct SplitOperand {
 #define XK 32
 #define XPAD 8   // row stride 40 halfs = 80 bytes: conflict-free 16-byte reads for 16 lanes
 
-template <class H, int EPI>
-__global__ __launch_bounds__(256) void k_gemm_x3(SplitOperand A, SplitOperand B, int K, int tiles_m,
-                                                 int tiles_n, int group_m, EpiParams ep)
+// One 128x128 tile, rows from m0, columns from n0. NP = 2 (FP16X2): Al Bh + Ah Bh, B's lo half
+// neither loaded nor read. LDS [operand][row][column], operands Ah, Al, Bh, Bl.
+template <class H, int EPI, int NP>
+__device__ __forceinline__ void x3_tile(H (&st)[NP + 1][GBM][XK + XPAD], const SplitOperand& A, const SplitOperand& B,
+                                        int K, long long m0, long long n0, const EpiParams& ep)
 {
     typedef typename Vec8<H>::type v8;
-    __shared__ __attribute__((aligned(16))) H Ash[GBM][XK + XPAD];
-    __shared__ __attribute__((aligned(16))) H Asl[GBM][XK + XPAD];
-    __shared__ __attribute__((aligned(16))) H Bsh[GBN][XK + XPAD];
-    __shared__ __attribute__((aligned(16))) H Bsl[GBN][XK + XPAD];
+    auto& Ash = st[0];
+    auto& Asl = st[1];
+    auto& Bsh = st[2];
+    auto& Bsl = st[NP];   // NP = 3: the fourth operand
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
-    int tm, tn;
-    tile_coords(blockIdx.x, tiles_m, tiles_n, group_m, tm, tn);
-    const long long m0 = (long long)tm * GBM, n0 = (long long)tn * GBN;
 
     floatx4 acc[4][4];
     for (int i = 0; i < 4; i++)
@@ -333,7 +300,11 @@ __global__ __launch_bounds__(256) void k_gemm_x3(SplitOperand A, SplitOperand B,
     uint4 pa0h = *reinterpret_cast<const uint4*>(Ah + ra0), pa1h = *reinterpret_cast<const uint4*>(Ah + ra1);
     uint4 pa0l = *reinterpret_cast<const uint4*>(Al + ra0), pa1l = *reinterpret_cast<const uint4*>(Al + ra1);
     uint4 pb0h = *reinterpret_cast<const uint4*>(Bh + rb0), pb1h = *reinterpret_cast<const uint4*>(Bh + rb1);
-    uint4 pb0l = *reinterpret_cast<const uint4*>(Bl + rb0), pb1l = *reinterpret_cast<const uint4*>(Bl + rb1);
+    uint4 pb0l = {}, pb1l = {};
+    if (NP == 3) {
+        pb0l = *reinterpret_cast<const uint4*>(Bl + rb0);
+        pb1l = *reinterpret_cast<const uint4*>(Bl + rb1);
+    }
 
     for (int k0 = 0; k0 < K; k0 += XK) {
         __syncthreads();
@@ -343,8 +314,10 @@ __global__ __launch_bounds__(256) void k_gemm_x3(SplitOperand A, SplitOperand B,
         *reinterpret_cast<uint4*>(&Asl[lrow + 64][lc]) = pa1l;
         *reinterpret_cast<uint4*>(&Bsh[lrow][lc]) = pb0h;
         *reinterpret_cast<uint4*>(&Bsh[lrow + 64][lc]) = pb1h;
-        *reinterpret_cast<uint4*>(&Bsl[lrow][lc]) = pb0l;
-        *reinterpret_cast<uint4*>(&Bsl[lrow + 64][lc]) = pb1l;
+        if (NP == 3) {
+            *reinterpret_cast<uint4*>(&Bsl[lrow][lc]) = pb0l;
+            *reinterpret_cast<uint4*>(&Bsl[lrow + 64][lc]) = pb1l;
+        }
         __syncthreads();
         if (k0 + XK < K) {
             const int kn = k0 + XK;
@@ -354,8 +327,10 @@ __global__ __launch_bounds__(256) void k_gemm_x3(SplitOperand A, SplitOperand B,
             pa1l = *reinterpret_cast<const uint4*>(Al + ra1 + kn);
             pb0h = *reinterpret_cast<const uint4*>(Bh + rb0 + kn);
             pb1h = *reinterpret_cast<const uint4*>(Bh + rb1 + kn);
-            pb0l = *reinterpret_cast<const uint4*>(Bl + rb0 + kn);
-            pb1l = *reinterpret_cast<const uint4*>(Bl + rb1 + kn);
+            if (NP == 3) {
+                pb0l = *reinterpret_cast<const uint4*>(Bl + rb0 + kn);
+                pb1l = *reinterpret_cast<const uint4*>(Bl + rb1 + kn);
+            }
         }
         const int kc = (lane >> 4) * 8;
         v8 ah[4], al[4], bh[4], bl[4];
@@ -367,20 +342,43 @@ __global__ __launch_bounds__(256) void k_gemm_x3(SplitOperand A, SplitOperand B,
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             bh[j] = *reinterpret_cast<const v8*>(&Bsh[wn * 64 + j * 16 + (lane & 15)][kc]);
-            bl[j] = *reinterpret_cast<const v8*>(&Bsl[wn * 64 + j * 16 + (lane & 15)][kc]);
+            if (NP == 3) bl[j] = *reinterpret_cast<const v8*>(&Bsl[wn * 64 + j * 16 + (lane & 15)][kc]);
         }
 #pragma unroll
         for (int i = 0; i < 4; i++) {
 #pragma unroll
             for (int j = 0; j < 4; j++) acc[i][j] = mfma16x16x32<H>(al[i], bh[j], acc[i][j]);
+            if (NP == 3) {
 #pragma unroll
-            for (int j = 0; j < 4; j++) acc[i][j] = mfma16x16x32<H>(ah[i], bl[j], acc[i][j]);
+                for (int j = 0; j < 4; j++) acc[i][j] = mfma16x16x32<H>(ah[i], bl[j], acc[i][j]);
+            }
 #pragma unroll
             for (int j = 0; j < 4; j++) acc[i][j] = mfma16x16x32<H>(ah[i], bh[j], acc[i][j]);
         }
     }
 
     gemm_epilogue<4, EPI>(acc, m0 + wm * 64, n0 + wn * 64, lane, A.inv_scale, B.inv_scale, ep);
+}
+
+// LIST (the pruned coarse pass): a persistent grid over the tiles listed in ep.tile_list
+// (*ep.tile_count of them, indices tm * tiles_n + tn).
+template <class H, int EPI, int NP = 3, bool LIST = false>
+__global__ __launch_bounds__(256) void k_gemm_x3(SplitOperand A, SplitOperand B, int K, int tiles_m,
+                                                 int tiles_n, int group_m, EpiParams ep)
+{
+    __shared__ __attribute__((aligned(16))) H st[NP + 1][GBM][XK + XPAD];
+    if constexpr (LIST) {
+        const unsigned n = *ep.tile_count;
+        for (unsigned it = blockIdx.x; it < n; it += gridDim.x) {
+            const unsigned t = ep.tile_list[it];
+            x3_tile<H, EPI, NP>(st, A, B, K, (long long)(t / (unsigned)tiles_n) * GBM,
+                                (long long)(t % (unsigned)tiles_n) * GBN, ep);
+        }   // (the tile's K loop starts with a barrier: its LDS is free again)
+    } else {
+        int tm, tn;
+        tile_coords(blockIdx.x, tiles_m, tiles_n, group_m, tm, tn);
+        x3_tile<H, EPI, NP>(st, A, B, K, (long long)tm * GBM, (long long)tn * GBN, ep);
+    }
 }
 
 // Wide variant: 256x256 tile per workgroup of 8 waves, each wave 128x64 (8x4 MFMA tiles), so
@@ -603,30 +601,16 @@ __device__ __forceinline__ void lds_dma16(const H* src, H* lds_dst)
 template <class H>
 __device__ __forceinline__ void x3_group(floatx4 (&acc)[4], typename Vec8<H>::type al, typename Vec8<H>::type ah,
                                          const typename Vec8<H>::type (&bh)[4], const typename Vec8<H>::type (&bl)[4],
-                                         bool with_bl = true, bool with_al = true)
+                                         bool with_bl = true)
 {
-    if (with_al) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) acc[j] = mfma16x16x32<H>(al, bh[j], acc[j]);
-    }
+    for (int j = 0; j < 4; j++) acc[j] = mfma16x16x32<H>(al, bh[j], acc[j]);
     if (with_bl) {
 #pragma unroll
         for (int j = 0; j < 4; j++) acc[j] = mfma16x16x32<H>(ah, bl[j], acc[j]);
     }
 #pragma unroll
     for (int j = 0; j < 4; j++) acc[j] = mfma16x16x32<H>(ah, bh[j], acc[j]);
-}
-
-// NP = 4 (one product over two K chunks per stage): the hi halves of chunk 0 (ah, bh) and of
-// chunk 1 (al, bl, held in the lo slots).
-template <class H>
-__device__ __forceinline__ void x3_group2(floatx4 (&acc)[4], typename Vec8<H>::type a1, typename Vec8<H>::type a0,
-                                          const typename Vec8<H>::type (&b0)[4], const typename Vec8<H>::type (&b1)[4])
-{
-#pragma unroll
-    for (int j = 0; j < 4; j++) acc[j] = mfma16x16x32<H>(a1, b1[j], acc[j]);
-#pragma unroll
-    for (int j = 0; j < 4; j++) acc[j] = mfma16x16x32<H>(a0, b0[j], acc[j]);
 }
 
 // Epilogue inputs of one 256x256 tile, staged in LDS before the K loop so that their global
@@ -681,7 +665,7 @@ __device__ __forceinline__ bool stage_epilogue(EpiStage& es, long long m0l, long
             const unsigned ms = max(m0, (p0 + s) * T);   // a valid row of slot s
             const unsigned p = rowmap ? (unsigned)rowmap[ms] / T : p0 + s;
             const long long n = n0 + c;
-            es.cbn1[s][c] = ep.Cb[p] + (double)(n < ep.N ? n1_at(ep, p, n) : 0.f);
+            es.cbn1[s][c] = ep.Cb[p] + (double)(n < ep.N ? ep.N1[(long long)p * ep.ldn + n] : 0.f);
         }
         if (tid < EPI_SLOTS) {
             int p = -1;   // no particle: slot beyond the tile's valid rows
@@ -765,7 +749,7 @@ __device__ __forceinline__ void gemm_epilogue_staged(const floatx4 (&acc)[MI][4]
                     rmin = (nval[j] && scored[j]) ? fminf(rmin, dv[j]) : rmin;
                 }
                 rmin = min_row16(rmin);
-                bool store = rv && ep.C != nullptr;   // null: a bounds-only launch (block minima alone)
+                bool store = rv;
                 if (lazy) {
                     // the particle's final minimum is <= es_q, so a block more than the cut (60,
                     // plus one for rounding) above es_q is negligible whatever the final minimum
@@ -793,9 +777,7 @@ __device__ __forceinline__ void gemm_epilogue_staged(const floatx4 (&acc)[MI][4]
 }
 
 // NP = 3: Al Bh + Ah Bl + Ah Bh; NP = 2 (FP16X2): Al Bh + Ah Bh, the B operand's hi half alone
-// (its lo half neither loaded nor read); NP = 1 (a bounds form of the pruned coarse pass):
-// Ah Bh alone; NP = 4 (the other bounds form): Ah Bh alone over two K chunks per stage, the lo
-// slots holding the hi halves of the second chunk (K a multiple of 64).
+// (its lo half neither loaded nor read).
 // One tile, rows [m0, m0 + WBM) x columns [n0, n0 + WBN): stage s of the K loop lives in st0
 // (s even) or st1 (s odd); [operand][row * 32 + chunk] with operands Ah, Al, Bh, Bl and 16-byte
 // chunks swizzled as swz().
@@ -808,7 +790,6 @@ __device__ __forceinline__ void x3p_tile(H (&st0)[4][WBM * 32], H (&st1)[4][WBM 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave & 1, wn = wave >> 1;
-    constexpr int KS = NP == 4 ? 2 * XK : XK;   // K columns per stage
 
     floatx4 acc[8][4];
 #pragma unroll
@@ -841,22 +822,13 @@ __device__ __forceinline__ void x3p_tile(H (&st0)[4][WBM * 32], H (&st1)[4][WBM 
         const long long kb = (long long)(k) * (long long)sizeof(H);                               \
         lds_dma16<H>(reinterpret_cast<const H*>(Ah + kb + oa0), &ST[0][rb0 * 32]);               \
         lds_dma16<H>(reinterpret_cast<const H*>(Ah + kb + oa1), &ST[0][rb1 * 32]);               \
-        if (NP == 2 || NP == 3) {                                                                 \
-            lds_dma16<H>(reinterpret_cast<const H*>(Al + kb + oa0), &ST[1][rb0 * 32]);           \
-            lds_dma16<H>(reinterpret_cast<const H*>(Al + kb + oa1), &ST[1][rb1 * 32]);           \
-        }                                                                                         \
+        lds_dma16<H>(reinterpret_cast<const H*>(Al + kb + oa0), &ST[1][rb0 * 32]);               \
+        lds_dma16<H>(reinterpret_cast<const H*>(Al + kb + oa1), &ST[1][rb1 * 32]);               \
         lds_dma16<H>(reinterpret_cast<const H*>(Bh + kb + ob0), &ST[2][rb0 * 32]);               \
         lds_dma16<H>(reinterpret_cast<const H*>(Bh + kb + ob1), &ST[2][rb1 * 32]);               \
         if (NP == 3) {                                                                            \
             lds_dma16<H>(reinterpret_cast<const H*>(Bl + kb + ob0), &ST[3][rb0 * 32]);           \
             lds_dma16<H>(reinterpret_cast<const H*>(Bl + kb + ob1), &ST[3][rb1 * 32]);           \
-        }                                                                                         \
-        if (NP == 4) {   /* the hi halves' next K chunk into the lo slots */                      \
-            const long long kc = kb + XK * (long long)sizeof(H);                                  \
-            lds_dma16<H>(reinterpret_cast<const H*>(Ah + kc + oa0), &ST[1][rb0 * 32]);           \
-            lds_dma16<H>(reinterpret_cast<const H*>(Ah + kc + oa1), &ST[1][rb1 * 32]);           \
-            lds_dma16<H>(reinterpret_cast<const H*>(Bh + kc + ob0), &ST[3][rb0 * 32]);           \
-            lds_dma16<H>(reinterpret_cast<const H*>(Bh + kc + ob1), &ST[3][rb1 * 32]);           \
         }                                                                                         \
     } while (0)
 
@@ -868,14 +840,13 @@ __device__ __forceinline__ void x3p_tile(H (&st0)[4][WBM * 32], H (&st1)[4][WBM 
     do {                                                                         \
         _Pragma("unroll") for (int j = 0; j < 4; j++) {                          \
             BH[j] = *reinterpret_cast<const v8*>(&ST[2][ob + j * 512]);          \
-            if (NP >= 3) BL[j] = *reinterpret_cast<const v8*>(&ST[3][ob + j * 512]); \
+            if (NP == 3) BL[j] = *reinterpret_cast<const v8*>(&ST[3][ob + j * 512]); \
         }                                                                        \
     } while (0)
 #define X3P_READ_A(ST, i, AH, AL)                                                \
     do {                                                                         \
         AH = *reinterpret_cast<const v8*>(&ST[0][oa + (i) * 512]);               \
-        if (NP >= 2) AL = *reinterpret_cast<const v8*>(&ST[1][oa + (i) * 512]);  \
-        else AL = v8{};                                                          \
+        AL = *reinterpret_cast<const v8*>(&ST[1][oa + (i) * 512]);               \
     } while (0)
 
     // One K step on stage CUR (fragments bh/bl and A block 0 already in registers): A blocks
@@ -893,39 +864,36 @@ __device__ __forceinline__ void x3p_tile(H (&st0)[4][WBM * 32], H (&st1)[4][WBM 
                 X3P_READ_A(CUR, 6, a6h, a6l);                                    \
                 X3P_READ_A(CUR, 7, a7h, a7l);                                    \
             }                                                                    \
-            if (NP == 4) x3_group2<H>(acc[i], al, ah, bh, bl);                    \
-            else x3_group<H>(acc[i], al, ah, bh, bl, NP == 3, NP >= 2);          \
+            x3_group<H>(acc[i], al, ah, bh, bl, NP == 3);                        \
             if (i < 5) { ah = nh; al = nl; }                                     \
         }                                                                        \
         __builtin_amdgcn_s_waitcnt(0);                                           \
         __syncthreads();                                                         \
-        if ((s) + 2 < nk) X3P_LOAD(CUR, ((s) + 2) * KS);                         \
+        if ((s) + 2 < nk) X3P_LOAD(CUR, ((s) + 2) * XK);                         \
         const bool nxt = (s) + 1 < nk;                                           \
         if (nxt) X3P_READ_A(NXT, 0, ah, al);                                     \
         /* groups 6 and 7 column by column: B fragment j of this step is dead */ \
         /* after column j, and fragment j of the next step takes its registers */ \
         _Pragma("unroll") for (int j = 0; j < 4; j++) {                          \
-            if (NP == 2 || NP == 3) acc[6][j] = mfma16x16x32<H>(a6l, bh[j], acc[6][j]); \
+            acc[6][j] = mfma16x16x32<H>(a6l, bh[j], acc[6][j]);                  \
             if (NP == 3) acc[6][j] = mfma16x16x32<H>(a6h, bl[j], acc[6][j]);     \
-            if (NP == 4) acc[6][j] = mfma16x16x32<H>(a6l, bl[j], acc[6][j]);     \
             acc[6][j] = mfma16x16x32<H>(a6h, bh[j], acc[6][j]);                  \
-            if (NP == 2 || NP == 3) acc[7][j] = mfma16x16x32<H>(a7l, bh[j], acc[7][j]); \
+            acc[7][j] = mfma16x16x32<H>(a7l, bh[j], acc[7][j]);                  \
             if (NP == 3) acc[7][j] = mfma16x16x32<H>(a7h, bl[j], acc[7][j]);     \
-            if (NP == 4) acc[7][j] = mfma16x16x32<H>(a7l, bl[j], acc[7][j]);     \
             acc[7][j] = mfma16x16x32<H>(a7h, bh[j], acc[7][j]);                  \
             if (nxt) {                                                           \
                 bh[j] = *reinterpret_cast<const v8*>(&NXT[2][ob + j * 512]);     \
-                if (NP >= 3) bl[j] = *reinterpret_cast<const v8*>(&NXT[3][ob + j * 512]); \
+                if (NP == 3) bl[j] = *reinterpret_cast<const v8*>(&NXT[3][ob + j * 512]); \
             }                                                                    \
         }                                                                        \
     } while (0)
 
-    const int nk = K / KS;
+    const int nk = K / XK;
     X3P_LOAD(st0, 0);
     const bool staged = stage_epilogue<EPI>(es, m0, n0, A.inv_scale, B.inv_scale, ep, rowmap, tid);
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
-    if (nk > 1) X3P_LOAD(st1, KS);
+    if (nk > 1) X3P_LOAD(st1, XK);
     v8 bh[4], bl[4], ah, al;
     X3P_READ_B(st0, bh, bl);
     X3P_READ_A(st0, 0, ah, al);
@@ -943,9 +911,7 @@ __device__ __forceinline__ void x3p_tile(H (&st0)[4][WBM * 32], H (&st1)[4][WBM 
         gemm_epilogue<8, EPI>(acc, m0 + wm * 128, n0 + wn * 64, lane, A.inv_scale, B.inv_scale, ep, rowmap);
 }
 
-// LIST (the pruned coarse pass): a persistent grid over the tiles listed in ep.tile_list
-// (*ep.tile_count of them, indices tm * tiles_n + tn), no row map.
-template <class H, int EPI, int NP = 3, bool LIST = false>
+template <class H, int EPI, int NP = 3>
 __global__ __launch_bounds__(512) void k_gemm_x3p(SplitOperand A, SplitOperand B, int K, int tiles_m,
                                                   int tiles_n, int group_m, EpiParams ep,
                                                   const int* __restrict__ rowmap)
@@ -953,19 +919,9 @@ __global__ __launch_bounds__(512) void k_gemm_x3p(SplitOperand A, SplitOperand B
     __shared__ __attribute__((aligned(16))) H st0[4][WBM * 32];
     __shared__ __attribute__((aligned(16))) H st1[4][WBM * 32];
     __shared__ EpiStage es;
-    if constexpr (LIST) {
-        const unsigned n = *ep.tile_count;
-        for (unsigned it = blockIdx.x; it < n; it += gridDim.x) {
-            const unsigned t = ep.tile_list[it];
-            x3p_tile<H, EPI, NP>(st0, st1, es, A, B, K, (long long)(t / (unsigned)tiles_n) * WBM,
-                                 (long long)(t % (unsigned)tiles_n) * WBN, ep, nullptr);
-            __syncthreads();   // the next tile reuses the LDS stages
-        }
-    } else {
-        int tm, tn;
-        tile_coords(blockIdx.x, tiles_m, tiles_n, group_m, tm, tn);
-        x3p_tile<H, EPI, NP>(st0, st1, es, A, B, K, (long long)tm * WBM, (long long)tn * WBN, ep, rowmap);
-    }
+    int tm, tn;
+    tile_coords(blockIdx.x, tiles_m, tiles_n, group_m, tm, tn);
+    x3p_tile<H, EPI, NP>(st0, st1, es, A, B, K, (long long)tm * WBM, (long long)tn * WBN, ep, rowmap);
 }
 
 // Two-product half-height variant (FP16X2 only): tile 128 (M) x 256 (N), 4 waves of 64 x 128,
@@ -1020,7 +976,7 @@ __device__ __forceinline__ bool stage_epilogue_h(EpiStageH& es, long long m0l, l
         const unsigned ms = max(m0, (p0 + sl) * T);   // a valid row of slot sl
         const unsigned p = rowmap ? (unsigned)rowmap[ms] / T : p0 + sl;
         const long long n = n0 + c;
-        es.n1[sl][c] = n < ep.N ? n1_at(ep, p, n) : 0.f;
+        es.n1[sl][c] = n < ep.N ? ep.N1[(long long)p * ep.ldn + n] : 0.f;
     }
     if (tid < EPI_SLOTS) {
         int p = -1;
@@ -1034,9 +990,6 @@ __device__ __forceinline__ bool stage_epilogue_h(EpiStageH& es, long long m0l, l
     return true;
 }
 
-// ONE: the bounds form of the pruned coarse pass, one product (A hi . B hi) per element; A lo is
-// neither loaded nor multiplied (the caller allows for the dropped term in its bound).
-template <bool ONE>
 __device__ __forceinline__ void x2h_tile(_Float16 (&sa0)[2][128 * 32], _Float16 (&sb0)[256 * 32],
                                          _Float16 (&sa1)[2][128 * 32], _Float16 (&sb1)[256 * 32], EpiStageH& es,
                                          const SplitOperand& A, const SplitOperand& B, int K, long long m0,
@@ -1078,10 +1031,8 @@ __device__ __forceinline__ void x2h_tile(_Float16 (&sa0)[2][128 * 32], _Float16 
         const long long kb = (long long)(k) * (long long)sizeof(H);                          \
         lds_dma16<H>(reinterpret_cast<const H*>(Ah + kb + oa0), &SA[0][ra0 * 32]);          \
         lds_dma16<H>(reinterpret_cast<const H*>(Ah + kb + oa1), &SA[0][ra1 * 32]);          \
-        if constexpr (!ONE) {                                                                \
-            lds_dma16<H>(reinterpret_cast<const H*>(Al + kb + oa0), &SA[1][ra0 * 32]);      \
-            lds_dma16<H>(reinterpret_cast<const H*>(Al + kb + oa1), &SA[1][ra1 * 32]);      \
-        }                                                                                    \
+        lds_dma16<H>(reinterpret_cast<const H*>(Al + kb + oa0), &SA[1][ra0 * 32]);          \
+        lds_dma16<H>(reinterpret_cast<const H*>(Al + kb + oa1), &SA[1][ra1 * 32]);          \
         _Pragma("unroll") for (int q = 0; q < 4; q++)                                        \
             lds_dma16<H>(reinterpret_cast<const H*>(Bh + kb + obq + q * ob16), &SB[(rb + 16 * q) * 32]); \
     } while (0)
@@ -1091,16 +1042,13 @@ __device__ __forceinline__ void x2h_tile(_Float16 (&sa0)[2][128 * 32], _Float16 
 #define X2H_READ_A(SA, i, AH, AL)                                   \
     do {                                                            \
         AH = *reinterpret_cast<const v8*>(&SA[0][oa + (i) * 512]);  \
-        if constexpr (ONE) AL = v8{};                               \
-        else AL = *reinterpret_cast<const v8*>(&SA[1][oa + (i) * 512]); \
+        AL = *reinterpret_cast<const v8*>(&SA[1][oa + (i) * 512]);  \
     } while (0)
     // one A block against the 8 B fragments: lo.hi then hi.hi per element
 #define X2H_GROUP(i, AL, AH)                                                                        \
     do {                                                                                            \
-        if constexpr (!ONE) {                                                                       \
-            _Pragma("unroll") for (int j = 0; j < 8; j++)                                           \
-                acc[j >> 2][i][j & 3] = mfma16x16x32<H>(AL, bh[j], acc[j >> 2][i][j & 3]);          \
-        }                                                                                           \
+        _Pragma("unroll") for (int j = 0; j < 8; j++)                                               \
+            acc[j >> 2][i][j & 3] = mfma16x16x32<H>(AL, bh[j], acc[j >> 2][i][j & 3]);              \
         _Pragma("unroll") for (int j = 0; j < 8; j++)                                               \
             acc[j >> 2][i][j & 3] = mfma16x16x32<H>(AH, bh[j], acc[j >> 2][i][j & 3]);              \
     } while (0)
@@ -1124,7 +1072,7 @@ __device__ __forceinline__ void x2h_tile(_Float16 (&sa0)[2][128 * 32], _Float16 
         const bool nxt = (s) + 1 < nk;                                             \
         if (nxt) X2H_READ_A(NA, 0, ah, al);                                        \
         _Pragma("unroll") for (int j = 0; j < 8; j++) {                            \
-            if constexpr (!ONE) acc[j >> 2][3][j & 3] = mfma16x16x32<H>(a3l, bh[j], acc[j >> 2][3][j & 3]); \
+            acc[j >> 2][3][j & 3] = mfma16x16x32<H>(a3l, bh[j], acc[j >> 2][3][j & 3]); \
             acc[j >> 2][3][j & 3] = mfma16x16x32<H>(a3h, bh[j], acc[j >> 2][3][j & 3]); \
             if (nxt) bh[j] = *reinterpret_cast<const v8*>(&NB[ob + j * 512]);      \
         }                                                                          \
@@ -1158,7 +1106,6 @@ __device__ __forceinline__ void x2h_tile(_Float16 (&sa0)[2][128 * 32], _Float16 
     }
 }
 
-template <bool ONE>
 __global__ __launch_bounds__(256, 2) void k_gemm_x2h(SplitOperand A, SplitOperand B, int K, int tiles_m, int tiles_n,
                                                      int group_m, EpiParams ep, const int* __restrict__ rowmap)
 {
@@ -1169,7 +1116,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_x2h(SplitOperand A, SplitOperan
     __shared__ EpiStageH es;
     int tm, tn;
     tile_coords(blockIdx.x, tiles_m, tiles_n, group_m, tm, tn);
-    x2h_tile<ONE>(sa0, sb0, sa1, sb1, es, A, B, K, (long long)tm * 128, (long long)tn * 256, ep, rowmap);
+    x2h_tile(sa0, sb0, sa1, sb1, es, A, B, K, (long long)tm * 128, (long long)tn * 256, ep, rowmap);
 }
 
 // Learned-proposal variant: one workgroup per work item = (bin, row tile, column tile). The
@@ -1522,7 +1469,7 @@ static int launch_x3_variant(int prec, int epi, const SplitOperand& A, const Spl
             set_error("gemm_x3: tile 259 serves the FP16X2 diff2 GEMM only");
             return T2X_EINVAL;
         }
-        k_gemm_x2h<false><<<grid, 256, 0, st>>>(A, B, K, tm, tn, g, ep, rowmap);
+        k_gemm_x2h<<<grid, 256, 0, st>>>(A, B, K, tm, tn, g, ep, rowmap);
     } else if (tile == 257) {
         if (bf) { if (store) k_gemm_x3d<__bf16, EPI_STORE><<<grid, 256, 0, st>>>(A, B, K, tm, tn, g, ep);
                   else k_gemm_x3d<__bf16, EPI_DIFF2><<<grid, 256, 0, st>>>(A, B, K, tm, tn, g, ep); }
@@ -1551,65 +1498,24 @@ static int launch_x3_variant(int prec, int epi, const SplitOperand& A, const Spl
     return T2X_OK;
 }
 
-// Bounds form of the pruned coarse pass: block minima of the diff2 with one FP16 product per
-// element (A hi . B hi), no values stored (ep.C null): k_gemm_x3p with two K chunks per LDS stage
-// (the stage's lo slots hold the second chunk's hi halves), so each barrier and operand wait
-// covers twice the MFMA work of a one-chunk stage.
-int launch_gemm_h1_bounds(const void* Ah, const float* As, long long lda, long long a_rows, const void* Bh,
-                          const float* Bs, long long ldb, int K, int Mrows_pad, int Nrows_pad, const EpiParams& ep,
-                          hipStream_t st)
+// Pruned coarse pass, full GEMM: the diff2 GEMM over the listed tiles of PRUNED_TILE rows and columns
+// (*count of them) on a persistent grid of the workgroups that fit on the chip at once: k_gemm_x3 (2
+// products under FP16X2, else 3) or k_gemm_tn. Small tiles, since a tile is computed for any one of its
+// 64-column blocks: at class256 0.9% of the 128x128 tiles and 2.8% of the 256x256 ones are (0.73
+// against 1.06 ms per 800 particles with k_gemm_x3p, for all its faster K loop; 3 products at 500
+// particles 1.60 against 2.06 ms).
+int launch_gemm_pruned(int prec, const void* Ah, const void* Al, const float* As, long long lda, const void* Bh,
+                       const void* Bl, const float* Bs, long long ldb, int K, int Mrows_pad, int Nrows_pad,
+                       const EpiParams& ep, const unsigned* list, const unsigned* count, int n_cu, hipStream_t st)
 {
-    const long long lim = 1LL << 32;
-    if (a_rows * lda * 2 >= lim || (long long)Nrows_pad * ldb * 2 >= lim) {
-        set_error("gemm_h1_bounds: operands beyond 4 GiB (32-bit offsets)");
-        return T2X_EINVAL;
-    }
-    if (ep.C != nullptr || ep.pmin != nullptr) {
-        set_error("gemm_h1_bounds: a bounds-only launch (no stores, no lazy minima)");
-        return T2X_EINVAL;
-    }
-    if (K % XK != 0 || Mrows_pad % 128 != 0 || Nrows_pad % 256 != 0) {
-        set_error("gemm_h1_bounds: operands not padded to tile multiples");
-        return T2X_EINVAL;
-    }
-    // 260 (default): k_gemm_x3p NP = 4 (256x256, two K chunks per stage; K a multiple of 64);
-    // 258: k_gemm_x3p NP = 1; 259 (and the fallback): k_gemm_x2h<true> (128x256)
-    const char* env_t = getenv("T2X_BOUNDS_TILE");
-    const int bt = env_t ? atoi(env_t) : 260;
-    const bool wide = (bt == 258 || (bt == 260 && K % (2 * XK) == 0)) && Mrows_pad % 256 == 0;
-    const int tm = Mrows_pad / (wide ? 256 : 128), tn = Nrows_pad / 256;
-    const long long nwg = (long long)tm * tn;
-    if (nwg > 0x7fffffffLL) { set_error("gemm: grid too large"); return T2X_EINVAL; }
-    SplitOperand A{Ah, nullptr, As, lda}, B{Bh, nullptr, Bs, ldb};
-    const char* env_g = getenv("T2X_BOUNDS_GROUP");   // tile-walk group (tile rows per group)
-    const int g = env_g && atoi(env_g) > 0 ? atoi(env_g) : 32;
-    if (wide && bt == 260)
-        k_gemm_x3p<_Float16, EPI_DIFF2, 4><<<(unsigned)nwg, 512, 0, st>>>(A, B, K, tm, tn, g, ep, nullptr);
-    else if (wide)
-        k_gemm_x3p<_Float16, EPI_DIFF2, 1><<<(unsigned)nwg, 512, 0, st>>>(A, B, K, tm, tn, g, ep, nullptr);
-    else
-        k_gemm_x2h<true><<<(unsigned)nwg, 256, 0, st>>>(A, B, K, tm, tn, g, ep, nullptr);
-    T2X_HIP(hipGetLastError());
-    return T2X_OK;
-}
-
-// Pruned coarse pass, full GEMM: the tile plan (k_prune_plan over the tiles of the kernel that
-// follows, from the block bounds lb and the per-particle seeds) and then the diff2 GEMM over the
-// kept tiles: k_gemm_x3p (256x256 tiles; 2 products under FP16X2, else 3) on a persistent grid of
-// one workgroup per compute unit. list holds list_cap entries; count (one word) must be zero on
-// entry and holds the kept tiles' number on return.
-int launch_gemm_pruned(int prec, const void* Ah, const void* Al, const float* As, long long lda, long long a_rows,
-                       const void* Bh, const void* Bl, const float* Bs, long long ldb, int K, int Mrows_pad,
-                       int Nrows_pad, const EpiParams& ep, const float* lb, const float* seed, unsigned* list,
-                       long long list_cap, unsigned* count, int n_cu, hipStream_t st)
-{
-    const long long lim = 1LL << 32;
-    if (a_rows * lda * 2 >= lim || (long long)Nrows_pad * ldb * 2 >= lim) {
+    const bool fp32 = prec == T2X_PREC_FP32;
+    const long long lim = 1LL << 32;   // as the exhaustive FP16X2 GEMM, which the call's other batches may take
+    if (!fp32 && ((long long)Mrows_pad * lda * 2 >= lim || (long long)Nrows_pad * ldb * 2 >= lim)) {
         set_error("gemm_pruned: operands beyond 4 GiB (32-bit offsets)");
         return T2X_EINVAL;
     }
-    const int tr = WBM, tc = WBN;
-    if (K % XK != 0 || Mrows_pad % tr != 0 || Nrows_pad % tc != 0) {
+    static_assert(PRUNED_TILE == GBM && PRUNED_TILE == GBN, "tile of k_gemm_tn and k_gemm_x3");
+    if (K % (fp32 ? GBK : XK) != 0 || Mrows_pad % GBM != 0 || Nrows_pad % GBN != 0) {
         set_error("gemm_pruned: operands not padded to tile multiples");
         return T2X_EINVAL;
     }
@@ -1617,22 +1523,20 @@ int launch_gemm_pruned(int prec, const void* Ah, const void* Al, const float* As
         set_error("gemm_pruned: a diff2 launch with block minima");
         return T2X_EINVAL;
     }
-    const int tm = Mrows_pad / tr, tn = Nrows_pad / tc;
-    const long long ntiles = (long long)tm * tn;
-    if (ntiles > list_cap || ntiles > 0x7fffffffLL) { set_error("gemm_pruned: tile list too small"); return T2X_EINVAL; }
-    k_prune_plan<<<(unsigned)((ntiles + 3) / 4), 256, 0, st>>>(lb, seed, ep.rowmin, ep.rowmin_ld, ep.M, ep.T, tr, tc,
-                                                               tm, tn, list, count);
-    T2X_HIP(hipGetLastError());
+    const int tm = Mrows_pad / GBM, tn = Nrows_pad / GBN;
     EpiParams el = ep;
     el.tile_list = list;
     el.tile_count = count;
     SplitOperand A{Ah, Al, As, lda}, B{Bh, Bl, Bs, ldb};
-    if (prec == T2X_PREC_FP16X2)
-        k_gemm_x3p<_Float16, EPI_DIFF2, 2, true><<<(unsigned)n_cu, 512, 0, st>>>(A, B, K, tm, tn, 0, el, nullptr);
+    if (fp32)
+        k_gemm_tn<EPI_DIFF2, true><<<(unsigned)(4 * n_cu), 256, 0, st>>>((const float*)Ah, lda, (const float*)Bh, ldb, K,
+                                                                        tm, tn, 0, el);
+    else if (prec == T2X_PREC_FP16X2)
+        k_gemm_x3<_Float16, EPI_DIFF2, 2, true><<<(unsigned)(3 * n_cu), 256, 0, st>>>(A, B, K, tm, tn, 0, el);
     else if (prec == T2X_PREC_BF16X3)
-        k_gemm_x3p<__bf16, EPI_DIFF2, 3, true><<<(unsigned)n_cu, 512, 0, st>>>(A, B, K, tm, tn, 0, el, nullptr);
+        k_gemm_x3<__bf16, EPI_DIFF2, 3, true><<<(unsigned)(3 * n_cu), 256, 0, st>>>(A, B, K, tm, tn, 0, el);
     else
-        k_gemm_x3p<_Float16, EPI_DIFF2, 3, true><<<(unsigned)n_cu, 512, 0, st>>>(A, B, K, tm, tn, 0, el, nullptr);
+        k_gemm_x3<_Float16, EPI_DIFF2, 3, true><<<(unsigned)(3 * n_cu), 256, 0, st>>>(A, B, K, tm, tn, 0, el);
     T2X_HIP(hipGetLastError());
     return T2X_OK;
 }

@@ -165,6 +165,13 @@ struct Stats {
 
 namespace cnn { struct Net; }
 
+// Pruned coarse pass (t2x_prune.hip): the INT8 bounds GEMM's operands (reference side made with the
+// coarse projections, image side per batch), its base table, block bounds, seeds and tile list;
+// cnt[0] counts the list, cnt[1] the particles for which the bounds can pay.
+struct PruneBufs {
+    DevBuf w, B8, sb, nb, A8, pa, pf, base, lbs, seed, list, cnt;
+};
+
 struct Device;
 void destroy_graph(Device* d);
 
@@ -203,9 +210,8 @@ struct Device {
     // the phase tables' sizes and translations (ab_coarse / ab_fine hold them while unchanged)
     std::vector<double> ab_key;
     DevBuf prep_part;   // per particle and row band: background sums of the mask
-    // pruned coarse pass: N1 over the low-frequency prefix, its constant terms, the block lower
-    // bounds, the per-particle seeds and the tile counters
-    DevBuf prune_n1, prune_c, prune_seed, prune_cnt, prune_list;
+    PruneBufs prune;
+    std::string prune_key;   // the projections and prefix prune's reference side was made for
     bool graph_prune = false;   // the batch graph was captured with the pruned coarse pass
     DevBuf coarse_Ai;   // projection frames of the coarse orientations, for the angles in coarse_Ai_key
     std::vector<double> coarse_Ai_key;

@@ -159,17 +159,29 @@ struct EpiParams {
     // 64-column block whose minimum exceeds it by more than the negligible-weight cut are not
     // stored (the block minimum still is, so every reader skips the block). null: store all.
     unsigned int* pmin;
-    // Pruned coarse pass. C null: a bounds-only launch (EPI_DIFF2 writes the 64-column block
-    // minima, no values). tile_list: the tiles a list-driven (persistent) launch computes,
-    // *tile_count of them (read by the kernels of the LIST form only).
+    // Pruned coarse pass: the tiles a list-driven (persistent) launch computes, *tile_count of
+    // them (read by the kernels of the LIST form only).
     const unsigned int* tile_list;
     const unsigned int* tile_count;
-    // Bounds launch of the pruned coarse pass: N1h (the N1 term over the pixels beyond the
-    // low-frequency prefix, ld ldn) non-null turns each N1 read into N1 - c0 sqrt(N1h) -
-    // c1 sqrt(N1), with prune_c[2 p], prune_c[2 p + 1] = c0, c1 of particle p.
-    const float* N1h;
-    const double* prune_c;
 };
+
+// Rows and columns of the tiles of the pruned coarse pass's full GEMM.
+#define PRUNED_TILE 128
+
+// One batch of the pruned coarse pass (t2x_prune.hip).
+struct PruneCall {
+    int prec, B, T;
+    long long M_pad, O_all, O_pad;
+    int Kn;                    // columns of the N1 operands (pixels, padded); the GEMM's are 2 Kn
+    int n_low, K8;             // pixels of the low set; bytes of an INT8 row (a multiple of 128)
+    int force;                 // take the bounds whether or not they look to pay (tests)
+    const double* Cb;          // [B] C_b
+};
+// The reference side of the bounds (once per coarse projection), and a batch's bounds, seeds and list
+// of PRUNED_TILE tiles (in prune.list, prune.cnt[0] of them; both words of prune.cnt zero on entry). prune_bounds also
+// seeds the running minima pmin where the bounds are taken.
+int prune_prepare_refs(Device* d, long long O_all, long long O_pad, int Kc, int Kn, int n_low, int K8, hipStream_t st);
+int prune_bounds(Device* d, const PruneCall& c, const PartScalars* d_ps, const PassTables& tc, int Pw, hipStream_t st);
 
 struct SelParams {
     double fraction;
