@@ -124,7 +124,7 @@ extern "C" int t2x_device_close(t2x_device* h)
     for (DevBuf* b : bufs) b->release();
     PassTables* tabs[] = {&d->coarse_tab, &d->fine_tab};
     for (PassTables* t : tabs) {
-        t->d_pix.release(); t->d_win.release(); t->d_minv.release(); t->d_ires.release(); t->d_inproj.release();
+        t->d_pix.release(); t->d_gather.release(); t->d_win.release(); t->d_minv.release(); t->d_ires.release(); t->d_inproj.release();
     }
     if (d->fft_plan) (void)hipfftDestroy(d->fft_plan);
     if (d->noise_plan) (void)hipfftDestroy(d->noise_plan);
@@ -153,7 +153,8 @@ static int check_dims(int iclass, int ref_dim, int pad, int r_max, double pf)
     return T2X_OK;
 }
 
-// Interleaves re/im into the projector layout: a 2D plane row-major, a 3D volume in 4x4x4 bricks.
+// Interleaves re/im into the projector layout: a 2D plane row-major, a 3D volume in cells
+// (vol_cell_index).
 // Elements [base, base + n) of the caller's layout, re[k]/im[k] holding element base + k.
 __global__ void k_interleave(const float* __restrict__ re, const float* __restrict__ im,
                              float2* __restrict__ out, size_t base, size_t n, int ref_dim, int pad)
@@ -164,7 +165,10 @@ __global__ void k_interleave(const float* __restrict__ re, const float* __restri
     if (ref_dim == 2) { out[i] = make_float2(re[k], im[k]); return; }
     const int xdim = pad / 2 + 1;
     const int x = (int)(i % xdim), y = (int)((i / xdim) % pad), z = (int)(i / ((size_t)xdim * pad));
-    out[vol_brick_index(x, y, z, (xdim + 3) / 4, (pad + 3) / 4)] = make_float2(re[k], im[k]);
+    const size_t o = vol_cell_index(x, y, z, vol_cells_x(pad), vol_cells_y(pad));
+    const float2 v = make_float2(re[k], im[k]);
+    out[o] = v;
+    if (x > 0 && x % 3 == 0) out[vol_cell_index(x - 1, y, z, vol_cells_x(pad), vol_cells_y(pad)) + 1] = v;
 }
 
 extern "C" int t2x_projector_set(t2x_device* h, int iclass, int ref_dim, int pad_size, int r_max,
@@ -182,7 +186,7 @@ extern "C" int t2x_projector_set(t2x_device* h, int iclass, int ref_dim, int pad
         c.proj = nullptr;
     }
     if (!c.proj) {
-        const size_t ne = ref_dim == 3 ? vol_brick_elems(pad_size) : n;
+        const size_t ne = ref_dim == 3 ? vol_cell_elems(pad_size) : n;
         if (hipMalloc(&c.proj, ne * sizeof(float2)) != hipSuccess) {
             set_error("hipMalloc projector volume failed");
             return T2X_ENOMEM;
@@ -265,7 +269,7 @@ extern "C" int t2x_debug_projector_get(t2x_device* h, int iclass, float* re, flo
     if (it == d->classes.end() || !it->second.proj) { set_error("projector not set"); return T2X_ESTATE; }
     const ClassVolumes& c = it->second;
     const size_t n = vol_elems(c.p_ref_dim, c.p_pad);
-    const size_t ne = c.p_ref_dim == 3 ? vol_brick_elems(c.p_pad) : n;
+    const size_t ne = c.p_ref_dim == 3 ? vol_cell_elems(c.p_pad) : n;
     T2X_HIP(hipSetDevice(d->id));
     T2X_HIP(hipStreamSynchronize(d->stream));
     std::vector<float2> v(ne);
@@ -275,7 +279,7 @@ extern "C" int t2x_debug_projector_get(t2x_device* h, int iclass, float* re, flo
         size_t src = i;
         if (c.p_ref_dim == 3) {
             const int x = (int)(i % xdim), y = (int)((i / xdim) % pad), z = (int)(i / ((size_t)xdim * pad));
-            src = vol_brick_index(x, y, z, (xdim + 3) / 4, (pad + 3) / 4);
+            src = vol_cell_index(x, y, z, vol_cells_x(pad), vol_cells_y(pad));
         }
         re[i] = v[src].x;
         im[i] = v[src].y;

@@ -310,34 +310,72 @@ __global__ __launch_bounds__(256) void k_const_term(const float2* __restrict__ F
 // Coarse pass
 // ------------------------------------------------------------------------------------------
 
+// One chunk of a slice: the reference sampled in frame a at the pixels base .. base + GATHER_CHUNK - 1
+// (in gather order, 256 at a time, a thread's own sample and its quad's four in turn), the values left
+// in LDS in stored order (zero where not projected, outside the volume, or from npix up to ld).
+// 256 threads. Bound by the vector ALU (78% busy: address and interpolation) and the L1's line rate. Of
+// 224,000 slices of 10,000 pixels from a 415-voxel volume, in ms: a thread a sample in stored order 46.7;
+// in patches 24.5 (with 4096-pixel chunks 31: 20 waves' lines no longer fit the L1); a quad a sample 21;
+// cells instead of disjoint bricks 17.3. Chunks of 1024 pixels equal 4096 in this form and leave more
+// LDS to other workgroups.
+__device__ __forceinline__ void slice_chunk(const float2* __restrict__ vol, int pad, int ref2d, const float (&a)[6],
+                                            const int2* __restrict__ gather, int npix, int ld, int base, float2* sf)
+{
+    const int n = min(GATHER_CHUNK, npix - base);
+    for (int q = max(n, 0) + threadIdx.x; q < min(GATHER_CHUNK, ld - base); q += 256) sf[q] = make_float2(0.f, 0.f);
+    const int l = threadIdx.x & 3;
+    const unsigned ymask = (l & 1) ? ~0u : 0u, zmask = (l & 2) ? ~0u : 0u;
+    for (int q0 = 0; q0 < n; q0 += 256) {
+        const int q = q0 + threadIdx.x;
+        const int2 g = gather[base + min(q, n - 1)];
+        const float x = (float)(g.x & 0xffff), y = (float)(g.x >> 16);
+        float2 f = make_float2(0.f, 0.f);
+        if (ref2d) {
+            float2 v;
+            if (g.y >= 0 && bilinear_sample(vol, pad, a[0] * x + a[1] * y, a[2] * x + a[3] * y, &v)) f = v;
+        } else {
+            const TriPos t = trilinear_pos(pad, a[0] * x + a[1] * y, a[2] * x + a[3] * y, a[4] * x + a[5] * y);
+            const float2 v0 = trilinear_quad<0>(vol, t, ymask, zmask), v1 = trilinear_quad<1>(vol, t, ymask, zmask);
+            const float2 v2 = trilinear_quad<2>(vol, t, ymask, zmask), v3 = trilinear_quad<3>(vol, t, ymask, zmask);
+            const float2 v = (l & 2) ? ((l & 1) ? v3 : v2) : ((l & 1) ? v1 : v0);
+            if (t.ok && g.y >= 0) f = make_float2(v.x, t.neg ? -v.y : v.y);
+        }
+        if (q < n) sf[g.y >= 0 ? g.y : -1 - g.y] = f;
+    }
+}
+
 // Slices of all coarse orientations (Projector::project, projector.cpp:524-691): one workgroup
-// per (class, orientation), threads over the compact coarse pixels. Writes re/im interleaved
-// into B[n][2p..2p+1] and |F|^2 into B2[n][p].
+// per (class, orientation), chunk by chunk over the compact coarse pixels. Writes re/im interleaved
+// into B[n][2p..2p+1] and |F|^2 into B2[n][p], padding columns included. The XCDs (workgroup
+// index & 7) take contiguous orientations: a direction's psi rotations share its central plane, which
+// then comes from one L2.
 __global__ __launch_bounds__(256) void k_project_coarse(const float2* const* __restrict__ vols,
                                                         const int* __restrict__ pads,
                                                         const float* __restrict__ Ai,   // [Norient][9]
-                                                        int Norient, const int2* __restrict__ pix,
-                                                        const unsigned char* __restrict__ inproj,
+                                                        int Norient, int O_all, const int2* __restrict__ gather,
                                                         int npix, float* __restrict__ Bm, long long ldb,
                                                         float* __restrict__ B2, long long ldb2, int ref2d)
 {
-    const int n = blockIdx.x;
+    __shared__ __attribute__((aligned(16))) float2 sf[GATHER_CHUNK];
+    const int n = (int)(blockIdx.x % 8) * (int)(gridDim.x / 8) + (int)(blockIdx.x / 8);
+    if (n >= O_all) return;
     const int c = n / Norient, o = n - c * Norient;
-    const float2* vol = vols[c];
-    const int pad = pads[c];
     float a[6];
     for (int i = 0; i < 6; i++) a[i] = Ai[o * 9 + (i / 2) * 3 + (i % 2)];  // rows 0..2, cols 0..1
-    for (int p = threadIdx.x; p < npix; p += blockDim.x) {
-        float2 f = make_float2(0.f, 0.f);
-        if (inproj[p]) {
-            float x = (float)pix[p].x, y = (float)pix[p].y;
-            float xp = a[0] * x + a[1] * y, yp = a[2] * x + a[3] * y, zp = a[4] * x + a[5] * y;
-            float2 v;
-            if (ref_sample(vol, pad, ref2d, xp, yp, zp, &v)) f = v;
+    for (int base = 0; base < ldb2; base += GATHER_CHUNK) {
+        slice_chunk(vols[c], pads[c], ref2d, a, gather, npix, (int)ldb2, base, sf);
+        __syncthreads();
+        for (int q = 4 * threadIdx.x; q < min(GATHER_CHUNK, (int)ldb2 - base); q += 1024) {   // ldb2: a multiple of 32
+            const int p = base + q;
+            const float4 u = *reinterpret_cast<const float4*>(&sf[q]);
+            const float4 v = *reinterpret_cast<const float4*>(&sf[q + 2]);
+            float* d = Bm + (size_t)n * ldb + 2 * p;
+            *reinterpret_cast<float4*>(d) = u;
+            *reinterpret_cast<float4*>(d + 4) = v;
+            *reinterpret_cast<float4*>(B2 + (size_t)n * ldb2 + p) =
+                make_float4(u.x * u.x + u.y * u.y, u.z * u.z + u.w * u.w, v.x * v.x + v.y * v.y, v.z * v.z + v.w * v.w);
         }
-        Bm[(size_t)n * ldb + 2 * p] = f.x;
-        Bm[(size_t)n * ldb + 2 * p + 1] = f.y;
-        B2[(size_t)n * ldb2 + p] = f.x * f.x + f.y * f.y;
+        __syncthreads();
     }
 }
 
@@ -913,12 +951,6 @@ __global__ void k_fine_tmask(const long long* __restrict__ pair_off, const int2*
     for (int w = threadIdx.x; w < TW; w += blockDim.x) tmask[(size_t)b * TW + w] = m[w];
 }
 
-// Zero columns [n, ld) of each float2 row.
-__global__ void k_zero_row_tails(float2* __restrict__ F, int n, int ld)
-{
-    for (int p = n + threadIdx.x; p < ld; p += blockDim.x) F[(size_t)blockIdx.x * ld + p] = make_float2(0.f, 0.f);
-}
-
 // |F|^2 of float2 rows (the n1 term's operand when the split rows are made from FP32 rows).
 __global__ void k_abs2(const float2* __restrict__ F, long long n, float* __restrict__ F2)
 {
@@ -960,16 +992,19 @@ __global__ void k_fine_ab_rows(const float2* __restrict__ ab, int npix, int ldk,
 // The batch's distinct in-range orientations projected once (exact FP32 slices at coarse size,
 // XCD-aware order as k_local_zrows), shared by every particle whose range holds them. SPLIT 0:
 // float2 rows F (the FP32 path); SPLIT 1: the rows straight into the split operand (hi, lo and a
-// power-of-two row scale for FP16, as k_split_rows) plus |F|^2 for the n1 term.
+// power-of-two row scale for FP16, as k_split_rows) plus |F|^2 for the n1 term; SPLIT 2: BF16 halves
+// (no scale, chunk by chunk) plus |F|^2. Padding columns are written as zero.
 template <class H, int SPLIT>
 __global__ __launch_bounds__(256) void k_project_list(long long nu, const int* __restrict__ ulist, FineGeom g,
                                                       const float2* const* __restrict__ vols,
-                                                      const int* __restrict__ pads, const int2* __restrict__ pix,
-                                                      const unsigned char* __restrict__ inproj, int npix, int ldf,
+                                                      const int* __restrict__ pads, const int2* __restrict__ gather,
+                                                      int npix, int ldf,
                                                       float2* __restrict__ F, H* __restrict__ fh, H* __restrict__ fl,
-                                                      float* __restrict__ fs, int use_scale, float* __restrict__ F2)
+                                                      float* __restrict__ fs, float* __restrict__ F2)
 {
-    extern __shared__ float frow[];   // [2 ldf] (split only)
+    typedef typename Vec8<H>::type v8;
+    extern __shared__ __attribute__((aligned(16))) float frow[];   // the whole row, [2 ldf] (SPLIT 1 only)
+    __shared__ __attribute__((aligned(16))) float2 chunk[GATHER_CHUNK];   // (not SPLIT 1)
     __shared__ float redf[4];
     const long long per = (long long)gridDim.x / 8;
     const long long u = (long long)(blockIdx.x % 8) * per + blockIdx.x / 8;
@@ -978,34 +1013,41 @@ __global__ __launch_bounds__(256) void k_project_list(long long nu, const int* _
     int c, idir;
     fine_matrix(g, ulist[u], 0, A, &c, &idir);
     inv3(A, Ai);
-    const float a0 = (float)(Ai[0] * g.pf), a1 = (float)(Ai[1] * g.pf);
-    const float a2 = (float)(Ai[3] * g.pf), a3 = (float)(Ai[4] * g.pf);
-    const float a4 = (float)(Ai[6] * g.pf), a5 = (float)(Ai[7] * g.pf);
-    const float2* vol = vols[c];
-    const int pad = pads[c];
+    const float a[6] = {(float)(Ai[0] * g.pf), (float)(Ai[1] * g.pf), (float)(Ai[3] * g.pf),
+                        (float)(Ai[4] * g.pf), (float)(Ai[6] * g.pf), (float)(Ai[7] * g.pf)};
     float mx = 0.f;
-    for (int p = threadIdx.x; p < ldf; p += blockDim.x) {
-        float2 f = make_float2(0.f, 0.f);
-        if (p < npix && inproj[p]) {
-            const float x = (float)pix[p].x, y = (float)pix[p].y;
-            float2 v;
-            if (ref_sample(vol, pad, g.ref2d, a0 * x + a1 * y, a2 * x + a3 * y, a4 * x + a5 * y, &v)) f = v;
+    for (int base = 0; base < ldf; base += GATHER_CHUNK) {
+        float2* sf = (SPLIT == 1) ? reinterpret_cast<float2*>(frow) + base : chunk;
+        slice_chunk(vols[c], pads[c], g.ref2d, a, gather, npix, ldf, base, sf);
+        __syncthreads();
+        for (int q = 4 * threadIdx.x; q < min(GATHER_CHUNK, ldf - base); q += 1024) {   // ldf: a multiple of 32
+            const int p = base + q;
+            const float4 v0 = *reinterpret_cast<const float4*>(&sf[q]);
+            const float4 v1 = *reinterpret_cast<const float4*>(&sf[q + 2]);
+            const float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+            if (SPLIT)   // |F|^2 for the n1 term
+                *reinterpret_cast<float4*>(F2 + u * ldf + p) =
+                    make_float4(v[0] * v[0] + v[1] * v[1], v[2] * v[2] + v[3] * v[3], v[4] * v[4] + v[5] * v[5],
+                                v[6] * v[6] + v[7] * v[7]);
+            if (SPLIT == 2) {   // BF16: FP32's exponent range, no row scale: the halves straight out
+                v8 hi, lo;
+#pragma unroll
+                for (int k = 0; k < 8; k++) {
+                    hi[k] = (H)v[k];
+                    lo[k] = (H)(v[k] - (float)hi[k]);
+                }
+                *reinterpret_cast<v8*>(fh + u * 2 * ldf + 2 * p) = hi;
+                *reinterpret_cast<v8*>(fl + u * 2 * ldf + 2 * p) = lo;
+            } else if (SPLIT) {
+#pragma unroll
+                for (int k = 0; k < 8; k++) mx = fmaxf(mx, fabsf(v[k]));
+            } else {
+                float* d = reinterpret_cast<float*>(F + u * ldf + p);
+                *reinterpret_cast<float4*>(d) = v0;
+                *reinterpret_cast<float4*>(d + 4) = v1;
+            }
         }
-        if (SPLIT == 2) {   // BF16: FP32's exponent range, no row scale: the halves straight out
-            const H hx = (H)f.x, hy = (H)f.y;
-            fh[u * 2 * ldf + 2 * p] = hx;
-            fh[u * 2 * ldf + 2 * p + 1] = hy;
-            fl[u * 2 * ldf + 2 * p] = (H)(f.x - (float)hx);
-            fl[u * 2 * ldf + 2 * p + 1] = (H)(f.y - (float)hy);
-            F2[u * ldf + p] = f.x * f.x + f.y * f.y;
-        } else if (SPLIT) {
-            frow[2 * p] = f.x;
-            frow[2 * p + 1] = f.y;
-            mx = fmaxf(mx, fmaxf(fabsf(f.x), fabsf(f.y)));
-            F2[u * ldf + p] = f.x * f.x + f.y * f.y;   // |F|^2 for the n1 term
-        } else if (p < npix) {
-            F[u * ldf + p] = f;
-        }
+        __syncthreads();
     }
     if (SPLIT == 2) {
         if (threadIdx.x == 0) fs[u] = 1.f;
@@ -1013,23 +1055,22 @@ __global__ __launch_bounds__(256) void k_project_list(long long nu, const int* _
         for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
         if ((threadIdx.x & 63) == 0) redf[threadIdx.x >> 6] = mx;
         __syncthreads();
-        float sc = 1.f;
-        if (use_scale) {
-            mx = fmaxf(fmaxf(redf[0], redf[1]), fmaxf(redf[2], redf[3]));
-            int e = 0;
-            if (mx > 0.f) (void)frexpf(mx, &e);
-            sc = ldexpf(1.f, -e);
-            if (threadIdx.x == 0) fs[u] = ldexpf(1.f, e);
-        } else if (threadIdx.x == 0) {
-            fs[u] = 1.f;
-        }
+        mx = fmaxf(fmaxf(redf[0], redf[1]), fmaxf(redf[2], redf[3]));
+        int e = 0;
+        if (mx > 0.f) (void)frexpf(mx, &e);
+        const float sc = ldexpf(1.f, -e);
+        if (threadIdx.x == 0) fs[u] = ldexpf(1.f, e);
         const int Kc = 2 * ldf;
-        for (int k = threadIdx.x; k < Kc; k += blockDim.x) {
-            const float v = frow[k] * sc;
-            const H h = (H)v;
-            const H l = (H)(v - (float)h);
-            fh[u * Kc + k] = h;
-            fl[u * Kc + k] = l;
+        for (int k = 8 * threadIdx.x; k < Kc; k += 8 * blockDim.x) {
+            v8 hi, lo;
+#pragma unroll
+            for (int q = 0; q < 8; q++) {
+                const float v = frow[k + q] * sc;
+                hi[q] = (H)v;
+                lo[q] = (H)(v - (float)hi[q]);
+            }
+            *reinterpret_cast<v8*>(fh + u * Kc + k) = hi;
+            *reinterpret_cast<v8*>(fl + u * Kc + k) = lo;
         }
     }
 }
@@ -2186,6 +2227,7 @@ static void build_table(int size, int cur, const double* sigma2, int nsig2, int 
 {
     const int xs = size / 2 + 1, xc = cur / 2 + 1;
     t.size = size;
+    t.store = store;
     t.h_x.clear(); t.h_y.clear(); t.h_win.clear(); t.h_ires.clear(); t.h_minv.clear(); t.h_inproj.clear();
     const int rmo = xs - 1;
     std::vector<int> keep_ires;
@@ -2244,6 +2286,34 @@ static void build_table(int size, int cur, const double* sigma2, int nsig2, int 
     t.npix_pad = (int)round_up(t.npix, 32);   // K of the N1 GEMM: a multiple of the split GEMM's K step
 }
 
+// The sampling order of a diff2 table's pixels. They are stored by |frequency| (rings), in which
+// neighbours lie anywhere around the ring and a wave's 64 trilinear samples in as many bricks; within
+// each chunk of GATHER_CHUNK stored pixels (an annulus) this order goes through 4 x 4 patches, so that
+// the 16 samples of a load instruction (trilinear_quad) read few cache lines. The sampled values go through LDS to their stored places.
+static std::vector<int2> gather_order(const PassTables& t)
+{
+    std::vector<int2> g(t.npix);
+    std::vector<int> o(t.npix);
+    for (int i = 0; i < t.npix; i++) o[i] = i;
+    for (int c = 0; c < t.npix; c += GATHER_CHUNK) {
+        const int e = std::min(c + GATHER_CHUNK, t.npix);
+        std::sort(o.begin() + c, o.begin() + e, [&](int i, int j) {
+            for (int b = 5; b >= 2; b--) {   // patches of 32, 16, 8, 4 pixels a side
+                const int ya = t.h_y[i] >> b, yb = t.h_y[j] >> b, xa = t.h_x[i] >> b, xb = t.h_x[j] >> b;
+                if (ya != yb) return ya < yb;
+                if (xa != xb) return xa < xb;
+            }
+            return t.h_y[i] != t.h_y[j] ? t.h_y[i] < t.h_y[j] : t.h_x[i] < t.h_x[j];
+        });
+        for (int q = c, w = c; w < e; w += 64)
+            for (int k = 0; k < 16; k++)       // sample 16 i + k of a wave's 64 to lane 4 k + i
+                for (int i = w + k; i < std::min(w + 64, e); i += 16, q++)
+                    g[q] = make_int2((t.h_x[o[i]] & 0xffff) | (int)((unsigned)t.h_y[o[i]] << 16),
+                                     t.h_inproj[o[i]] ? o[i] - c : -1 - (o[i] - c));
+    }
+    return g;
+}
+
 static int upload_table(PassTables& t, hipStream_t st)
 {
     T2X_TRY(t.d_pix.ensure(sizeof(int2) * t.npix));
@@ -2258,6 +2328,12 @@ static int upload_table(PassTables& t, hipStream_t st)
     T2X_HIP(hipMemcpyAsync(t.d_minv.ptr, t.h_minv.data(), sizeof(float) * t.h_minv.size(), hipMemcpyHostToDevice, st));
     T2X_HIP(hipMemcpyAsync(t.d_ires.ptr, t.h_ires.data(), sizeof(int) * t.npix, hipMemcpyHostToDevice, st));
     T2X_HIP(hipMemcpyAsync(t.d_inproj.ptr, t.h_inproj.data(), t.npix, hipMemcpyHostToDevice, st));
+    std::vector<int2> gather;
+    if (!t.store) {
+        gather = gather_order(t);
+        T2X_TRY(t.d_gather.ensure(sizeof(int2) * t.npix));
+        T2X_HIP(hipMemcpyAsync(t.d_gather.ptr, gather.data(), sizeof(int2) * t.npix, hipMemcpyHostToDevice, st));
+    }
     // the frequency window of the pixels: x in [0, size/2], y in [-size/2, size/2]
     t.px_w = t.size / 2 + 1;
     t.py0 = t.size / 2;
@@ -2692,8 +2768,10 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
     if (!local_pairs && key != d->coarse_key) {
         T2X_TRY(d->coarse_B.ensure(sizeof(float) * O_pad * Kc));
         T2X_TRY(d->coarse_B2.ensure(sizeof(float) * O_pad * Kn));
-        T2X_HIP(hipMemsetAsync(d->coarse_B.ptr, 0, sizeof(float) * O_pad * Kc, st));
-        T2X_HIP(hipMemsetAsync(d->coarse_B2.ptr, 0, sizeof(float) * O_pad * Kn, st));
+        if (O_pad > O_all) {   // padding orientations
+            T2X_TRY(zero_async(d->coarse_B.as<float>() + (size_t)O_all * Kc, sizeof(float) * (O_pad - O_all) * Kc, st));
+            T2X_TRY(zero_async(d->coarse_B2.as<float>() + (size_t)O_all * Kn, sizeof(float) * (O_pad - O_all) * Kn, st));
+        }
         // the projection frames pf * A^-1 of the orientations (kept while the angles are the same)
         std::vector<double> akey = {pf, (double)Nd, (double)Npsi};
         akey.insert(akey.end(), S.rot.begin(), S.rot.begin() + Nd);
@@ -2714,10 +2792,9 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
             T2X_TRY(upload(d_Ai, Ai, st));
             d->coarse_Ai_key = akey;
         }
-        k_project_coarse<<<(unsigned)O_all, 256, 0, st>>>(
-            d_vols.as<const float2*>(), d_pads.as<int>(), d_Ai.as<float>(), (int)Norient,
-            tc.d_pix.as<int2>(), tc.d_inproj.as<unsigned char>(), tc.npix, d->coarse_B.as<float>(), Kc,
-            d->coarse_B2.as<float>(), Kn, ref2d);
+        k_project_coarse<<<(unsigned)round_up(O_all, 8), 256, 0, st>>>(
+            d_vols.as<const float2*>(), d_pads.as<int>(), d_Ai.as<float>(), (int)Norient, (int)O_all,
+            tc.d_gather.as<int2>(), tc.npix, d->coarse_B.as<float>(), Kc, d->coarse_B2.as<float>(), Kn, ref2d);
         T2X_HIP(hipGetLastError());
         if (prec != T2X_PREC_FP32) {
             T2X_TRY(d->coarse_Bh.ensure(sizeof(uint16_t) * O_pad * Kc));
@@ -3133,9 +3210,8 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
                 const unsigned ugrid = (unsigned)round_up(nu, 8);
                 if (prec == T2X_PREC_FP32) {
                     k_project_list<_Float16, 0><<<ugrid, 256, 0, st>>>(
-                        nu, d->lc_ulist.as<int>(), gc, d_vols.as<const float2*>(), d_pads.as<int>(), tc.d_pix.as<int2>(),
-                        tc.d_inproj.as<unsigned char>(), tc.npix, ldf, d->lc_F.as<float2>(), nullptr, nullptr, nullptr,
-                        0, nullptr);
+                        nu, d->lc_ulist.as<int>(), gc, d_vols.as<const float2*>(), d_pads.as<int>(), tc.d_gather.as<int2>(),
+                        tc.npix, ldf, d->lc_F.as<float2>(), nullptr, nullptr, nullptr, nullptr);
                 } else {
                     T2X_TRY(d->lc_fh.ensure(sizeof(uint16_t) * nu * Kc));
                     T2X_TRY(d->lc_fl.ensure(sizeof(uint16_t) * nu * Kc));
@@ -3144,18 +3220,16 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
                     if (prec == T2X_PREC_BF16X3) {
                         k_project_list<__bf16, 2><<<ugrid, 256, 0, st>>>(
                             nu, d->lc_ulist.as<int>(), gc, d_vols.as<const float2*>(), d_pads.as<int>(),
-                            tc.d_pix.as<int2>(), tc.d_inproj.as<unsigned char>(), tc.npix, ldf, nullptr,
-                            (__bf16*)d->lc_fh.ptr, (__bf16*)d->lc_fl.ptr, d->lc_fs.as<float>(), 0, d->lc_F2.as<float>());
+                            tc.d_gather.as<int2>(), tc.npix, ldf, nullptr,
+                            (__bf16*)d->lc_fh.ptr, (__bf16*)d->lc_fl.ptr, d->lc_fs.as<float>(), d->lc_F2.as<float>());
                     } else if (lds > kRowLdsMax) {
                         // rows beyond the LDS row buffer: FP32 slices in HBM, then the same split
                         // (row maximum, power-of-two scale, hi / lo) and |F|^2 from them: the same bits
                         T2X_TRY(d->lc_F.ensure(sizeof(float2) * nu * ldf));
                         k_project_list<_Float16, 0><<<ugrid, 256, 0, st>>>(
                             nu, d->lc_ulist.as<int>(), gc, d_vols.as<const float2*>(), d_pads.as<int>(),
-                            tc.d_pix.as<int2>(), tc.d_inproj.as<unsigned char>(), tc.npix, ldf, d->lc_F.as<float2>(),
-                            nullptr, nullptr, nullptr, 0, nullptr);
-                        // k_project_list leaves the padding columns npix..ldf-1 unwritten in FP32 rows
-                        k_zero_row_tails<<<(unsigned)nu, 64, 0, st>>>(d->lc_F.as<float2>(), tc.npix, ldf);
+                            tc.d_gather.as<int2>(), tc.npix, ldf, d->lc_F.as<float2>(), nullptr, nullptr, nullptr,
+                            nullptr);
                         T2X_HIP(hipGetLastError());
                         T2X_TRY(launch_split(prec, d->lc_F.as<float>(), Kc, Kc, (int)nu, (int)nu, d->lc_fh.ptr,
                                              d->lc_fl.ptr, Kc, d->lc_fs.as<float>(), st));
@@ -3164,8 +3238,8 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
                     } else
                         k_project_list<_Float16, 1><<<ugrid, 256, lds, st>>>(
                             nu, d->lc_ulist.as<int>(), gc, d_vols.as<const float2*>(), d_pads.as<int>(),
-                            tc.d_pix.as<int2>(), tc.d_inproj.as<unsigned char>(), tc.npix, ldf, nullptr,
-                            (_Float16*)d->lc_fh.ptr, (_Float16*)d->lc_fl.ptr, d->lc_fs.as<float>(), 1, d->lc_F2.as<float>());
+                            tc.d_gather.as<int2>(), tc.npix, ldf, nullptr,
+                            (_Float16*)d->lc_fh.ptr, (_Float16*)d->lc_fl.ptr, d->lc_fs.as<float>(), d->lc_F2.as<float>());
                 }
                 T2X_HIP(hipGetLastError());
                 // rows = the batch's (particle, orientation) pairs, columns = translations

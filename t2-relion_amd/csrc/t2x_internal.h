@@ -111,7 +111,7 @@ struct ClassVolumes {
     // projector
     int p_ref_dim = 0, p_pad = 0, p_rmax = 0;
     double p_pf = 0;
-    // 3D references: pad x pad x (pad/2+1) complex values in 4x4x4 bricks (vol_brick_index);
+    // 3D references: pad x pad x (pad/2+1) complex values in overlapping cells (vol_cell_index);
     // 2D references: the pad x (pad/2+1) plane, row-major
     float2* proj = nullptr;
     uint64_t proj_version = 0;
@@ -148,16 +148,21 @@ struct PassTables {
     int npix = 0;          // compact pixels with Minvsigma2 != 0
     int npix_pad = 0;      // padded to a multiple of 16
     int n_og = 1;          // optics groups: rows of the Minvsigma2 table
+    bool store = false;    // the weighted sums' table (every pixel, in window order)
     DevBuf d_pix;          // int2 (x, y) logical frequencies, y signed
     DevBuf d_win;          // int: index into the current-size window of each compact pixel
     DevBuf d_minv;         // float Minvsigma2 of each compact pixel, one row per optics group
     DevBuf d_ires;         // int shell index of each compact pixel
     DevBuf d_inproj;       // uchar: pixel inside the projected disc x^2+y^2 <= (size/2)^2
     int px_w = 0, py0 = 0, py_h = 0;   // frequency window (x, y + py0) of the pixels
+    // diff2 tables: the pixels in the order in which slices are sampled (gather_order), per place the
+    // pixel's x | y << 16 and its place in its chunk of GATHER_CHUNK pixels (-1 - place: not projected)
+    DevBuf d_gather;
     std::vector<int> h_x, h_y, h_win, h_ires;
     std::vector<float> h_minv;
     std::vector<unsigned char> h_inproj;
 };
+#define GATHER_CHUNK 1024
 
 struct Stats {
     t2x_stats s{};
@@ -334,51 +339,123 @@ __host__ __device__ inline void inv3(const double* A, double* R)
     for (int i = 0; i < 9; i++) R[i] /= tmp;
 }
 
+// A projector volume is stored in cells of 4 x 2 x 2 values (x, y, z; x fastest, then y, z), one cache
+// line of 128 bytes each, cells x fastest. In x they overlap by one value (cell c holds x = 3c .. 3c + 3),
+// so that x and x + 1 always lie in one cell, 16 bytes to load. A trilinear sample then touches 2.25
+// lines on average and needs four loads, whatever the slice orientation; disjoint bricks of 4 x 4 x 4
+// (a third less memory) had it touch 3.1 in eight loads.
+// Element (x, y, z) as the lower one of its pair; the copy in slot 3 of the cell before it, for x a
+// positive multiple of 3, is at vol_cell_index(x - 1, y, z) + 1.
+__host__ __device__ __forceinline__ size_t vol_cell_index(int x, int y, int z, int ncx, int ncy)
+{
+    return (((size_t)(z >> 1) * ncy + (y >> 1)) * ncx + x / 3) * 16 + ((z & 1) * 8 + (y & 1) * 4 + x % 3);
+}
+__host__ __device__ __forceinline__ int vol_cells_x(int pad) { return (pad / 2 + 1 + 2) / 3; }
+__host__ __device__ __forceinline__ int vol_cells_y(int pad) { return (pad + 1) / 2; }
+
+__host__ __device__ __forceinline__ size_t vol_cell_elems(int pad)
+{
+    return (size_t)vol_cells_x(pad) * vol_cells_y(pad) * vol_cells_y(pad) * 16;
+}
+
 // Trilinear sample of the half-complex projector volume at logical (xp, yp, zp) (already
 // multiplied by the padding factor), with the Friedel flip of projector.cpp:583-640.
 // Returns false where the reference skips the pixel (outside the box).
-// Element (x, y, z) of a projector volume stored in 4x4x4 bricks (x fastest inside a brick,
-// bricks x fastest): the 8 corners of a trilinear sample lie in at most 8 bricks of 512 bytes
-// whatever the slice orientation, instead of 4 rows and 2 planes far apart.
-__host__ __device__ __forceinline__ size_t vol_brick_index(int x, int y, int z, int nbx, int nby)
+// A sample's address and the interpolation are apart, so that the lanes of a quad can share a sample's
+// loads. The offset of (x, y, z) is a sum of one term per axis, so the other (y, z) corners are the
+// lower one plus a step per axis (32-bit: within one layer of cells).
+struct TriPos {
+    size_t o;                // offset of the lower corner
+    unsigned sy, sz;         // steps to y + 1, z + 1
+    float fx, fy, fz;
+    bool neg, ok;
+};
+
+__device__ __forceinline__ TriPos trilinear_pos(int pad, float xp, float yp, float zp)
 {
-    return ((((size_t)(z >> 2) * nby + (y >> 2)) * nbx + (x >> 2)) << 6) + (((z & 3) * 4 + (y & 3)) * 4 + (x & 3));
+    const int xdim = pad / 2 + 1, h = pad / 2;
+    TriPos t;
+    t.neg = xp < 0.f;
+    if (t.neg) { xp = -xp; yp = -yp; zp = -zp; }
+    const float fx0 = floorf(xp), fy0 = floorf(yp), fz0 = floorf(zp);
+    const int x0 = (int)fx0, y0 = (int)fy0 + h, z0 = (int)fz0 + h;
+    t.fx = xp - fx0;
+    t.fy = yp - fy0;
+    t.fz = zp - fz0;
+    t.ok = !(x0 < 0 || x0 + 1 >= xdim || y0 < 0 || y0 + 1 >= pad || z0 < 0 || z0 + 1 >= pad);
+    // positions outside read the first voxels (their value is not used)
+    const unsigned x = t.ok ? x0 : 0, y = t.ok ? y0 : 0, z = t.ok ? z0 : 0;
+    const unsigned row = (unsigned)vol_cells_x(pad) * 16, layer = row * (unsigned)vol_cells_y(pad), cx = x / 3;
+    t.o = (size_t)(z >> 1) * layer + ((y >> 1) * row + cx * 13 + x + (z & 1) * 8 + (y & 1) * 4);
+    t.sy = (y & 1) ? row - 4 : 4;
+    t.sz = (z & 1) ? layer - 8 : 8;
+    return t;
 }
 
-__host__ __device__ __forceinline__ size_t vol_brick_elems(int pad)
+// Two x neighbours, one 16-byte load (8-byte aligned).
+struct VolPair { float2 a, b; };
+__device__ __forceinline__ VolPair vol_pair(const float2* v)
 {
-    const size_t nbx = (pad / 2 + 1 + 3) / 4, nb = (pad + 3) / 4;
-    return nbx * nb * nb * 64;
+    typedef float float4u __attribute__((ext_vector_type(4), aligned(8)));
+    const float4u q = *reinterpret_cast<const float4u*>(v);
+    return {make_float2(q.x, q.y), make_float2(q.z, q.w)};
 }
 
 __device__ __forceinline__ bool trilinear_sample(const float2* __restrict__ vol, int pad, float xp,
                                                  float yp, float zp, float2* out)
 {
-    const int xdim = pad / 2 + 1, h = pad / 2;
-    bool neg = xp < 0.f;
-    if (neg) { xp = -xp; yp = -yp; zp = -zp; }
-    float fx0 = floorf(xp), fy0 = floorf(yp), fz0 = floorf(zp);
-    int x0 = (int)fx0, y0 = (int)fy0 + h, z0 = (int)fz0 + h;
-    float fx = xp - fx0, fy = yp - fy0, fz = zp - fz0;
-    if (x0 < 0 || x0 + 1 >= xdim || y0 < 0 || y0 + 1 >= pad || z0 < 0 || z0 + 1 >= pad) return false;
-    const int nbx = (xdim + 3) / 4, nby = (pad + 3) / 4;
-    float2 d000 = vol[vol_brick_index(x0, y0, z0, nbx, nby)], d001 = vol[vol_brick_index(x0 + 1, y0, z0, nbx, nby)];
-    float2 d010 = vol[vol_brick_index(x0, y0 + 1, z0, nbx, nby)];
-    float2 d011 = vol[vol_brick_index(x0 + 1, y0 + 1, z0, nbx, nby)];
-    float2 d100 = vol[vol_brick_index(x0, y0, z0 + 1, nbx, nby)];
-    float2 d101 = vol[vol_brick_index(x0 + 1, y0, z0 + 1, nbx, nby)];
-    float2 d110 = vol[vol_brick_index(x0, y0 + 1, z0 + 1, nbx, nby)];
-    float2 d111 = vol[vol_brick_index(x0 + 1, y0 + 1, z0 + 1, nbx, nby)];
+    const TriPos t = trilinear_pos(pad, xp, yp, zp);
+    if (!t.ok) return false;
+    const float2* v = vol + t.o;
+    const VolPair p00 = vol_pair(v), p10 = vol_pair(v + t.sy), p01 = vol_pair(v + t.sz), p11 = vol_pair(v + (t.sy + t.sz));
+    const float2 d000 = p00.a, d001 = p00.b, d010 = p10.a, d011 = p10.b;
+    const float2 d100 = p01.a, d101 = p01.b, d110 = p11.a, d111 = p11.b;
+    const float fx = t.fx, fy = t.fy, fz = t.fz;
     float2 dx00 = make_float2(d000.x + (d001.x - d000.x) * fx, d000.y + (d001.y - d000.y) * fx);
     float2 dx01 = make_float2(d100.x + (d101.x - d100.x) * fx, d100.y + (d101.y - d100.y) * fx);
     float2 dx10 = make_float2(d010.x + (d011.x - d010.x) * fx, d010.y + (d011.y - d010.y) * fx);
     float2 dx11 = make_float2(d110.x + (d111.x - d110.x) * fx, d110.y + (d111.y - d110.y) * fx);
     float2 dxy0 = make_float2(dx00.x + (dx10.x - dx00.x) * fy, dx00.y + (dx10.y - dx00.y) * fy);
     float2 dxy1 = make_float2(dx01.x + (dx11.x - dx01.x) * fy, dx01.y + (dx11.y - dx01.y) * fy);
-    float2 v = make_float2(dxy0.x + (dxy1.x - dxy0.x) * fz, dxy0.y + (dxy1.y - dxy0.y) * fz);
-    if (neg) v.y = -v.y;
-    *out = v;
+    out->x = dxy0.x + (dxy1.x - dxy0.x) * fz;
+    out->y = dxy0.y + (dxy1.y - dxy0.y) * fz;
+    if (t.neg) out->y = -out->y;
     return true;
+}
+
+// Value of quad lane P0 .. P3 in lanes 0 .. 3 of each quad (all lanes active).
+template <int P0, int P1, int P2, int P3>
+__device__ __forceinline__ unsigned quad_perm(unsigned v)
+{
+    return __builtin_amdgcn_mov_dpp(v, P0 | P1 << 2 | P2 << 4 | P3 << 6, 0xf, 0xf, true);
+}
+template <int P0, int P1, int P2, int P3>
+__device__ __forceinline__ float quad_perm(float v)
+{
+    return __uint_as_float(quad_perm<P0, P1, P2, P3>(__float_as_uint(v)));
+}
+
+// The sample of quad lane I's position, taken by the quad together: each lane loads one (y, z) corner's
+// two x neighbours and interpolates them in x, the lanes then in y and z across the quad: the arithmetic
+// of trilinear_sample (the result, before the conjugation, in all four lanes). A load instruction then
+// reads 16 whole samples instead of one corner pair of 64: the corners of a sample lie in two or three
+// cache lines, which the one-thread form had lost from the L1 before it came to the next corner.
+template <int I>
+__device__ __forceinline__ float2 trilinear_quad(const float2* __restrict__ vol, const TriPos& t, unsigned ymask,
+                                                 unsigned zmask)
+{
+    const unsigned lo = quad_perm<I, I, I, I>((unsigned)t.o), hi = quad_perm<I, I, I, I>((unsigned)(t.o >> 32));
+    const unsigned sy = quad_perm<I, I, I, I>(t.sy) & ymask, sz = quad_perm<I, I, I, I>(t.sz) & zmask;
+    const float fx = quad_perm<I, I, I, I>(t.fx), fy = quad_perm<I, I, I, I>(t.fy), fz = quad_perm<I, I, I, I>(t.fz);
+    const VolPair p = vol_pair(vol + (((size_t)hi << 32 | lo) + (sy + sz)));
+    const float2 d0 = p.a, d1 = p.b;
+    const float2 dx = make_float2(d0.x + (d1.x - d0.x) * fx, d0.y + (d1.y - d0.y) * fx);
+    const float2 y0 = make_float2(quad_perm<0, 0, 2, 2>(dx.x), quad_perm<0, 0, 2, 2>(dx.y));
+    const float2 y1 = make_float2(quad_perm<1, 1, 3, 3>(dx.x), quad_perm<1, 1, 3, 3>(dx.y));
+    const float2 dy = make_float2(y0.x + (y1.x - y0.x) * fy, y0.y + (y1.y - y0.y) * fy);
+    const float2 z0 = make_float2(quad_perm<0, 0, 0, 0>(dy.x), quad_perm<0, 0, 0, 0>(dy.y));
+    const float2 z1 = make_float2(quad_perm<2, 2, 2, 2>(dy.x), quad_perm<2, 2, 2, 2>(dy.y));
+    return make_float2(z0.x + (z1.x - z0.x) * fz, z0.y + (z1.y - z0.y) * fz);
 }
 
 // Bilinear sample of a half-complex 2D reference ([pad][pad/2+1], y centred) at logical
