@@ -379,29 +379,159 @@ __global__ __launch_bounds__(256) void k_project_coarse(const float2* const* __r
     }
 }
 
-// Image side of the coarse GEMM: A[(b,t)][2p..] = minv ctf X_t and A1[b][p] = minv ctf^2 / 2,
-// with X_t = X * exp(-2 pi i (x sx + y sy)/N) (shiftImageInFourierTransform, fftw.cpp:842-930).
+// Image side of the coarse GEMM: row (b, t) = minv ctf X_t, re/im interleaved, and A1[b][p] =
+// minv ctf^2 / 2, with X_t = X * exp(-2 pi i (x sx + y sy)/N) (shiftImageInFourierTransform,
+// fftw.cpp:842-930). FORM 0: FP32 rows in hi; 1: FP16 halves hi and lo with a power-of-two row scale (as
+// k_split_rows); 2: BF16 halves, no scale. Padding columns, and the padding rows M .. rows - 1, are zero.
+//
+// Bound by the address units: the gathers from the particle's window, the phase table (8 bytes a pixel
+// and pass, from the L2) and the rows (8 bytes a pixel). A workgroup takes tg translations of one
+// particle and gathers each IMG_CHUNK pixels of its window once for up to IMG_TG rows (rows of one chunk:
+// once for all tg) into LDS; a thread takes four pixels, so that loads and stores are 16 bytes; `width`
+// threads (whole waves, by the length of a row) share a row, 256 / width rows at a time. FP16 forms its
+// values twice, first for the row maxima: cheaper than a row buffer, and rows may have any length. Rows
+// of 10,000 pixels in BF16 (3000 particles of 113 translations): 25 -> 12.1 ms; of 1,450 in FP16 (8192
+// particles of 88): 5.3 -> 2.9 ms (gathered by every row group and pass: 3.6).
+#define IMG_TG 8
+#define IMG_CHUNK 2048
+template <class H, int FORM>
 __global__ __launch_bounds__(256) void k_coarse_imgside(const float2* __restrict__ Fimg,
                                                         const float* __restrict__ Fctf, int Pw,
-                                                        const int* __restrict__ win,
-                                                        const float* __restrict__ minv, int npix,
-                                                        const PartScalars* __restrict__ ps,
-                                                        const float2* __restrict__ ab, int T,
-                                                        float* __restrict__ A, long long lda,
-                                                        float* __restrict__ A1, long long lda1)
+                                                        const int* __restrict__ win, const float* __restrict__ minv,
+                                                        int npix, const PartScalars* __restrict__ ps,
+                                                        const float2* __restrict__ ab, int B, int T, long long rows,
+                                                        int Kc, int tg, int width, void* __restrict__ hi_,
+                                                        H* __restrict__ lo, float* __restrict__ inv_scale,
+                                                        float* __restrict__ A1)
 {
-    const int b = blockIdx.y, t = blockIdx.x;
+    typedef typename Vec8<H>::type v8;
+    __shared__ __attribute__((aligned(16))) float2 xs[IMG_CHUNK];
+    __shared__ __attribute__((aligned(16))) float ss[IMG_CHUNK];
+    __shared__ float red[IMG_TG][4];
+    float* out = static_cast<float*>(hi_);
+    H* hi = static_cast<H*>(hi_);
+    const int ng = (T + tg - 1) / tg, Kn = Kc / 2;
+    const long long blk = blockIdx.x;
+    if (blk >= (long long)B * ng) {   // padding rows
+        const long long r0 = (long long)B * T + (blk - (long long)B * ng) * tg;
+        for (long long r = r0; r < min(r0 + tg, rows); r++) {
+            for (int k = 8 * threadIdx.x; k < Kc; k += 8 * 256) {
+                if (FORM == 0) {
+                    *reinterpret_cast<float4*>(out + r * Kc + k) = make_float4(0.f, 0.f, 0.f, 0.f);
+                    *reinterpret_cast<float4*>(out + r * Kc + k + 4) = make_float4(0.f, 0.f, 0.f, 0.f);
+                } else {
+                    *reinterpret_cast<v8*>(hi + r * Kc + k) = v8{};
+                    *reinterpret_cast<v8*>(lo + r * Kc + k) = v8{};
+                }
+            }
+            if (FORM && threadIdx.x == 0) inv_scale[r] = 1.f;
+        }
+        return;
+    }
+    const int b = (int)(blk / ng), tb = (int)(blk - (long long)b * ng) * tg, te = min(tb + tg, T);
+    const int step = 256 / width, sub = threadIdx.x / width, l = threadIdx.x - sub * width;
     const float* mv = minv + (size_t)ps[b].og * npix;
-    for (int p = threadIdx.x; p < npix; p += blockDim.x) {
-        const size_t w = (size_t)b * Pw + win[p];
-        float2 x = Fimg[w];
-        float ctf = Fctf[w], m = mv[p];
-        float s = m * ctf;
-        float2 sh = ab[(size_t)t * npix + p];
-        float xr = x.x * sh.x - x.y * sh.y, xi = x.x * sh.y + x.y * sh.x;
-        A[((size_t)b * T + t) * lda + 2 * p] = s * xr;
-        A[((size_t)b * T + t) * lda + 2 * p + 1] = s * xi;
-        if (t == 0) A1[(size_t)b * lda1 + p] = 0.5f * m * ctf * ctf;
+    int staged = -1;   // the chunk in LDS
+    for (int t0 = tb; t0 < te; t0 += IMG_TG) {
+        const int nt = min(IMG_TG, te - t0);
+        float sc[IMG_TG];
+#pragma unroll
+        for (int j = 0; j < IMG_TG; j++) sc[j] = 0.f;
+        for (int pass = (FORM == 1 ? 0 : 1); pass < 2; pass++) {
+            for (int base = 0; base < Kn; base += IMG_CHUNK) {
+                const int n = min(IMG_CHUNK, Kn - base);
+                if (staged != base) {
+                    __syncthreads();
+                    for (int q = threadIdx.x; q < n; q += 256) {
+                        const int p = base + q;
+                        float2 x = make_float2(0.f, 0.f);
+                        float s = 0.f, a1 = 0.f;
+                        if (p < npix) {
+                            const size_t w = (size_t)b * Pw + win[p];
+                            const float ctf = Fctf[w], m = mv[p];
+                            x = Fimg[w];
+                            s = m * ctf;
+                            a1 = 0.5f * m * ctf * ctf;
+                        }
+                        xs[q] = x;
+                        ss[q] = s;
+                        if (t0 == 0) A1[(size_t)b * Kn + p] = a1;
+                    }
+                    staged = base;
+                    __syncthreads();
+                }
+                for (int q = 4 * l; q < n; q += 4 * width) {
+                    const int p = base + q;
+                    const float4 x01 = *reinterpret_cast<const float4*>(&xs[q]), x23 = *reinterpret_cast<const float4*>(&xs[q + 2]);
+                    const float4 s4 = *reinterpret_cast<const float4*>(&ss[q]);
+                    const float xr[4] = {x01.x, x01.z, x23.x, x23.z}, xi[4] = {x01.y, x01.w, x23.y, x23.w};
+                    const float s[4] = {s4.x, s4.y, s4.z, s4.w};
+#pragma unroll
+                    for (int j = 0; j < IMG_TG; j++) {
+                        const int t = sub + j * step;
+                        if (t >= nt) break;
+                        const float2* sh = ab + (size_t)(t0 + t) * npix + p;
+                        VolPair e01{}, e23{};
+                        if (p + 4 <= npix) {
+                            e01 = vol_pair(sh);
+                            e23 = vol_pair(sh + 2);
+                        } else if (p < npix) {
+                            e01.a = sh[0];
+                            if (p + 1 < npix) e01.b = sh[1];
+                            if (p + 2 < npix) e23.a = sh[2];
+                        }
+                        const float2 e[4] = {e01.a, e01.b, e23.a, e23.b};
+                        float v[8];
+#pragma unroll
+                        for (int k = 0; k < 4; k++) {
+                            const float yr = xr[k] * e[k].x - xi[k] * e[k].y, yi = xr[k] * e[k].y + xi[k] * e[k].x;
+                            v[2 * k] = s[k] * yr;
+                            v[2 * k + 1] = s[k] * yi;
+                        }
+                        if (pass == 0) {
+#pragma unroll
+                            for (int k = 0; k < 8; k++) sc[j] = fmaxf(sc[j], fabsf(v[k]));
+                            continue;
+                        }
+                        const size_t o = ((size_t)b * T + t0 + t) * Kc + 2 * p;
+                        if (FORM == 0) {
+                            *reinterpret_cast<float4*>(out + o) = make_float4(v[0], v[1], v[2], v[3]);
+                            *reinterpret_cast<float4*>(out + o + 4) = make_float4(v[4], v[5], v[6], v[7]);
+                        } else {
+                            v8 h, d;
+#pragma unroll
+                            for (int k = 0; k < 8; k++) {
+                                const float u = FORM == 1 ? v[k] * sc[j] : v[k];
+                                h[k] = (H)u;
+                                d[k] = (H)(u - (float)h[k]);
+                            }
+                            *reinterpret_cast<v8*>(hi + o) = h;
+                            *reinterpret_cast<v8*>(lo + o) = d;
+                        }
+                    }
+                }
+            }
+            if (pass == 0) {
+                __syncthreads();   // the last group's maxima have been read
+#pragma unroll
+                for (int j = 0; j < IMG_TG; j++) {
+                    for (int o = 32; o > 0; o >>= 1) sc[j] = fmaxf(sc[j], __shfl_xor(sc[j], o));
+                    if ((threadIdx.x & 63) == 0) red[j][threadIdx.x >> 6] = sc[j];
+                }
+                __syncthreads();
+#pragma unroll
+                for (int j = 0; j < IMG_TG; j++) {
+                    float mx = 0.f;
+                    for (int w = sub * width / 64; w < (sub + 1) * width / 64; w++) mx = fmaxf(mx, red[j][w]);
+                    int e = 0;
+                    if (mx > 0.f) (void)frexpf(mx, &e);
+                    sc[j] = ldexpf(1.f, -e);
+                    const int t = sub + j * step;
+                    if (l == 0 && t < nt) inv_scale[(size_t)b * T + t0 + t] = ldexpf(1.f, e);
+                }
+            }
+        }
+        if (FORM == 2 && (int)threadIdx.x < nt) inv_scale[(size_t)b * T + t0 + threadIdx.x] = 1.f;
     }
 }
 
@@ -461,75 +591,6 @@ __global__ __launch_bounds__(128) void k_prior_t(const PartScalars* __restrict__
     __syncthreads();
     const double m = s_mean;
     for (int t = threadIdx.x; t < T; t += blockDim.x) prior_t[(size_t)b * T + t] = (m > 0.) ? pt[t] / m : pt[t];
-}
-
-// k_coarse_imgside followed by the split of each row into hi + lo halves (k_split_rows), fused:
-// one workgroup per GEMM row (particle b, translation t; rows >= M are zero). FP16 (use_scale):
-// the row's values kept in LDS between the max-abs reduction and the scaled split; BF16: no
-// scale, the halves written as the values are formed (no LDS). The FP32 A matrix is neither
-// cleared, written nor read back. Same arithmetic as the two kernels, so the same bits.
-template <class H>
-__global__ __launch_bounds__(256) void k_coarse_imgside_split(const float2* __restrict__ Fimg,
-                                                              const float* __restrict__ Fctf, int Pw,
-                                                              const int* __restrict__ win,
-                                                              const float* __restrict__ minv, int npix,
-                                                              const PartScalars* __restrict__ ps,
-                                                              const float2* __restrict__ ab, int T, int M, int Kc,
-                                                              H* __restrict__ hi, H* __restrict__ lo,
-                                                              float* __restrict__ inv_scale, int use_scale,
-                                                              float* __restrict__ A1, long long lda1)
-{
-    extern __shared__ float row[];   // [Kc]
-    __shared__ float red[4];
-    const int r = blockIdx.x;
-    const bool valid = r < M;
-    const int b = valid ? r / T : 0, t = valid ? r - b * T : 0;
-    const float* mv = minv + (valid ? (size_t)ps[b].og * npix : 0);
-    float mx = 0.f;
-    for (int p = threadIdx.x; p < Kc / 2; p += blockDim.x) {
-        float vr = 0.f, vi = 0.f;
-        if (valid && p < npix) {
-            const size_t w = (size_t)b * Pw + win[p];
-            const float2 x = Fimg[w];
-            const float ctf = Fctf[w], m = mv[p];
-            const float s = m * ctf;
-            const float2 sh = ab[(size_t)t * npix + p];
-            const float xr = x.x * sh.x - x.y * sh.y, xi = x.x * sh.y + x.y * sh.x;
-            vr = s * xr;
-            vi = s * xi;
-            if (t == 0) A1[(size_t)b * lda1 + p] = 0.5f * m * ctf * ctf;
-        }
-        if (!use_scale) {   // BF16: no row scale, so no row buffer: the halves straight out
-            const H hr = (H)vr, hi_ = (H)vi;
-            hi[(size_t)r * Kc + 2 * p] = hr;
-            hi[(size_t)r * Kc + 2 * p + 1] = hi_;
-            lo[(size_t)r * Kc + 2 * p] = (H)(vr - (float)hr);
-            lo[(size_t)r * Kc + 2 * p + 1] = (H)(vi - (float)hi_);
-            continue;
-        }
-        row[2 * p] = vr;
-        row[2 * p + 1] = vi;
-        mx = fmaxf(mx, fmaxf(fabsf(vr), fabsf(vi)));
-    }
-    if (!use_scale) {
-        if (threadIdx.x == 0) inv_scale[r] = 1.f;
-        return;
-    }
-    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
-    __syncthreads();
-    mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-    int e = 0;
-    if (mx > 0.f) (void)frexpf(mx, &e);
-    const float sc = ldexpf(1.f, -e);
-    if (threadIdx.x == 0) inv_scale[r] = ldexpf(1.f, e);
-    for (int k = threadIdx.x; k < Kc; k += blockDim.x) {
-        const float v = row[k] * sc;
-        const H h = (H)v;
-        const H l = (H)(v - (float)h);
-        hi[(size_t)r * Kc + k] = h;
-        lo[(size_t)r * Kc + k] = l;
-    }
 }
 
 // ------------------------------------------------------------------------------------------
@@ -2389,38 +2450,35 @@ static int ensure_fft(Device* d, int N, int batch)
     return T2X_OK;
 }
 
-// The image side of the split GEMMs: rows (b, t) < M of minv ctf X_t as hi / lo halves with their
-// row scales (rows M..rows-1 zero), and A1 = minv ctf^2 / 2 for the N1 term. Rows that fit the
-// LDS row buffer go through k_coarse_imgside_split; longer ones (coarse images beyond 8,192
-// pixels) through an FP32 matrix in HBM and k_split_rows, with the same bits.
-static int imgside_split(Device* d, int prec, const PassTables& tc, const PartScalars* d_ps, int Pw, int T, int B,
-                         long long rows, int Kc, int Kn, hipStream_t st)
+// Image-side operand of the coarse GEMMs, `rows` rows (those past B T zero): FP32 rows in d->A, or hi /
+// lo halves and row scales in d->Ah, d->Al, d->As; A1 for the B particles. Translations are grouped
+// where that leaves at least eight workgroups a compute unit.
+static int imgside(Device* d, int prec, const PassTables& tc, const PartScalars* d_ps, int Pw, int T, int B,
+                   long long rows, int Kc, hipStream_t st)
 {
     const long long M = (long long)B * T;
-    const size_t lds = sizeof(float) * Kc;
-    if (lds <= kRowLdsMax || prec == T2X_PREC_BF16X3) {
-        if (prec == T2X_PREC_BF16X3)   // no row scale: the kernel needs no row buffer
-            k_coarse_imgside_split<__bf16><<<(unsigned)rows, 256, 0, st>>>(
-                d->Fimg_cur.as<float2>(), d->Fctf_cur.as<float>(), Pw, tc.d_win.as<int>(), tc.d_minv.as<float>(),
-                tc.npix, d_ps, d->ab_coarse.as<float2>(), T, (int)M, Kc, (__bf16*)d->Ah.ptr, (__bf16*)d->Al.ptr,
-                d->As.as<float>(), 0, d->A1.as<float>(), Kn);
-        else
-            k_coarse_imgside_split<_Float16><<<(unsigned)rows, 256, lds, st>>>(
-                d->Fimg_cur.as<float2>(), d->Fctf_cur.as<float>(), Pw, tc.d_win.as<int>(), tc.d_minv.as<float>(),
-                tc.npix, d_ps, d->ab_coarse.as<float2>(), T, (int)M, Kc, (_Float16*)d->Ah.ptr, (_Float16*)d->Al.ptr,
-                d->As.as<float>(), 1, d->A1.as<float>(), Kn);
-        T2X_HIP(hipGetLastError());
-        return T2X_OK;
-    }
-    T2X_TRY(d->A.ensure(sizeof(float) * rows * Kc));
-    T2X_TRY(zero_async(d->A.ptr, sizeof(float) * rows * Kc, st));
-    if (B > 0) {
-        k_coarse_imgside<<<dim3((unsigned)T, (unsigned)B), 256, 0, st>>>(
-            d->Fimg_cur.as<float2>(), d->Fctf_cur.as<float>(), Pw, tc.d_win.as<int>(), tc.d_minv.as<float>(), tc.npix,
-            d_ps, d->ab_coarse.as<float2>(), T, d->A.as<float>(), Kc, d->A1.as<float>(), Kn);
-        T2X_HIP(hipGetLastError());
-    }
-    return launch_split(prec, d->A.as<float>(), Kc, Kc, (int)rows, (int)M, d->Ah.ptr, d->Al.ptr, Kc, d->As.as<float>(), st);
+    const int tg = (int)std::min<long long>(4 * IMG_TG, std::max<long long>(1, M / 2048));
+    int width = 256;   // the widest that leaves the fewest lanes without a pixel
+    for (int w = 128; w >= 64; w /= 2)
+        if (round_up(Kc / 2, 4 * w) < round_up(Kc / 2, 4 * width)) width = w;
+    const unsigned grid = (unsigned)((long long)B * ((T + tg - 1) / tg) + (rows - M + tg - 1) / tg);
+    if (grid == 0) return T2X_OK;
+    const float2 *F = d->Fimg_cur.as<float2>(), *ab = d->ab_coarse.as<float2>();
+    const float *ctf = d->Fctf_cur.as<float>(), *minv = tc.d_minv.as<float>();
+    const int* win = tc.d_win.as<int>();
+    if (prec == T2X_PREC_FP32)
+        k_coarse_imgside<_Float16, 0><<<grid, 256, 0, st>>>(F, ctf, Pw, win, minv, tc.npix, d_ps, ab, B, T, rows, Kc, tg,
+                                                            width, d->A.ptr, nullptr, nullptr, d->A1.as<float>());
+    else if (prec == T2X_PREC_BF16X3)
+        k_coarse_imgside<__bf16, 2><<<grid, 256, 0, st>>>(F, ctf, Pw, win, minv, tc.npix, d_ps, ab, B, T, rows, Kc, tg,
+                                                          width, d->Ah.ptr, (__bf16*)d->Al.ptr, d->As.as<float>(),
+                                                          d->A1.as<float>());
+    else
+        k_coarse_imgside<_Float16, 1><<<grid, 256, 0, st>>>(F, ctf, Pw, win, minv, tc.npix, d_ps, ab, B, T, rows, Kc, tg,
+                                                            width, d->Ah.ptr, (_Float16*)d->Al.ptr, d->As.as<float>(),
+                                                            d->A1.as<float>());
+    T2X_HIP(hipGetLastError());
+    return T2X_OK;
 }
 
 struct EventTimer {
@@ -3274,7 +3332,7 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
                     T2X_TRY(d->Al.ensure(sizeof(uint16_t) * wrows * Kc));
                     T2X_TRY(d->As.ensure(sizeof(float) * wrows));
                     T2X_TRY(d->A1.ensure(sizeof(float) * B * Kn));
-                    T2X_TRY(imgside_split(d, prec, tc, d_ps, Pw, (int)T, B, wrows, Kc, Kn, st));
+                    T2X_TRY(imgside(d, prec, tc, d_ps, Pw, (int)T, B, wrows, Kc, st));
                     k_local_n1<<<(unsigned)((rows + 3) / 4), 256, 0, st>>>(
                         B, rows, d->lc_orient_off.as<long long>(), d->lc_rowu.as<int>(), d->lc_F2.as<float>(), ldf,
                         d->A1.as<float>(), Kn, tc.npix, d->lc_n1.as<double>());
@@ -3324,22 +3382,13 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
             const int rowmin_ld = (int)(O_pad / 64);
             DevBuf& d_rowmin = d->minb;
             T2X_TRY(d_rowmin.ensure(sizeof(float) * M_pad * rowmin_ld));
-            T2X_TRY(zero_async(d->A1.ptr, sizeof(float) * B_pad * Kn, st));
-            if (prec == T2X_PREC_FP32) {
-                T2X_TRY(zero_async(d->A.ptr, sizeof(float) * M_pad * Kc, st));
-                dim3 grid((unsigned)T, (unsigned)B);
-                k_coarse_imgside<<<grid, 256, 0, st>>>(d->Fimg_cur.as<float2>(), d->Fctf_cur.as<float>(), Pw,
-                                                       tc.d_win.as<int>(), tc.d_minv.as<float>(), tc.npix, d_ps,
-                                                       d->ab_coarse.as<float2>(), (int)T, d->A.as<float>(), Kc,
-                                                       d->A1.as<float>(), Kn);
-                T2X_HIP(hipGetLastError());
-            } else {
-                // the image side straight into the split operand (hi, lo, per-row scale)
+            if (B_pad > B) T2X_TRY(zero_async(d->A1.as<float>() + (size_t)B * Kn, sizeof(float) * (B_pad - B) * Kn, st));
+            if (prec != T2X_PREC_FP32) {
                 T2X_TRY(d->Ah.ensure(sizeof(uint16_t) * M_pad * Kc));
                 T2X_TRY(d->Al.ensure(sizeof(uint16_t) * M_pad * Kc));
                 T2X_TRY(d->As.ensure(sizeof(float) * M_pad));
-                T2X_TRY(imgside_split(d, prec, tc, d_ps, Pw, (int)T, B, M_pad, Kc, Kn, st));
             }
+            T2X_TRY(imgside(d, prec, tc, d_ps, Pw, (int)T, B, M_pad, Kc, st));
             {
                 EpiParams ep{};
                 ep.C = d->N1.as<float>();
