@@ -129,6 +129,8 @@ extern "C" int t2x_device_close(t2x_device* h)
     if (d->fft_plan) (void)hipfftDestroy(d->fft_plan);
     if (d->noise_plan) (void)hipfftDestroy(d->noise_plan);
     if (d->prop_plan) (void)hipfftDestroy(d->prop_plan);
+    for (hipfftHandle pl : d->recon.plan)
+        if (pl) (void)hipfftDestroy(pl);
     d->net.reset();
     for (auto& e : d->ev) (void)hipEventDestroy(e);
     (void)hipStreamDestroy(d->stream);

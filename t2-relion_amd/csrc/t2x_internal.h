@@ -180,6 +180,18 @@ struct PruneBufs {
 struct Device;
 void destroy_graph(Device* d);
 
+// What the reconstruction and the FSC keep between calls (used under the device lock, freed with the
+// device): one arena for all their buffers, up to kReconKeep bytes, and one FFT plan of each kind with
+// the arena as its work area. Creating the plans and allocating afresh had been 35 of the 38 ms of a
+// 64-box iteration's two maps and their FSC.
+struct ReconWork {
+    DevBuf arena;
+    HostBuf host;               // page-locked staging
+    hipfftHandle plan[2] = {0, 0};   // complex to real (reconstruction), real to complex (FSC)
+    int plan_n[2] = {0, 0};
+    size_t plan_work[2] = {0, 0};
+};
+
 struct Device {
     int id = 0;
     hipStream_t stream = nullptr;
@@ -216,6 +228,7 @@ struct Device {
     std::vector<double> ab_key;
     DevBuf prep_part;   // per particle and row band: background sums of the mask
     PruneBufs prune;
+    ReconWork recon;
     std::string prune_key;   // the projections and prefix prune's reference side was made for
     bool graph_prune = false;   // the batch graph was captured with the pruned coarse pass
     DevBuf coarse_Ai;   // projection frames of the coarse orientations, for the angles in coarse_Ai_key

@@ -15,7 +15,11 @@
 #include <hipfft/hipfft.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
+#include <cstring>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 namespace t2x {
@@ -268,10 +272,125 @@ __global__ void k_bp_widen(size_t n, const float2* __restrict__ d, const float* 
     }
 }
 
-struct FftPlan {
-    hipfftHandle h = 0;
-    ~FftPlan() { if (h) hipfftDestroy(h); }
+// The kept arena is given back after a call that needed more (a 256 box takes 4 GiB).
+constexpr size_t kReconKeep = (size_t)8 << 30;
+
+// Places of one call's buffers in the arena.
+struct Arena {
+    size_t bytes = 0;
+    size_t take(size_t n) { const size_t o = bytes; bytes += (n + 255) / 256 * 256; return o; }
 };
+
+struct ArenaRelease {
+    ReconWork& w;
+    ~ArenaRelease() { if (w.arena.bytes > kReconKeep) w.arena.release(); }
+};
+
+// A piece of a transfer between the caller's pageable memory and the device.
+struct Piece {
+    char* dev;
+    char* host;
+    size_t bytes;
+};
+
+// Copies pieces of up to kPiece bytes between pageable host memory and the device, on the stream, through
+// page-locked slots filled or emptied by several threads: a transfer from pageable memory passes the
+// driver's staging buffer in one thread (25 GB/s of the link's 57). Small totals and memory the runtime
+// knows (page-locked, device) go the plain way. To the device: the copies are queued on return, their
+// slots reused in stream order; to the host: complete on return.
+constexpr size_t kPiece = (size_t)4 << 20, kStagedMin = (size_t)16 << 20;
+constexpr int kCopyThreads = 8;
+
+int staged_copy(Device* d, const std::vector<Piece>& whole, bool to_device)
+{
+    hipStream_t st = d->stream;
+    size_t total = 0;
+    bool known = false;
+    for (const Piece& w : whole) {
+        total += w.bytes;
+        hipPointerAttribute_t at{};
+        if (hipPointerGetAttributes(&at, w.host) == hipSuccess) known |= at.type != hipMemoryTypeUnregistered;
+        else (void)hipGetLastError();
+    }
+    if (total < kStagedMin || known || d->recon.host.ensure(kPiece * 2 * kCopyThreads) != T2X_OK) {
+        for (const Piece& w : whole) {
+            if (to_device) T2X_HIP(hipMemcpyAsync(w.dev, w.host, w.bytes, hipMemcpyHostToDevice, st));
+            else T2X_HIP(hipMemcpyAsync(w.host, w.dev, w.bytes, hipMemcpyDeviceToHost, st));
+        }
+        if (!to_device) T2X_HIP(hipStreamSynchronize(st));
+        return T2X_OK;
+    }
+    std::vector<Piece> pieces;
+    for (const Piece& w : whole)
+        for (size_t o = 0; o < w.bytes; o += kPiece) pieces.push_back({w.dev + o, w.host + o, std::min(kPiece, w.bytes - o)});
+    T2X_HIP(hipStreamSynchronize(st));   // the slots' last use
+    std::atomic<int> err{(int)hipSuccess};
+    auto work = [&](int t) {
+        hipError_t e = hipSetDevice(d->id);
+        hipEvent_t ev[2] = {nullptr, nullptr};
+        for (hipEvent_t& x : ev)
+            if (e == hipSuccess) e = hipEventCreateWithFlags(&x, hipEventDisableTiming);
+        char* slot[2] = {d->recon.host.as<char>() + (size_t)(2 * t) * kPiece,
+                         d->recon.host.as<char>() + (size_t)(2 * t + 1) * kPiece};
+        size_t held[2] = {pieces.size(), pieces.size()};   // to the host: the piece on its way to the slot
+        int k = 0;
+        auto empty = [&](int q) {   // the slot's copy is over; to the host: its piece into place
+            if (held[q] == pieces.size()) return;
+            if (e == hipSuccess) e = hipEventSynchronize(ev[q]);
+            if (e == hipSuccess && !to_device) std::memcpy(pieces[held[q]].host, slot[q], pieces[held[q]].bytes);
+            held[q] = pieces.size();
+        };
+        for (size_t i = (size_t)t; i < pieces.size() && e == hipSuccess; i += kCopyThreads, k ^= 1) {
+            const Piece& p = pieces[i];
+            empty(k);
+            if (e != hipSuccess) break;
+            if (to_device) std::memcpy(slot[k], p.host, p.bytes);
+            e = to_device ? hipMemcpyAsync(p.dev, slot[k], p.bytes, hipMemcpyHostToDevice, st)
+                          : hipMemcpyAsync(slot[k], p.dev, p.bytes, hipMemcpyDeviceToHost, st);
+            if (e == hipSuccess) e = hipEventRecord(ev[k], st);
+            held[k] = i;
+        }
+        if (!to_device) {
+            empty(k);
+            empty(k ^ 1);
+        }
+        for (hipEvent_t x : ev)
+            if (x) (void)hipEventDestroy(x);
+        if (e != hipSuccess) err = (int)e;
+    };
+    std::vector<std::thread> th;
+    try {
+        for (int t = 1; t < kCopyThreads; t++) th.emplace_back(work, t);
+    } catch (const std::system_error&) {   // no more threads: their share in this one
+    }
+    const int first = (int)th.size() + 1;
+    work(0);
+    for (int t = first; t < kCopyThreads; t++) work(t);
+    for (std::thread& x : th) x.join();
+    T2X_HIP((hipError_t)err.load());
+    return T2X_OK;
+}
+
+// The n^3 double plan of a kind (0: Z2D, 1: D2Z), made when the size changes; its work area is placed by
+// the caller (plan_work bytes, hipfftSetWorkArea).
+int recon_plan(ReconWork& w, int kind, int n, hipStream_t st)
+{
+    if (w.plan_n[kind] == n) return T2X_OK;
+    if (w.plan[kind]) (void)hipfftDestroy(w.plan[kind]);
+    w.plan[kind] = 0;
+    w.plan_n[kind] = 0;
+    hipfftHandle h = 0;
+    if (hipfftCreate(&h) != HIPFFT_SUCCESS) return T2X_EDEVICE;
+    if (hipfftSetAutoAllocation(h, 0) != HIPFFT_SUCCESS ||
+        hipfftMakePlan3d(h, n, n, n, kind == 0 ? HIPFFT_Z2D : HIPFFT_D2Z, &w.plan_work[kind]) != HIPFFT_SUCCESS ||
+        hipfftSetStream(h, st) != HIPFFT_SUCCESS) {
+        (void)hipfftDestroy(h);
+        return T2X_EDEVICE;
+    }
+    w.plan[kind] = h;
+    w.plan_n[kind] = n;
+    return T2X_OK;
+}
 
 }  // namespace
 
@@ -327,33 +446,37 @@ static int reconstruct_run(Device* d, const t2x_recon_params* p, const double* d
     const size_t nr = (size_t)P * P * P;
     const size_t no = (size_t)g.ori * g.ori * g.ori;
     const int nshell_tau = g.ori / 2 + 1;
-    DevBuf b_re, b_im, b_w, b_tau, b_Fw, b_ps, b_pc, b_floor, b_err, b_W, b_R, b_vol, b_bg, b_bw;
-    T2X_TRY(b_re.ensure(nv * 8));
-    T2X_TRY(b_im.ensure(nv * 8));
-    T2X_TRY(b_w.ensure(nv * 8));
-    T2X_TRY(b_tau.ensure((size_t)nshell_tau * 8));
-    T2X_TRY(b_Fw.ensure(nv * 8));
-    T2X_TRY(b_ps.ensure((size_t)kShellBlocks * g.r_max * 8));
-    T2X_TRY(b_pc.ensure((size_t)kShellBlocks * g.r_max * 8));
-    T2X_TRY(b_floor.ensure((size_t)g.r_max * 8));
-    T2X_TRY(b_err.ensure(sizeof(int)));
-    T2X_TRY(b_W.ensure(nw * 16));
-    T2X_TRY(b_R.ensure(nr * 8));
-    T2X_TRY(b_vol.ensure(no * 8));
-    T2X_TRY(b_bg.ensure(kShellBlocks * 8));
-    T2X_TRY(b_bw.ensure(kShellBlocks * 8));
+    ReconWork& rw = d->recon;
+    if (recon_plan(rw, 0, (int)P, st) != T2X_OK) {
+        set_error("t2x_reconstruct: hipFFT Z2D plan failed");
+        return T2X_EDEVICE;
+    }
+    Arena ar;
+    const size_t o_re = ar.take(nv * 8), o_im = ar.take(nv * 8), o_w = ar.take(nv * 8), o_Fw = ar.take(nv * 8),
+                 o_tau = ar.take((size_t)nshell_tau * 8), o_ps = ar.take((size_t)kShellBlocks * g.r_max * 8),
+                 o_pc = ar.take((size_t)kShellBlocks * g.r_max * 8), o_floor = ar.take((size_t)g.r_max * 8),
+                 o_err = ar.take(sizeof(int)), o_W = ar.take(nw * 16), o_R = ar.take(nr * 8),
+                 o_vol = ar.take(no * 8), o_bg = ar.take(kShellBlocks * 8), o_bw = ar.take(kShellBlocks * 8),
+                 o_fft = ar.take(rw.plan_work[0]);
+    ArenaRelease release{rw};
+    T2X_TRY(rw.arena.ensure(ar.bytes));
+    char* base = rw.arena.as<char>();
+    auto at = [&](size_t o) { return reinterpret_cast<double*>(base + o); };
+    double *b_re = at(o_re), *b_im = at(o_im), *b_w = at(o_w), *b_Fw = at(o_Fw), *b_tau = at(o_tau), *b_ps = at(o_ps),
+           *b_pc = at(o_pc), *b_floor = at(o_floor), *b_R = at(o_R), *b_vol = at(o_vol), *b_bg = at(o_bg), *b_bw = at(o_bw);
+    double2* b_W = reinterpret_cast<double2*>(base + o_W);
+    int* b_err = reinterpret_cast<int*>(base + o_err);
     if (bp) {
         k_bp_widen<<<(unsigned)std::min<size_t>((nv + 255) / 256, 65536), 256, 0, st>>>(
-            nv, bp->bp_data, bp->bp_weight, b_re.as<double>(), b_im.as<double>(), b_w.as<double>());
+            nv, bp->bp_data, bp->bp_weight, b_re, b_im, b_w);
         T2X_HIP(hipGetLastError());
     } else {
-        T2X_HIP(hipMemcpyAsync(b_re.ptr, data_re, nv * 8, hipMemcpyHostToDevice, st));
-        T2X_HIP(hipMemcpyAsync(b_im.ptr, data_im, nv * 8, hipMemcpyHostToDevice, st));
-        T2X_HIP(hipMemcpyAsync(b_w.ptr, weight, nv * 8, hipMemcpyHostToDevice, st));
+        T2X_TRY(staged_copy(d, {{(char*)b_re, (char*)data_re, nv * 8}, {(char*)b_im, (char*)data_im, nv * 8},
+                                {(char*)b_w, (char*)weight, nv * 8}}, true));
     }
-    if (p->do_map) T2X_HIP(hipMemcpyAsync(b_tau.ptr, tau2, (size_t)nshell_tau * 8, hipMemcpyHostToDevice, st));
-    else T2X_HIP(hipMemsetAsync(b_tau.ptr, 0, (size_t)nshell_tau * 8, st));
-    T2X_HIP(hipMemsetAsync(b_err.ptr, 0, sizeof(int), st));
+    if (p->do_map) T2X_HIP(hipMemcpyAsync(b_tau, tau2, (size_t)nshell_tau * 8, hipMemcpyHostToDevice, st));
+    else T2X_HIP(hipMemsetAsync(b_tau, 0, (size_t)nshell_tau * 8, st));
+    T2X_HIP(hipMemsetAsync(b_err, 0, sizeof(int), st));
     // the MAP shell index ROUND(|k|/pf) for |k|^2 < max_r2 stays below r_max + 1 <= ori/2 + 1
     if (p->do_map && (long long)p->r_max + 1 > nshell_tau) {
         set_error("t2x_reconstruct: r_max exceeds the tau2 spectrum (ori_size/2+1 shells)");
@@ -361,40 +484,33 @@ static int reconstruct_run(Device* d, const t2x_recon_params* p, const double* d
     }
 
     k_recon_weights<<<kShellBlocks, 256, 2 * sizeof(double) * g.r_max, st>>>(
-        g, b_w.as<double>(), b_tau.as<double>(), b_Fw.as<double>(), b_ps.as<double>(), b_pc.as<double>(),
-        b_err.as<int>());
+        g, b_w, b_tau, b_Fw, b_ps, b_pc,
+        b_err);
     T2X_HIP(hipGetLastError());
-    k_recon_floor<<<(g.r_max + 255) / 256, 256, 0, st>>>(g, b_ps.as<double>(), b_pc.as<double>(), kShellBlocks,
-                                                         b_floor.as<double>(), b_err.as<int>());
+    k_recon_floor<<<(g.r_max + 255) / 256, 256, 0, st>>>(g, b_ps, b_pc, kShellBlocks,
+                                                         b_floor, b_err);
     T2X_HIP(hipGetLastError());
     k_recon_window<<<(unsigned)std::min<size_t>((nw + 255) / 256, 65536), 256, 0, st>>>(
-        g, b_re.as<double>(), b_im.as<double>(), b_Fw.as<double>(), b_floor.as<double>(), b_W.as<double2>());
+        g, b_re, b_im, b_Fw, b_floor, b_W);
     T2X_HIP(hipGetLastError());
     int herr = 0;
-    T2X_HIP(hipMemcpyAsync(&herr, b_err.ptr, sizeof(int), hipMemcpyDeviceToHost, st));
+    T2X_HIP(hipMemcpyAsync(&herr, b_err, sizeof(int), hipMemcpyDeviceToHost, st));
     T2X_HIP(hipStreamSynchronize(st));
     if (herr == 2) { set_error("t2x_reconstruct: negative tau2 values"); return T2X_EINVAL; }
     if (herr == 3 || herr == 4) { set_error("t2x_reconstruct: empty or inconsistent weight shells"); return T2X_EINVAL; }
 
-    FftPlan plan;
-    if (hipfftPlan3d(&plan.h, (int)P, (int)P, (int)P, HIPFFT_Z2D) != HIPFFT_SUCCESS ||
-        hipfftSetStream(plan.h, st) != HIPFFT_SUCCESS) {
-        set_error("t2x_reconstruct: hipFFT Z2D plan failed");
-        return T2X_EDEVICE;
-    }
-    if (hipfftExecZ2D(plan.h, b_W.as<hipfftDoubleComplex>(), b_R.as<hipfftDoubleReal>()) != HIPFFT_SUCCESS) {
+    if (hipfftSetWorkArea(rw.plan[0], base + o_fft) != HIPFFT_SUCCESS ||
+        hipfftExecZ2D(rw.plan[0], reinterpret_cast<hipfftDoubleComplex*>(b_W), b_R) != HIPFFT_SUCCESS) {
         set_error("t2x_reconstruct: hipFFT Z2D failed");
         return T2X_EDEVICE;
     }
-    k_recon_crop<<<kShellBlocks, 1024, 0, st>>>(g, b_R.as<double>(), b_vol.as<double>(), b_bg.as<double>(),
-                                                b_bw.as<double>());
+    k_recon_crop<<<kShellBlocks, 1024, 0, st>>>(g, b_R, b_vol, b_bg,
+                                                b_bw);
     T2X_HIP(hipGetLastError());
     k_recon_finish<<<(unsigned)std::min<size_t>((no + 255) / 256, 65536), 256, 0, st>>>(
-        g, b_bg.as<double>(), b_bw.as<double>(), kShellBlocks, b_vol.as<double>());
+        g, b_bg, b_bw, kShellBlocks, b_vol);
     T2X_HIP(hipGetLastError());
-    T2X_HIP(hipMemcpyAsync(vol_out, b_vol.ptr, no * 8, hipMemcpyDeviceToHost, st));
-    T2X_HIP(hipStreamSynchronize(st));
-    return T2X_OK;
+    return staged_copy(d, {{(char*)b_vol, (char*)vol_out, no * 8}}, false);
 }
 
 extern "C" int t2x_reconstruct(t2x_device* hdev, const t2x_recon_params* p, const double* data_re,
@@ -430,31 +546,33 @@ extern "C" int t2x_fsc(t2x_device* hdev, int n, const double* map1, const double
     hipStream_t st = d->stream;
     const long long N = n, xh = N / 2 + 1;
     const size_t nr = (size_t)N * N * N, nc = (size_t)N * N * xh;
-    DevBuf r1, r2, c1, c2, part, out;
-    T2X_TRY(r1.ensure(nr * 8));
-    T2X_TRY(r2.ensure(nr * 8));
-    T2X_TRY(c1.ensure(nc * 16));
-    T2X_TRY(c2.ensure(nc * 16));
-    T2X_TRY(part.ensure((size_t)kShellBlocks * 3 * xh * 8));
-    T2X_TRY(out.ensure((size_t)xh * 8));
-    T2X_HIP(hipMemcpyAsync(r1.ptr, map1, nr * 8, hipMemcpyHostToDevice, st));
-    T2X_HIP(hipMemcpyAsync(r2.ptr, map2, nr * 8, hipMemcpyHostToDevice, st));
-    FftPlan plan;
-    if (hipfftPlan3d(&plan.h, n, n, n, HIPFFT_D2Z) != HIPFFT_SUCCESS || hipfftSetStream(plan.h, st) != HIPFFT_SUCCESS) {
+    ReconWork& rw = d->recon;
+    if (recon_plan(rw, 1, n, st) != T2X_OK) {
         set_error("t2x_fsc: hipFFT D2Z plan failed");
         return T2X_EDEVICE;
     }
-    if (hipfftExecD2Z(plan.h, r1.as<hipfftDoubleReal>(), c1.as<hipfftDoubleComplex>()) != HIPFFT_SUCCESS ||
-        hipfftExecD2Z(plan.h, r2.as<hipfftDoubleReal>(), c2.as<hipfftDoubleComplex>()) != HIPFFT_SUCCESS) {
+    Arena ar;
+    const size_t o_r1 = ar.take(nr * 8), o_r2 = ar.take(nr * 8), o_c1 = ar.take(nc * 16), o_c2 = ar.take(nc * 16),
+                 o_part = ar.take((size_t)kShellBlocks * 3 * xh * 8), o_out = ar.take((size_t)xh * 8),
+                 o_fft = ar.take(rw.plan_work[1]);
+    ArenaRelease release{rw};
+    T2X_TRY(rw.arena.ensure(ar.bytes));
+    char* base = rw.arena.as<char>();
+    double *r1 = reinterpret_cast<double*>(base + o_r1), *r2 = reinterpret_cast<double*>(base + o_r2),
+           *part = reinterpret_cast<double*>(base + o_part), *out = reinterpret_cast<double*>(base + o_out);
+    double2 *c1 = reinterpret_cast<double2*>(base + o_c1), *c2 = reinterpret_cast<double2*>(base + o_c2);
+    T2X_TRY(staged_copy(d, {{(char*)r1, (char*)map1, nr * 8}, {(char*)r2, (char*)map2, nr * 8}}, true));
+    if (hipfftSetWorkArea(rw.plan[1], base + o_fft) != HIPFFT_SUCCESS ||
+        hipfftExecD2Z(rw.plan[1], r1, reinterpret_cast<hipfftDoubleComplex*>(c1)) != HIPFFT_SUCCESS ||
+        hipfftExecD2Z(rw.plan[1], r2, reinterpret_cast<hipfftDoubleComplex*>(c2)) != HIPFFT_SUCCESS) {
         set_error("t2x_fsc: hipFFT D2Z failed");
         return T2X_EDEVICE;
     }
-    k_fsc_partial<<<kShellBlocks, 256, 3 * sizeof(double) * xh, st>>>(N, c1.as<double2>(), c2.as<double2>(),
-                                                                       part.as<double>());
+    k_fsc_partial<<<kShellBlocks, 256, 3 * sizeof(double) * xh, st>>>(N, c1, c2, part);
     T2X_HIP(hipGetLastError());
-    k_fsc_final<<<(unsigned)((xh + 255) / 256), 256, 0, st>>>(N, part.as<double>(), kShellBlocks, out.as<double>());
+    k_fsc_final<<<(unsigned)((xh + 255) / 256), 256, 0, st>>>(N, part, kShellBlocks, out);
     T2X_HIP(hipGetLastError());
-    T2X_HIP(hipMemcpyAsync(fsc, out.ptr, (size_t)xh * 8, hipMemcpyDeviceToHost, st));
+    T2X_HIP(hipMemcpyAsync(fsc, out, (size_t)xh * 8, hipMemcpyDeviceToHost, st));
     T2X_HIP(hipStreamSynchronize(st));
     return T2X_OK;
 }
