@@ -2871,6 +2871,14 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
         d->coarse_key = key;
         d->prune_key.clear();
     }
+    // The pruned coarse pass of a batch of B particles: its ten launches and the bounds GEMM pay where the
+    // exhaustive GEMM takes longer than about 0.15 ms (110 TFLOP/s in FP32, 1,150 TFLOP/s a product).
+    auto prune_pays = [&](int B) {
+        const double gemm_flop = 4. * (double)T * (double)O_all * (double)tc.npix * B;
+        const double gemm_rate = prec == T2X_PREC_FP32 ? 110e12 : (prec == T2X_PREC_FP16X2 ? 575e12 : 383e12);
+        return prune_force || gemm_flop > 1.5e-4 * gemm_rate;
+    };
+    if (!prune_pays(n)) prune_call = false;   // no batch is larger: the reference side (30 us) is not needed either
     if (prune_call) {
         const std::string pkey = key + "/" + std::to_string(n_low);
         if (pkey != d->prune_key) {
@@ -3016,11 +3024,7 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
 
     for (int b0 = 0; b0 < n; b0 += Bmax) {
         const int B = std::min(Bmax, n - b0);
-        // the pruned coarse pass for this batch: its ten launches and the bounds GEMM pay where the
-        // exhaustive GEMM takes longer than about 0.15 ms (110 TFLOP/s in FP32, 1,150 TFLOP/s a product)
-        const double gemm_flop = 4. * (double)T * (double)O_all * (double)tc.npix * B;
-        const double gemm_rate = prec == T2X_PREC_FP32 ? 110e12 : (prec == T2X_PREC_FP16X2 ? 575e12 : 383e12);
-        const bool prune_batch = prune_call && (prune_force || gemm_flop > 1.5e-4 * gemm_rate);
+        const bool prune_batch = prune_call && prune_pays(B);
         // its full GEMM's tiles, known here for graph replays too
         const long long prune_ntiles =
             prune_batch ? (round_up((long long)B * T, 256) / PRUNED_TILE) * (O_pad / PRUNED_TILE) : 0;
