@@ -46,6 +46,9 @@ int launch_gemm_x3(int prec, int epi, const void* Ah, const void* Al, const floa
 int launch_gemm_pruned(int prec, const void* Ah, const void* Al, const float* As, long long lda, const void* Bh,
                        const void* Bl, const float* Bs, long long ldb, int K, int Mrows_pad, int Nrows_pad,
                        const EpiParams& ep, const unsigned* list, const unsigned* count, int n_cu, hipStream_t st);
+int launch_gemm_local_f32(const float2* F, const float2* Y, const double* W, int B, const long long* orient_off,
+                          const int* rowu, long long rows, const float* ab, int Kc, int Tl, const EpiParams& ep,
+                          double* n1, hipStream_t st);
 int launch_gemm_local_x3(int prec, const void* Sh, const void* Sl, const float* Ss, const void* Wh, const void* Wl,
                          const float* Ws, long long ld, int K, const int2* items, int n_items, int T,
                          const long long* orient_off, const int* rowu, const double* cb, const double* n1,
@@ -605,17 +608,6 @@ struct FineGeom {
     double pf;
 };
 
-__device__ __forceinline__ int find_particle(const long long* off, int B, long long i)
-{
-    int lo = 0, hi = B;   // off[lo] <= i < off[hi]
-    while (hi - lo > 1) {
-        int mid = (lo + hi) >> 1;
-        if (off[mid] <= i) lo = mid;
-        else hi = mid;
-    }
-    return lo;
-}
-
 __device__ __forceinline__ void fine_matrix(const FineGeom& g, int n, int ir, double* A, int* cls, int* idir)
 {
     const int c = n / g.Norient, o = n - c * g.Norient;
@@ -1047,11 +1039,11 @@ __global__ void k_fine_ab_rows(const float2* __restrict__ ab, int npix, int ldk,
 // Local searches, coarse pass (FP32) as a GEMM over the batch's (particle, orientation) rows:
 // G[(b,o)][t] = sum_p Re(Z_bo,p conj(AB_t,p)) with Z_bo = F_o conj(minv ctf X_b), i.e. the real
 // dot product of [Z.re, Z.im] with [AB.re, AB.im] over K = 2 P_c; the phase table AB is the
-// shared operand. k_local_zrows forms Z from the row's slice (projected once per batch by
-// k_project_list) and n1 = 1/2 sum minv ctf^2 |F|^2; k_local_diff2 forms
-// diff2 = C_coarse + n1 - G into the sample list (orientation-major, T per orientation).
-// The batch's distinct in-range orientations projected once (exact FP32 slices at coarse size,
-// XCD-aware order as k_local_zrows), shared by every particle whose range holds them. SPLIT 0:
+// shared operand. k_gemm_local (t2x_gemm.hip) forms Z and n1 = 1/2 sum minv ctf^2 |F|^2 as it loads;
+// k_local_diff2 forms diff2 = C_coarse + n1 - G into the sample list (orientation-major, T per orientation).
+
+// The batch's distinct in-range orientations projected once (exact FP32 slices at coarse size; each XCD,
+// workgroup index & 7, takes contiguous ones), shared by every particle whose range holds them. SPLIT 0:
 // float2 rows F (the FP32 path); SPLIT 1: the rows straight into the split operand (hi, lo and a
 // power-of-two row scale for FP16, as k_split_rows) plus |F|^2 for the n1 term; SPLIT 2: BF16 halves
 // (no scale, chunk by chunk) plus |F|^2. Padding columns are written as zero.
@@ -1155,49 +1147,27 @@ __global__ __launch_bounds__(256) void k_local_n1(int B, long long nrows, const 
     if (lane == 0) n1out[j] = acc;
 }
 
-__global__ __launch_bounds__(256) void k_local_zrows(int B, long long nrows, const long long* __restrict__ orient_off,
-                                                     const int* __restrict__ rowu, const float2* __restrict__ F,
-                                                     int ldf, const float* __restrict__ minv,
-                                                     const int* __restrict__ win, int npix,
-                                                     const PartScalars* __restrict__ ps,
-                                                     const float2* __restrict__ Fimg,
-                                                     const float* __restrict__ Fctf, int Pw, int Kc,
-                                                     float* __restrict__ zf, double* __restrict__ n1out)
+// A particle's side of the FP32 local search (k_gemm_local in t2x_gemm.hip): Y = minv ctf X, re/im
+// interleaved, and the weight 1/2 minv ctf^2 of n1 in FP64, over the coarse pixels (zero in the padding).
+__global__ __launch_bounds__(256) void k_local_y(const float* __restrict__ minv, const int* __restrict__ win, int npix,
+                                                 const PartScalars* __restrict__ ps, const float2* __restrict__ Fimg,
+                                                 const float* __restrict__ Fctf, int Pw, int Kn,
+                                                 float2* __restrict__ Y, double* __restrict__ W)
 {
-    __shared__ double red[4];
-    // XCD-aware row order: workgroups are dealt round-robin to the 8 XCDs, so XCD k is given the
-    // contiguous rows [k R/8, (k+1) R/8) (the grid is a multiple of 8)
-    const long long per = (long long)gridDim.x / 8;
-    const long long j = (long long)(blockIdx.x % 8) * per + blockIdx.x / 8;
-    const bool valid = j < nrows;
-    double n1 = 0.;
-    if (valid) {
-        const int b = find_particle(orient_off, B, j);
-        const float2* Fu = F + (long long)rowu[j] * ldf;
-        const float* mv = minv + (size_t)ps[b].og * npix;
-        for (int p = threadIdx.x; p < Kc / 2; p += blockDim.x) {
-            float zr = 0.f, zi = 0.f;
-            if (p < npix) {
-                const float2 f = Fu[p];
-                const size_t w = (size_t)b * Pw + win[p];
-                const float2 X = Fimg[w];
-                const float ctf = Fctf[w], m = mv[p];
-                const float s = m * ctf;
-                const float yr = s * X.x, yi = s * X.y;
-                zr = f.x * yr + f.y * yi;
-                zi = f.y * yr - f.x * yi;
-                n1 += 0.5 * (double)m * (double)ctf * ctf * ((double)f.x * f.x + (double)f.y * f.y);
-            }
-            zf[j * Kc + 2 * p] = zr;
-            zf[j * Kc + 2 * p + 1] = zi;
-        }
-    } else {
-        for (int k = threadIdx.x; k < Kc; k += blockDim.x) zf[j * Kc + k] = 0.f;
+    const int b = blockIdx.y, p = blockIdx.x * 256 + threadIdx.x;
+    if (p >= Kn) return;
+    float2 y = make_float2(0.f, 0.f);
+    double w1 = 0.;
+    if (p < npix) {
+        const size_t w = (size_t)b * Pw + win[p];
+        const float2 X = Fimg[w];
+        const float ctf = Fctf[w], m = minv[(size_t)ps[b].og * npix + p];
+        const float s = m * ctf;
+        y = make_float2(s * X.x, s * X.y);
+        w1 = 0.5 * (double)m * (double)ctf * ctf;
     }
-    for (int o = 32; o > 0; o >>= 1) n1 += __shfl_xor(n1, o);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = n1;
-    __syncthreads();
-    if (valid && threadIdx.x == 0) n1out[j] = red[0] + red[1] + red[2] + red[3];
+    Y[(size_t)b * Kn + p] = y;
+    W[(size_t)b * Kn + p] = w1;
 }
 
 // The phase table as the GEMM's shared operand: row t = [re, im] of AB_t over the coarse pixels,
@@ -2919,8 +2889,8 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
                               : std::min((double)Nd, Nd * (1. - std::cos(rd * kPi / 180.)) / 2. + 16.);
         const double np_est = (cfg->sigma_psi > 0.) ? std::min((double)Npsi, Npsi * (6. * cfg->sigma_psi + 2. * step_p) / 360. + 2.)
                                                     : (double)Npsi;
-        // per sample list entry 16 bytes; per (particle, orientation) row its Z row (4 bytes per K
-        // element), G row (Tl floats) and n1
+        // per sample list entry 16 bytes; per (particle, orientation) row a slice of its own at worst (4 bytes
+        // per K element), G row (Tl floats) and n1
         const double rows_est = Kact * nd_est * np_est;
         per_particle = (size_t)(16. * rows_est * T + rows_est * (4. * Kc + 4. * Tl + 8.)) + (size_t)4 * N * N * 4 +
                        (size_t)2 * N * xN * 8 * 2 + noise_bytes;
@@ -3315,15 +3285,15 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
                     eg.ldc = Tl;
                     eg.M = (int)rows;
                     eg.N = (int)T;
-                    T2X_TRY(d->lc_z.ensure(sizeof(float) * rows_pad * Kc));
-                    k_local_zrows<<<(unsigned)rows_pad, 256, 0, st>>>(
-                        B, rows, d->lc_orient_off.as<long long>(), d->lc_rowu.as<int>(), d->lc_F.as<float2>(), ldf,
-                        tc.d_minv.as<float>(), tc.d_win.as<int>(), tc.npix, d_ps,
-                        d->Fimg_cur.as<float2>(), d->Fctf_cur.as<float>(), Pw, Kc, d->lc_z.as<float>(),
-                        d->lc_n1.as<double>());
+                    T2X_TRY(d->lc_y.ensure(sizeof(float2) * B * Kn));
+                    T2X_TRY(d->lc_w.ensure(sizeof(double) * B * Kn));
+                    k_local_y<<<dim3((unsigned)((Kn + 255) / 256), (unsigned)B), 256, 0, st>>>(
+                        tc.d_minv.as<float>(), tc.d_win.as<int>(), tc.npix, d_ps, d->Fimg_cur.as<float2>(),
+                        d->Fctf_cur.as<float>(), Pw, Kn, d->lc_y.as<float2>(), d->lc_w.as<double>());
                     T2X_HIP(hipGetLastError());
-                    T2X_TRY(launch_gemm(EPI_STORE, d->lc_z.as<float>(), Kc, d->lc_ab.as<float>(), Kc, Kc,
-                                        (int)rows_pad, Tl, eg, st));
+                    T2X_TRY(launch_gemm_local_f32(d->lc_F.as<float2>(), d->lc_y.as<float2>(), d->lc_w.as<double>(), B,
+                                                  d->lc_orient_off.as<long long>(), d->lc_rowu.as<int>(), rows,
+                                                  d->lc_ab.as<float>(), Kc, Tl, eg, d->lc_n1.as<double>(), st));
                     k_local_diff2<<<(unsigned)rows, 128, 0, st>>>(B, rows, d->lc_orient_off.as<long long>(), d_ps,
                                                                  d->lc_n1.as<double>(), d->lc_G.as<float>(), Tl, (int)T,
                                                                  d->lc_d2.as<float>(), d->lc_min.as<unsigned int>());

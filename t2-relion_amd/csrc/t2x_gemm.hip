@@ -124,10 +124,45 @@ __device__ __forceinline__ void gemm_epilogue(const floatx4 (&acc)[MI][4], long 
 #define GBK 16
 #define GPAD 4
 
+// A thread's rows lrow and lrow + 64 of the first operand, four elements at k0 + lk4 of each: from memory.
+struct RowsOperand {
+    const float *p0, *p1;
+    float4 r0, r1;
+    __device__ __forceinline__ void fetch(int k) { r0 = *reinterpret_cast<const float4*>(p0 + k); r1 = *reinterpret_cast<const float4*>(p1 + k); }
+    __device__ __forceinline__ float4 row0() { return r0; }
+    __device__ __forceinline__ float4 row1() { return r1; }
+};
+
+// The same formed on the way to LDS: Z = F conj(Y), slice times particle, with the row's n1 = sum W |F|^2.
+struct LocalOperand {
+    const float *f0, *f1, *y0, *y1;
+    const double *w0, *w1;
+    float4 F0, F1, Y0, Y1;
+    double2 W0, W1;
+    double n0, n1;
+    __device__ __forceinline__ void fetch(int k)
+    {
+        F0 = *reinterpret_cast<const float4*>(f0 + k);
+        F1 = *reinterpret_cast<const float4*>(f1 + k);
+        Y0 = *reinterpret_cast<const float4*>(y0 + k);
+        Y1 = *reinterpret_cast<const float4*>(y1 + k);
+        W0 = *reinterpret_cast<const double2*>(w0 + k / 2);
+        W1 = *reinterpret_cast<const double2*>(w1 + k / 2);
+    }
+    static __device__ __forceinline__ float4 form(const float4& f, const float4& y, const double2& w, double& n)
+    {
+        n += w.x * ((double)f.x * f.x + (double)f.y * f.y);
+        n += w.y * ((double)f.z * f.z + (double)f.w * f.w);
+        return make_float4(f.x * y.x + f.y * y.y, f.y * y.x - f.x * y.y, f.z * y.z + f.w * y.w, f.w * y.z - f.z * y.w);
+    }
+    __device__ __forceinline__ float4 row0() { return form(F0, Y0, W0, n0); }
+    __device__ __forceinline__ float4 row1() { return form(F1, Y1, W1, n1); }
+};
+
 // One 128x128 tile of the FP32 GEMM, rows from m0, columns from n0.
-template <int EPI>
+template <int EPI, class OperandA>
 __device__ __forceinline__ void gemm_tn_tile(float (&As)[GBK][GBM + GPAD], float (&Bs)[GBK][GBN + GPAD],
-                                             const float* __restrict__ A, long long lda, const float* __restrict__ B,
+                                             OperandA& A, const float* __restrict__ B,
                                              long long ldb, int K, long long m0, long long n0, const EpiParams& ep)
 {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -139,17 +174,15 @@ __device__ __forceinline__ void gemm_tn_tile(float (&As)[GBK][GBM + GPAD], float
 
     // loader mapping: 128 rows x 16 k = 512 float4; 2 per thread
     const int lrow = tid >> 2, lk4 = (tid & 3) * 4;
-    const float* Ap0 = A + (m0 + lrow) * lda + lk4;
-    const float* Ap1 = A + (m0 + lrow + 64) * lda + lk4;
     const float* Bp0 = B + (n0 + lrow) * ldb + lk4;
     const float* Bp1 = B + (n0 + lrow + 64) * ldb + lk4;
 
-    float4 ra0 = *reinterpret_cast<const float4*>(Ap0);
-    float4 ra1 = *reinterpret_cast<const float4*>(Ap1);
+    A.fetch(0);
     float4 rb0 = *reinterpret_cast<const float4*>(Bp0);
     float4 rb1 = *reinterpret_cast<const float4*>(Bp1);
 
     for (int k0 = 0; k0 < K; k0 += GBK) {
+        const float4 ra0 = A.row0(), ra1 = A.row1();
         __syncthreads();
         As[lk4 + 0][lrow] = ra0.x; As[lk4 + 1][lrow] = ra0.y; As[lk4 + 2][lrow] = ra0.z; As[lk4 + 3][lrow] = ra0.w;
         As[lk4 + 0][lrow + 64] = ra1.x; As[lk4 + 1][lrow + 64] = ra1.y; As[lk4 + 2][lrow + 64] = ra1.z; As[lk4 + 3][lrow + 64] = ra1.w;
@@ -157,8 +190,7 @@ __device__ __forceinline__ void gemm_tn_tile(float (&As)[GBK][GBM + GPAD], float
         Bs[lk4 + 0][lrow + 64] = rb1.x; Bs[lk4 + 1][lrow + 64] = rb1.y; Bs[lk4 + 2][lrow + 64] = rb1.z; Bs[lk4 + 3][lrow + 64] = rb1.w;
         __syncthreads();
         if (k0 + GBK < K) {   // prefetch the next K slice into registers while the MFMAs run
-            ra0 = *reinterpret_cast<const float4*>(Ap0 + k0 + GBK);
-            ra1 = *reinterpret_cast<const float4*>(Ap1 + k0 + GBK);
+            A.fetch(k0 + GBK);
             rb0 = *reinterpret_cast<const float4*>(Bp0 + k0 + GBK);
             rb1 = *reinterpret_cast<const float4*>(Bp1 + k0 + GBK);
         }
@@ -182,6 +214,12 @@ __device__ __forceinline__ void gemm_tn_tile(float (&As)[GBK][GBM + GPAD], float
     gemm_epilogue<4, EPI>(acc, m0 + wm * 64, n0 + wn * 64, lane, nullptr, nullptr, ep);
 }
 
+__device__ __forceinline__ RowsOperand rows_operand(const float* __restrict__ A, long long lda, long long m0)
+{
+    const float* p = A + (m0 + (threadIdx.x >> 2)) * lda + (threadIdx.x & 3) * 4;
+    return {p, p + 64 * lda, {}, {}};
+}
+
 // LIST (the pruned coarse pass): a persistent grid over the tiles listed in ep.tile_list
 // (*ep.tile_count of them, indices tm * tiles_n + tn).
 template <int EPI, bool LIST = false>
@@ -195,13 +233,54 @@ __global__ __launch_bounds__(256) void k_gemm_tn(const float* __restrict__ A, lo
         const unsigned n = *ep.tile_count;
         for (unsigned it = blockIdx.x; it < n; it += gridDim.x) {
             const unsigned t = ep.tile_list[it];
-            gemm_tn_tile<EPI>(As, Bs, A, lda, B, ldb, K, (long long)(t / (unsigned)tiles_n) * GBM,
-                              (long long)(t % (unsigned)tiles_n) * GBN, ep);
+            const long long m0 = (long long)(t / (unsigned)tiles_n) * GBM;
+            RowsOperand a = rows_operand(A, lda, m0);
+            gemm_tn_tile<EPI>(As, Bs, a, B, ldb, K, m0, (long long)(t % (unsigned)tiles_n) * GBN, ep);
         }   // (the tile's K loop starts with a barrier: its LDS is free again)
     } else {
         int tm, tn;
         tile_coords(blockIdx.x, tiles_m, tiles_n, group_m, tm, tn);
-        gemm_tn_tile<EPI>(As, Bs, A, lda, B, ldb, K, (long long)tm * GBM, (long long)tn * GBN, ep);
+        RowsOperand a = rows_operand(A, lda, (long long)tm * GBM);
+        gemm_tn_tile<EPI>(As, Bs, a, B, ldb, K, (long long)tm * GBM, (long long)tn * GBN, ep);
+    }
+}
+
+// FP32 local searches: G = Z . AB over the batch's (particle, orientation) rows, Z formed from the shared
+// slices and the particles as the tiles load it, with n1. Z in memory cost twice as much to write and read
+// back as the product itself: 500 particles of a 360 box at 7 A 17.7 + 8.4 ms, so 9.2. Bound by the FP32
+// matrix units beside the operand's arithmetic. A tile's rows lie next to each other on an XCD (workgroup
+// index & 7), so that it reads a particle once.
+__global__ __launch_bounds__(256) void k_gemm_local(const float2* __restrict__ F, const float2* __restrict__ Y,
+                                                    const double* __restrict__ W, int nb,
+                                                    const long long* __restrict__ orient_off,
+                                                    const int* __restrict__ rowu, long long rows,
+                                                    const float* __restrict__ B, int K, int tiles_m,
+                                                    EpiParams ep, double* __restrict__ n1out)
+{
+    __shared__ float As[GBK][GBM + GPAD];
+    __shared__ float Bs[GBK][GBN + GPAD];
+    const int tm = (int)(blockIdx.x % 8) * (int)(gridDim.x / 8) + (int)(blockIdx.x / 8);
+    if (tm >= tiles_m) return;
+    const int lrow = threadIdx.x >> 2, lk4 = (threadIdx.x & 3) * 4;
+    const long long m0 = (long long)tm * GBM, j0 = m0 + lrow, j1 = j0 + 64;
+    const long long c0 = min(j0, rows - 1), c1 = min(j1, rows - 1);   // (rows past the end are not stored)
+    const long long b0 = find_particle(orient_off, nb, c0), b1 = find_particle(orient_off, nb, c1);
+    LocalOperand a;
+    a.f0 = reinterpret_cast<const float*>(F) + (long long)rowu[c0] * K + lk4;
+    a.f1 = reinterpret_cast<const float*>(F) + (long long)rowu[c1] * K + lk4;
+    a.y0 = reinterpret_cast<const float*>(Y) + b0 * K + lk4;
+    a.y1 = reinterpret_cast<const float*>(Y) + b1 * K + lk4;
+    a.w0 = W + b0 * (K / 2) + lk4 / 2;
+    a.w1 = W + b1 * (K / 2) + lk4 / 2;
+    a.n0 = a.n1 = 0.;
+    gemm_tn_tile<EPI_STORE>(As, Bs, a, B, K, K, m0, (long long)blockIdx.y * GBN, ep);
+    if (blockIdx.y == 0) {
+        for (int o = 1; o < 4; o <<= 1) {
+            a.n0 += __shfl_xor(a.n0, o);
+            a.n1 += __shfl_xor(a.n1, o);
+        }
+        if (lk4 == 0 && j0 < rows) n1out[j0] = a.n0;
+        if (lk4 == 0 && j1 < rows) n1out[j1] = a.n1;
     }
 }
 
@@ -214,6 +293,24 @@ static int gemm_group_m()
         return v > 0 ? v : 64;
     }();
     return g;
+}
+
+// G of an FP32 local search: `rows` rows against the Tl phase rows ab; Y, W: [B][Kc / 2], slices F of Kc / 2
+// pixels.
+int launch_gemm_local_f32(const float2* F, const float2* Y, const double* W, int B, const long long* orient_off,
+                          const int* rowu, long long rows, const float* ab, int Kc, int Tl, const EpiParams& ep,
+                          double* n1, hipStream_t st)
+{
+    if (Kc % GBK != 0 || Tl % GBN != 0 || rows < 1 || B < 1) {
+        set_error("gemm_local_f32: operands not padded to tile multiples");
+        return T2X_EINVAL;
+    }
+    const long long tm = (rows + GBM - 1) / GBM;
+    if (tm > 0x7ffffff0LL) { set_error("gemm_local_f32: grid too large"); return T2X_EINVAL; }
+    k_gemm_local<<<dim3((unsigned)((tm + 7) / 8 * 8), (unsigned)(Tl / GBN)), 256, 0, st>>>(F, Y, W, B, orient_off, rowu, rows, ab,
+                                                                                       Kc, (int)tm, ep, n1);
+    T2X_HIP(hipGetLastError());
+    return T2X_OK;
 }
 
 // Host launcher. A must have tiles_m*128 rows, B tiles_n*128 rows, both K (multiple of 16)

@@ -136,6 +136,18 @@ __device__ __forceinline__ bool coarse_allowed(const WeightSrc& s, int b, long l
     return (s.bin_mask[(size_t)b * s.mask_words + (bin >> 5)] >> (bin & 31)) & 1u;
 }
 
+// The particle whose range of the offsets off[0 .. B] holds i.
+__device__ __forceinline__ int find_particle(const long long* off, int B, long long i)
+{
+    int lo = 0, hi = B;   // off[lo] <= i < off[hi]
+    while (hi - lo > 1) {
+        int mid = (lo + hi) >> 1;
+        if (off[mid] <= i) lo = mid;
+        else hi = mid;
+    }
+    return lo;
+}
+
 // Epilogue parameters of the coarse cross-term GEMMs.
 // Variant of the split-precision GEMM: tile 128 / 256 / 257 / 258 (0: autotuned) and tile-walk
 // group in tile rows (0: the variant's default).
