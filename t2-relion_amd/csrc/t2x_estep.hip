@@ -2345,31 +2345,72 @@ static std::vector<int2> gather_order(const PassTables& t)
     return g;
 }
 
-static int upload_table(PassTables& t, hipStream_t st)
+// A call's tables, gathered on the host and brought to their buffers by one kernel that reads them from
+// page-locked memory: about thirty copies of some KB each, with a launch and a trip through the driver's
+// staging buffer apiece, had been a tenth of a call of one particle (one particle of a 64 box: 925 -> 850 us).
+struct TablePiece {
+    unsigned* dst;
+    unsigned off, words;   // offset in words from the first table
+};
+#define TABLE_PIECE 4096   // words of a workgroup
+
+__global__ __launch_bounds__(256) void k_tables(const TablePiece* __restrict__ pieces, const unsigned* __restrict__ src)
 {
-    T2X_TRY(t.d_pix.ensure(sizeof(int2) * t.npix));
-    T2X_TRY(t.d_win.ensure(sizeof(int) * t.npix));
-    T2X_TRY(t.d_minv.ensure(sizeof(float) * t.h_minv.size()));
-    T2X_TRY(t.d_ires.ensure(sizeof(int) * t.npix));
-    T2X_TRY(t.d_inproj.ensure(t.npix));
+    const TablePiece p = pieces[blockIdx.x];
+    for (unsigned i = threadIdx.x; i < p.words; i += 256) p.dst[i] = src[p.off + i];
+}
+
+struct TableUpload {
+    std::vector<TablePiece> pieces;
+    std::vector<unsigned> data;
+    int add(DevBuf& buf, const void* v, size_t bytes)
+    {
+        const size_t words = (bytes + 3) / 4;
+        T2X_TRY(buf.ensure(std::max<size_t>(4 * words, 4)));
+        const size_t off = data.size();
+        data.resize(off + words);
+        if (bytes) std::memcpy(&data[off], v, bytes);
+        for (size_t o = 0; o < words; o += TABLE_PIECE)
+            pieces.push_back({buf.as<unsigned>() + o, (unsigned)(off + o), (unsigned)std::min<size_t>(TABLE_PIECE, words - o)});
+        return T2X_OK;
+    }
+    template <class T> int add(DevBuf& buf, const std::vector<T>& v) { return add(buf, v.data(), sizeof(T) * v.size()); }
+    int launch(Device* d, hipStream_t st)
+    {
+        const size_t np = pieces.size() * sizeof(TablePiece);
+        T2X_HIP(hipStreamSynchronize(st));   // the last call's kernel has read the buffer
+        T2X_TRY(d->tab_host.ensure(np + 4 * data.size()));
+        std::memcpy(d->tab_host.ptr, pieces.data(), np);
+        std::memcpy(d->tab_host.as<char>() + np, data.data(), 4 * data.size());
+        k_tables<<<(unsigned)pieces.size(), 256, 0, st>>>(d->tab_host.as<TablePiece>(),
+                                                          reinterpret_cast<const unsigned*>(d->tab_host.as<char>() + np));
+        T2X_HIP(hipGetLastError());
+        return T2X_OK;
+    }
+};
+
+static int upload_table(PassTables& t, TableUpload& up)
+{
     std::vector<int2> xy(t.npix);
     for (int i = 0; i < t.npix; i++) xy[i] = make_int2(t.h_x[i], t.h_y[i]);
-    T2X_HIP(hipMemcpyAsync(t.d_pix.ptr, xy.data(), sizeof(int2) * t.npix, hipMemcpyHostToDevice, st));
-    T2X_HIP(hipMemcpyAsync(t.d_win.ptr, t.h_win.data(), sizeof(int) * t.npix, hipMemcpyHostToDevice, st));
-    T2X_HIP(hipMemcpyAsync(t.d_minv.ptr, t.h_minv.data(), sizeof(float) * t.h_minv.size(), hipMemcpyHostToDevice, st));
-    T2X_HIP(hipMemcpyAsync(t.d_ires.ptr, t.h_ires.data(), sizeof(int) * t.npix, hipMemcpyHostToDevice, st));
-    T2X_HIP(hipMemcpyAsync(t.d_inproj.ptr, t.h_inproj.data(), t.npix, hipMemcpyHostToDevice, st));
-    std::vector<int2> gather;
-    if (!t.store) {
-        gather = gather_order(t);
-        T2X_TRY(t.d_gather.ensure(sizeof(int2) * t.npix));
-        T2X_HIP(hipMemcpyAsync(t.d_gather.ptr, gather.data(), sizeof(int2) * t.npix, hipMemcpyHostToDevice, st));
+    // (the order is kept while the pixels are the same)
+    if (!t.store && (!t.gather_ok || xy.size() != t.gather_xy.size() ||
+                     std::memcmp(xy.data(), t.gather_xy.data(), sizeof(int2) * xy.size()) != 0 ||
+                     t.h_inproj != t.gather_inproj)) {
+        t.gather_ok = false;
+        T2X_TRY(up.add(t.d_gather, gather_order(t)));
+        t.gather_xy = xy;
+        t.gather_inproj = t.h_inproj;
     }
+    T2X_TRY(up.add(t.d_pix, xy));
+    T2X_TRY(up.add(t.d_win, t.h_win));
+    T2X_TRY(up.add(t.d_minv, t.h_minv));
+    T2X_TRY(up.add(t.d_ires, t.h_ires));
+    T2X_TRY(up.add(t.d_inproj, t.h_inproj));
     // the frequency window of the pixels: x in [0, size/2], y in [-size/2, size/2]
     t.px_w = t.size / 2 + 1;
     t.py0 = t.size / 2;
     t.py_h = t.size + 1;
-    T2X_HIP(hipStreamSynchronize(st));
     return T2X_OK;
 }
 
@@ -2595,6 +2636,7 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
     // Equal for every class (the first iteration): one translation prior table per particle;
     // otherwise one per (particle, class), tK = K (k_prior_t, trans_prior).
     double class_prior_x = 0., class_prior_y = 0.;
+    TableUpload up;
     int tK = 0;
     if (ref2d && model->prior_offset_class) {
         class_prior_x = model->prior_offset_class[0];
@@ -2609,17 +2651,17 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
                 tK = K;
         if (tK) {
             std::vector<double> cp(model->prior_offset_class, model->prior_offset_class + 2 * K);
-            T2X_TRY(upload(d->cls_prior, cp, st));
+            T2X_TRY(up.add(d->cls_prior, cp));
         }
     }
-    // ---- per-configuration tables ----
+    // ---- per-configuration tables, in one upload ----
     const double* sigma2 = model->sigma2_noise;
     build_table(cc, cs, sigma2, xN, n_og, cfg->sigma2_fudge, false, d->coarse_tab);
     build_table(cs, cs, sigma2, xN, n_og, cfg->sigma2_fudge, true, d->fine_tab);
     PassTables& tc = d->coarse_tab;
     PassTables& tf = d->fine_tab;
-    T2X_TRY(upload_table(tc, st));
-    T2X_TRY(upload_table(tf, st));
+    T2X_TRY(upload_table(tc, up));
+    T2X_TRY(upload_table(tf, up));
     // fine diff2 pixel subset: pixels with minv != 0 come first? (all store pixels are used;
     // the diff2 kernel reads minv of the diff2 definition)
     std::vector<float> minv_diff2((size_t)n_og * tf.npix);
@@ -2629,15 +2671,15 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
     // noise spectra (mask background) and the scale sums' shell mask
     {
         std::vector<double> s2(sigma2, sigma2 + (size_t)n_og * xN);
-        T2X_TRY(upload(d->sigma2_tab, s2, st));
+        T2X_TRY(up.add(d->sigma2_tab, s2));
         if (cfg->do_scale_correction && model->data_vs_prior_class) {
             std::vector<double> dv(model->data_vs_prior_class, model->data_vs_prior_class + (size_t)K * xN);
-            T2X_TRY(upload(d->dvp_tab, dv, st));
+            T2X_TRY(up.add(d->dvp_tab, dv));
         }
     }
     const bool scale_sums = cfg->do_scale_correction && model->data_vs_prior_class;
     DevBuf& d_minv_fd = d->minv_fd;
-    T2X_TRY(upload(d_minv_fd, minv_diff2, st));
+    T2X_TRY(up.add(d_minv_fd, minv_diff2));
     // phase tables (kept from the previous call when its sizes and translations were the same)
     {
         std::vector<double> key = {(double)N, (double)cc, (double)cs, (double)tc.npix, (double)tf.npix,
@@ -2705,28 +2747,25 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
             if (mean_o != 0. && !local) p /= mean_o;
             prior_o[(size_t)c * Norient + o] = scored ? p : 0.;
         }
-    T2X_TRY(upload(d->prior_o, prior_o, st));
+    T2X_TRY(up.add(d->prior_o, prior_o));
     T2X_TRY(d->log_prior_o.ensure(sizeof(double) * std::max<long>(1, O_all)));
-    k_log_prior<<<(unsigned)std::min<long>((O_all + 255) / 256, 65536), 256, 0, st>>>(d->prior_o.as<double>(), O_all,
-                                                                                  d->log_prior_o.as<double>());
-    T2X_HIP(hipGetLastError());
     // device copies of angle tables and class pointer arrays
     DevBuf &d_dirsc = d->dirsc, &d_psisc = d->psisc, &d_ftx = d->ftx, &d_fty = d->fty, &d_vols = d->vols_tab,
            &d_pads = d->pads_tab, &d_bpd = d->bpd_tab, &d_bpw = d->bpw_tab, &d_bpads = d->bpads_tab,
            &d_bprmax = d->bprmax_tab;
-    T2X_TRY(upload(d_dirsc, S.sub_dir_sc, st));
-    T2X_TRY(upload(d_psisc, S.sub_psi_sc, st));
-    T2X_TRY(upload(d_ftx, S.fine_tx_px, st));
-    T2X_TRY(upload(d_fty, S.fine_ty_px, st));
-    T2X_TRY(upload(d_vols, h_vols, st));
-    T2X_TRY(upload(d_pads, h_pads, st));
-    T2X_TRY(upload(d_bpd, h_bpd, st));
-    T2X_TRY(upload(d_bpw, h_bpw, st));
-    T2X_TRY(upload(d_bpads, h_bpads, st));
-    T2X_TRY(upload(d_bprmax, h_bprmax, st));
+    T2X_TRY(up.add(d_dirsc, S.sub_dir_sc));
+    T2X_TRY(up.add(d_psisc, S.sub_psi_sc));
+    T2X_TRY(up.add(d_ftx, S.fine_tx_px));
+    T2X_TRY(up.add(d_fty, S.fine_ty_px));
+    T2X_TRY(up.add(d_vols, h_vols));
+    T2X_TRY(up.add(d_pads, h_pads));
+    T2X_TRY(up.add(d_bpd, h_bpd));
+    T2X_TRY(up.add(d_bpw, h_bpw));
+    T2X_TRY(up.add(d_bpads, h_bpads));
+    T2X_TRY(up.add(d_bprmax, h_bprmax));
     DevBuf &d_ctx = d->ctx, &d_cty = d->cty;   // coarse translations (A) for k_prior_t
-    T2X_TRY(upload(d_ctx, S.tx, st));
-    T2X_TRY(upload(d_cty, S.ty, st));
+    T2X_TRY(up.add(d_ctx, S.tx));
+    T2X_TRY(up.add(d_cty, S.ty));
     LocalSelParams lsp{};
     // local searches score each particle's own sample list (T2X_LOCAL_DENSE=1: the dense pass over
     // every orientation with out-of-range ones masked, kept for comparison)
@@ -2736,7 +2775,7 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
         std::vector<int> cls;
         for (int c = 0; c < K; c++) if (model->pdf_class[c] > 0.) cls.push_back(c);
         Kact = (int)cls.size();
-        T2X_TRY(upload(d->lc_cls, cls, st));
+        T2X_TRY(up.add(d->lc_cls, cls));
         std::vector<double> dsc(4 * Nd), psc(2 * Npsi);
         for (long dd = 0; dd < Nd; dd++) {
             const double a = S.rot[dd] * kPi / 180, b = S.tilt[dd] * kPi / 180;
@@ -2747,14 +2786,14 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
             const double g = S.psi[p] * kPi / 180;
             psc[2 * p] = std::sin(g); psc[2 * p + 1] = std::cos(g);
         }
-        T2X_TRY(upload(d->lc_dirsc, dsc, st));
-        T2X_TRY(upload(d->lc_psisc, psc, st));
+        T2X_TRY(up.add(d->lc_dirsc, dsc));
+        T2X_TRY(up.add(d->lc_psisc, psc));
     }
     if (local) {
         std::vector<double> tab(2 * Nd + Npsi);
         for (long dd = 0; dd < Nd; dd++) { tab[dd] = S.rot[dd]; tab[Nd + dd] = S.tilt[dd]; }
         for (long p = 0; p < Npsi; p++) tab[2 * Nd + p] = S.psi[p];
-        T2X_TRY(upload(d->loc_tab, tab, st));
+        T2X_TRY(up.add(d->loc_tab, tab));
         lsp.dir_rot = d->loc_tab.as<double>();
         lsp.dir_tilt = lsp.dir_rot + Nd;
         lsp.psi = lsp.dir_rot + 2 * Nd;
@@ -2764,6 +2803,12 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
         lsp.sig_dir = ref2d ? 0. : std::max(cfg->sigma_rot, cfg->sigma_tilt);
         lsp.sig_psi = cfg->sigma_psi;
     }
+
+    T2X_TRY(up.launch(d, st));
+    tc.gather_ok = true;
+    k_log_prior<<<(unsigned)std::min<long>((O_all + 255) / 256, 65536), 256, 0, st>>>(d->prior_o.as<double>(), O_all,
+                                                                                  d->log_prior_o.as<double>());
+    T2X_HIP(hipGetLastError());
 
     // ---- pruned coarse pass (t2x_prune.hip): global searches without the proposal or diagnostics ----
     // The low set: the (|frequency|-ordered) coarse pixels within 0.80 of the coarse radius, filled up

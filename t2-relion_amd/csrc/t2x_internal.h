@@ -158,6 +158,9 @@ struct PassTables {
     // diff2 tables: the pixels in the order in which slices are sampled (gather_order), per place the
     // pixel's x | y << 16 and its place in its chunk of GATHER_CHUNK pixels (-1 - place: not projected)
     DevBuf d_gather;
+    bool gather_ok = false;        // d_gather is on the device, for the pixels
+    std::vector<int2> gather_xy;   // gather_xy, gather_inproj
+    std::vector<unsigned char> gather_inproj;
     std::vector<int> h_x, h_y, h_win, h_ires;
     std::vector<float> h_minv;
     std::vector<unsigned char> h_inproj;
@@ -221,6 +224,7 @@ struct Device {
     // the batch's readback: its vectors packed into rb_dev by one kernel, then one copy to rb_host
     DevBuf rb_dev;
     HostBuf rb_host;
+    HostBuf tab_host;   // the call's tables on their way to the device (TableUpload)
     // brick backprojection: item planes, frames and pixel values, the call's bricks, the batch's
     // items by class and its units of work
     DevBuf bp_filt, bp_geom, bp_val, bp_units, bp_cls, bp_boff;
