@@ -691,8 +691,8 @@ def main():
     roof = {"bound": "mfma", "achieved": achieved, "peak": peak, "unit": "TFLOP/s",
             "frac": achieved / peak, "traffic": float(traffic) if traffic else None,
             "traffic_unit": "bytes per launch", "traffic_source": traffic_src,
-            "kernel": ("coarse diff2 of local searches: (particle, orientation) rows x translations, k_local_zrows + "
-                       + ("k_gemm_tn (FP32 MFMA)" if head == "fp32" else "k_gemm_local_x3 (split MFMA, grouped)") + " + k_local_diff2" if local
+            "kernel": ("coarse diff2 of local searches: (particle, orientation) rows x translations, "
+                       + ("k_gemm_local (FP32 MFMA)" if head == "fp32" else "k_gemm_local_x3 (split MFMA, grouped)") + " + k_local_diff2" if local
                        else "coarse diff2 cross term, " + KERNELS.get(f"{hb}/{st.gemm_tile_used}", KERNELS[hb])),
             "gemm_variant": [st.gemm_tile_used, st.gemm_group_used] if st.gemm_tile_used else None,
             "avg_launch_ms": avg_ms, "launches": launches, "flop_per_launch": flop_per_launch,
