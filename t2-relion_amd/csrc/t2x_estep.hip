@@ -2353,6 +2353,9 @@ struct TablePiece {
     unsigned off, words;   // offset in words from the first table
 };
 #define TABLE_PIECE 4096   // words of a workgroup
+// Larger tables (fine samplings' priors: 19 MB at 2.4 million orientations) are copied on their own: the
+// gathering costs them more (12 ms there) than a launch.
+static const size_t kTableGather = 256 << 10;
 
 __global__ __launch_bounds__(256) void k_tables(const TablePiece* __restrict__ pieces, const unsigned* __restrict__ src)
 {
@@ -2363,10 +2366,16 @@ __global__ __launch_bounds__(256) void k_tables(const TablePiece* __restrict__ p
 struct TableUpload {
     std::vector<TablePiece> pieces;
     std::vector<unsigned> data;
+    hipStream_t st;
     int add(DevBuf& buf, const void* v, size_t bytes)
     {
         const size_t words = (bytes + 3) / 4;
         T2X_TRY(buf.ensure(std::max<size_t>(4 * words, 4)));
+        if (bytes > kTableGather) {
+            T2X_HIP(hipMemcpyAsync(buf.ptr, v, bytes, hipMemcpyHostToDevice, st));
+            T2X_HIP(hipStreamSynchronize(st));   // v may go
+            return T2X_OK;
+        }
         const size_t off = data.size();
         data.resize(off + words);
         if (bytes) std::memcpy(&data[off], v, bytes);
@@ -2375,7 +2384,7 @@ struct TableUpload {
         return T2X_OK;
     }
     template <class T> int add(DevBuf& buf, const std::vector<T>& v) { return add(buf, v.data(), sizeof(T) * v.size()); }
-    int launch(Device* d, hipStream_t st)
+    int launch(Device* d)
     {
         const size_t np = pieces.size() * sizeof(TablePiece);
         T2X_HIP(hipStreamSynchronize(st));   // the last call's kernel has read the buffer
@@ -2637,6 +2646,7 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
     // otherwise one per (particle, class), tK = K (k_prior_t, trans_prior).
     double class_prior_x = 0., class_prior_y = 0.;
     TableUpload up;
+    up.st = st;
     int tK = 0;
     if (ref2d && model->prior_offset_class) {
         class_prior_x = model->prior_offset_class[0];
@@ -2804,7 +2814,7 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
         lsp.sig_psi = cfg->sigma_psi;
     }
 
-    T2X_TRY(up.launch(d, st));
+    T2X_TRY(up.launch(d));
     tc.gather_ok = true;
     k_log_prior<<<(unsigned)std::min<long>((O_all + 255) / 256, 65536), 256, 0, st>>>(d->prior_o.as<double>(), O_all,
                                                                                   d->log_prior_o.as<double>());
