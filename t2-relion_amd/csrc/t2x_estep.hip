@@ -396,6 +396,12 @@ __global__ __launch_bounds__(256) void k_project_coarse(const float2* const* __r
 // of 10,000 pixels in BF16 (3000 particles of 113 translations): 25 -> 12.1 ms; of 1,450 in FP16 (8192
 // particles of 88): 5.3 -> 2.9 ms (gathered by every row group and pass: 3.6).
 #define IMG_TG 8
+// u - h of the rounded value u (never fused with the product that made it: the low half is u's own rest).
+__device__ __forceinline__ float split_rest(float u, float h)
+{
+#pragma clang fp contract(off)
+    return u - h;
+}
 #define IMG_CHUNK 2048
 template <class H, int FORM>
 __global__ __launch_bounds__(256) void k_coarse_imgside(const float2* __restrict__ Fimg,
@@ -506,7 +512,7 @@ __global__ __launch_bounds__(256) void k_coarse_imgside(const float2* __restrict
                             for (int k = 0; k < 8; k++) {
                                 const float u = FORM == 1 ? v[k] * sc[j] : v[k];
                                 h[k] = (H)u;
-                                d[k] = (H)(u - (float)h[k]);
+                                d[k] = (H)split_rest(u, (float)h[k]);
                             }
                             *reinterpret_cast<v8*>(hi + o) = h;
                             *reinterpret_cast<v8*>(lo + o) = d;
