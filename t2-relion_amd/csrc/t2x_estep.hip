@@ -4005,16 +4005,16 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
         return T2X_OK;
         };
         // graph mode: global searches without the proposal and without diagnostics; a batch
-        // size is captured only after it ran once eagerly in this call (the GEMM autotuner
-        // has timed its shapes), and a graph is replayed only while no device buffer has
-        // been reallocated since its capture
+        // size is captured only after it ran once eagerly in this call with the same coarse GEMM,
+        // listed or exhaustive (the GEMM autotuner has timed its shapes), and a graph is
+        // replayed only while no device buffer has been reallocated since its capture
         const bool gmode = cfg->launch_graph && !local && !use_prop && !(dbg && dbg->n_debug > 0);
         bool graph_used = false;
         for (int attempt = 0;; attempt++) {
         if (attempt == 0) {
             const bool replay = gmode && d->graph_exec && d->graph_call == call_id && d->graph_B == B &&
                                 d->graph_prune == prune_batch && d->graph_gen == alloc_generation();
-            if (replay || (gmode && d->eager_B.count(B))) {
+            if (replay || (gmode && d->eager_B.count({B, prune_batch}))) {
                 if (!replay) {
                     destroy_graph(d);
                     T2X_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeRelaxed));
@@ -4051,7 +4051,7 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
                 T2X_TRY(coarse_part());
                 ev_plan = ev;
                 T2X_TRY(post_part());
-                if (gmode) d->eager_B.insert(B);
+                if (gmode) d->eager_B.insert({B, prune_listed});
             }
         } else {
             ev = ev_plan;

@@ -1720,6 +1720,14 @@ int launch_gemm_x3(int prec, int epi, const void* Ah, const void* Al, const floa
             return launch_x3_variant(prec, epi, A, B, K, Mrows_pad, Nrows_pad, ep, st, hit.tile, hit.group, rowmap);
         }
     }
+    // nothing can be timed on a stream that is being captured: the default variant, not kept
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    T2X_HIP(hipStreamIsCapturing(st, &cap));
+    if (cap != hipStreamCaptureStatusNone) {
+        c = {off32 ? 258 : 256, 32};
+        if (used) *used = c;
+        return launch_x3_variant(prec, epi, A, B, K, Mrows_pad, Nrows_pad, ep, st, c.tile, c.group, rowmap);
+    }
     GemmChoice best{0, 0};
     float best_ms = 3.0e38f;
     hipEvent_t e0, e1;

@@ -244,7 +244,7 @@ struct Device {
     hipGraphExec_t graph_exec = nullptr;
     int graph_B = 0;
     unsigned long long graph_gen = 0, graph_call = 0, call_counter = 0;
-    std::set<int> eager_B;
+    std::set<std::pair<int, bool>> eager_B;   // (batch size, tile list or exhaustive coarse GEMM) run eagerly in this call
 
     // cached coarse projections
     std::string coarse_key;

@@ -114,6 +114,33 @@ def test_pruned_graph_replays_count_tiles(gpu_device, monkeypatch):
     same(graph, eager)
 
 
+@pytest.mark.parametrize("prec", [T.T2X_PREC_FP32, T.T2X_PREC_FP16X2, T.T2X_PREC_BF16X3])
+def test_later_batches_that_do_not_prune(gpu_device, monkeypatch, prec):
+    """Five batches, of which the first two prune and the particles of the others (an optics group of
+    thirty times the noise) do not: the pass is turned off after the third, and the exhaustive GEMM of
+    the last two, whose shape has not been tuned in the process, runs eagerly before it is captured."""
+    lib = T.load()
+    monkeypatch.setenv("T2X_BATCH", "24")
+    wl = H.Workload("refine64", n=120, seed_offset=87, precision=prec, snr=1.0, overrides=dict(healpix_order=3))
+    later = (np.arange(120) >= 48).astype(int)
+    wl.set_groups([wl.sigma2, 30.0 * wl.sigma2], group_of=np.zeros(120, int), optics_of=later)
+    tiles = 16 * 288   # of a batch: 24 x 81 rows and 36,864 orientations, 128 x 128
+    wl.cfg.launch_graph = 1
+    graph, cnt_g = run(wl, gpu_device, False)   # first, so that no exhaustive launch has been tuned
+    wl.cfg.launch_graph = 0
+    st = T.Stats()
+    T.check(lib.t2x_stats_get(gpu_device, C.byref(st)))
+    eager, cnt_e = run(wl, gpu_device, False)
+    ex, _ = run(wl, gpu_device, True)
+    print(f"\n[prune] precision {prec}: {st.n_graph_launches} graph launches, {cnt_g[0]:.0f} of {cnt_g[1]:.0f} tiles "
+          f"pruned (eager {cnt_e[0]:.0f} of {cnt_e[1]:.0f})")
+    assert st.n_graph_launches == 3   # batches 2 (captured), 3 (replayed) and 5 (captured)
+    assert cnt_g[1] == cnt_e[1] == 3 * tiles
+    assert 1.7 * tiles < cnt_g[0] < 2.1 * tiles and cnt_g[0] == cnt_e[0]
+    same(graph, ex)
+    same(eager, ex)
+
+
 @pytest.mark.parametrize("tile", ["259", "258"])
 def test_pruned_other_bounds_kernels(gpu_device, monkeypatch, tile):
     """The bounds GEMM as k_gemm_x2h<true> (128x256 tiles) or as k_gemm_x3p with one K chunk per
