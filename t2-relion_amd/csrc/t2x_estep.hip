@@ -45,7 +45,8 @@ int launch_gemm_x3(int prec, int epi, const void* Ah, const void* Al, const floa
                    const int* rowmap, GemmChoice* used);
 int launch_gemm_pruned(int prec, const void* Ah, const void* Al, const float* As, long long lda, const void* Bh,
                        const void* Bl, const float* Bs, long long ldb, int K, int Mrows_pad, int Nrows_pad,
-                       const EpiParams& ep, const unsigned* list, const unsigned* count, int n_cu, hipStream_t st);
+                       const EpiParams& ep, const unsigned* list, const unsigned* count, unsigned most, int n_cu,
+                       hipStream_t st);
 int launch_gemm_local_f32(const float2* F, const float2* Y, const double* W, int B, const long long* orient_off,
                           const int* rowu, long long rows, const float* ab, int Kc, int Tl, const EpiParams& ep,
                           double* n1, hipStream_t st);
@@ -3060,9 +3061,9 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
         const long long prune_ntiles =
             prune_batch ? (round_up((long long)B * T, 256) / PRUNED_TILE) * (O_pad / PRUNED_TILE) : 0;
         // Most tiles that the listed GEMM may keep: a listed tile of the split precisions costs about six
-        // times its share of the exhaustive GEMM (128 x 128 tiles picked one by one; 4096 particles of a
-        // 72 box, all tiles kept: 9.7 against 1.6 ms), an FP32 one the same, and the bounds come on top.
-        const double prune_most = prec == T2X_PREC_FP32 ? 0.6 : 0.15;
+        // times its share of the exhaustive GEMM (launch_gemm_pruned), an FP32 one the same, and the
+        // bounds come on top.
+        const unsigned prune_most = (unsigned)((prec == T2X_PREC_FP32 ? 0.6 : 0.15) * (double)prune_ntiles);
         bool prune_listed = prune_batch;
         const size_t NN = (size_t)N * N;
         int ev = 0;
@@ -3558,12 +3559,12 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
                     pc.force = prune_force;
                     T2X_TRY(prune_bounds(d, pc, d_ps, tc, Pw, st));
                     // the call's first batch looks at what the bounds left before it takes the list; the
-                    // later ones go by the batch before them
+                    // later ones go by the batch before them, and on the device by their own list
                     if (b0 == 0 && !capturing && !prune_force) {
                         unsigned kept = 0;
                         T2X_HIP(hipMemcpyAsync(&kept, d->prune.cnt.ptr, sizeof(unsigned), hipMemcpyDeviceToHost, st));
                         T2X_HIP(hipStreamSynchronize(st));
-                        prune_listed = (double)kept <= prune_most * (double)prune_ntiles;
+                        prune_listed = kept <= prune_most;
                     }
                 }
                 if (prune_listed) {
@@ -3571,7 +3572,8 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
                     T2X_TRY(launch_gemm_pruned(prec, f32 ? d->A.ptr : d->Ah.ptr, d->Al.ptr, d->As.as<float>(), Kc,
                                                f32 ? d->coarse_B.ptr : d->coarse_Bh.ptr, d->coarse_Bl.ptr,
                                                d->coarse_Bs.as<float>(), Kc, Kc, (int)M_pad, (int)O_pad, ep,
-                                               d->prune.list.as<unsigned>(), d->prune.cnt.as<unsigned>(), d->n_cu, st));
+                                               d->prune.list.as<unsigned>(), d->prune.cnt.as<unsigned>(),
+                                               prune_force ? 0xffffffffu : prune_most, d->n_cu, st));
                     if (!f32) {   // group 0: the tile list
                         d->stats.s.gemm_tile_used = PRUNED_TILE;
                         d->stats.s.gemm_group_used = 0;
@@ -4089,12 +4091,17 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
         nitems = hplan.nitems;
         if (bp_bricks) stt.bp_brick_items += (double)std::min(nitems, bp_item_cap);
         if (prune_batch) {
-            const double skipped = (double)prune_ntiles - (double)hprune;
-            if (prune_listed) stt.coarse_tiles_pruned += skipped;
+            const bool short_list = hprune <= prune_most || prune_force;
+            if (prune_listed && (short_list || prec == T2X_PREC_FP32))
+                stt.coarse_tiles_pruned += (double)prune_ntiles - (double)hprune;
+            else if (prune_listed) {   // all tiles, by k_gemm_x3p
+                stt.gemm_tile_used = 258;
+                stt.gemm_group_used = 32;
+            }
             stt.coarse_tiles_checked += (double)prune_ntiles;
             stt.coarse_bound_flop += 4.0 * (double)T * (double)O_all * (double)n_low * B;
             // a pass that prunes little does not pay for its bounds: off for the call's rest
-            if (!prune_force && (double)hprune > prune_most * (double)prune_ntiles) prune_call = false;
+            if (!short_list) prune_call = false;
         }
         if (!cand_path) {
             stt.n_select_fallbacks += 1;

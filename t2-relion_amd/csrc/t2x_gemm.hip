@@ -458,7 +458,7 @@ __device__ __forceinline__ void x3_tile(H (&st)[NP + 1][GBM][XK + XPAD], const S
 }
 
 // LIST (the pruned coarse pass): a persistent grid over the tiles listed in ep.tile_list
-// (*ep.tile_count of them, indices tm * tiles_n + tn).
+// (*ep.tile_count of them, at most ep.tile_most, indices tm * tiles_n + tn).
 template <class H, int EPI, int NP = 3, bool LIST = false>
 __global__ __launch_bounds__(256) void k_gemm_x3(SplitOperand A, SplitOperand B, int K, int tiles_m,
                                                  int tiles_n, int group_m, EpiParams ep)
@@ -466,6 +466,7 @@ __global__ __launch_bounds__(256) void k_gemm_x3(SplitOperand A, SplitOperand B,
     __shared__ __attribute__((aligned(16))) H st[NP + 1][GBM][XK + XPAD];
     if constexpr (LIST) {
         const unsigned n = *ep.tile_count;
+        if (n > ep.tile_most) return;
         for (unsigned it = blockIdx.x; it < n; it += gridDim.x) {
             const unsigned t = ep.tile_list[it];
             x3_tile<H, EPI, NP>(st, A, B, K, (long long)(t / (unsigned)tiles_n) * GBM,
@@ -1008,7 +1009,9 @@ __device__ __forceinline__ void x3p_tile(H (&st0)[4][WBM * 32], H (&st1)[4][WBM 
         gemm_epilogue<8, EPI>(acc, m0 + wm * 128, n0 + wn * 64, lane, A.inv_scale, B.inv_scale, ep, rowmap);
 }
 
-template <class H, int EPI, int NP = 3>
+// ALL (the pruned coarse pass, after the listed launch): a persistent grid over every tile where the
+// list was too long for that launch, nothing otherwise.
+template <class H, int EPI, int NP = 3, bool ALL = false>
 __global__ __launch_bounds__(512) void k_gemm_x3p(SplitOperand A, SplitOperand B, int K, int tiles_m,
                                                   int tiles_n, int group_m, EpiParams ep,
                                                   const int* __restrict__ rowmap)
@@ -1017,8 +1020,17 @@ __global__ __launch_bounds__(512) void k_gemm_x3p(SplitOperand A, SplitOperand B
     __shared__ __attribute__((aligned(16))) H st1[4][WBM * 32];
     __shared__ EpiStage es;
     int tm, tn;
-    tile_coords(blockIdx.x, tiles_m, tiles_n, group_m, tm, tn);
-    x3p_tile<H, EPI, NP>(st0, st1, es, A, B, K, (long long)tm * WBM, (long long)tn * WBN, ep, rowmap);
+    if constexpr (ALL) {
+        if (*ep.tile_count <= ep.tile_most) return;
+        for (int t = blockIdx.x; t < tiles_m * tiles_n; t += gridDim.x) {
+            tile_coords(t, tiles_m, tiles_n, group_m, tm, tn);
+            x3p_tile<H, EPI, NP>(st0, st1, es, A, B, K, (long long)tm * WBM, (long long)tn * WBN, ep, nullptr);
+            __syncthreads();   // the next tile reuses the LDS stages
+        }
+    } else {
+        tile_coords(blockIdx.x, tiles_m, tiles_n, group_m, tm, tn);
+        x3p_tile<H, EPI, NP>(st0, st1, es, A, B, K, (long long)tm * WBM, (long long)tn * WBN, ep, rowmap);
+    }
 }
 
 // Two-product half-height variant (FP16X2 only): tile 128 (M) x 256 (N), 4 waves of 64 x 128,
@@ -1600,10 +1612,14 @@ static int launch_x3_variant(int prec, int epi, const SplitOperand& A, const Spl
 // products under FP16X2, else 3) or k_gemm_tn. Small tiles, since a tile is computed for any one of its
 // 64-column blocks: at class256 0.9% of the 128x128 tiles and 2.8% of the 256x256 ones are (0.73
 // against 1.06 ms per 800 particles with k_gemm_x3p, for all its faster K loop; 3 products at 500
-// particles 1.60 against 2.06 ms).
+// particles 1.60 against 2.06 ms). A list of more than `most` tiles of a split precision, which the
+// launch cannot know (a listed tile costs about six times its share of the exhaustive GEMM, so a full
+// list 9.7 ms against 1.6 for 4096 particles of a 72 box), is left to a persistent k_gemm_x3p over all
+// tiles, at the exhaustive GEMM's cost; that launch otherwise ends at once.
 int launch_gemm_pruned(int prec, const void* Ah, const void* Al, const float* As, long long lda, const void* Bh,
                        const void* Bl, const float* Bs, long long ldb, int K, int Mrows_pad, int Nrows_pad,
-                       const EpiParams& ep, const unsigned* list, const unsigned* count, int n_cu, hipStream_t st)
+                       const EpiParams& ep, const unsigned* list, const unsigned* count, unsigned most, int n_cu,
+                       hipStream_t st)
 {
     const bool fp32 = prec == T2X_PREC_FP32;
     const long long lim = 1LL << 32;   // as the exhaustive FP16X2 GEMM, which the call's other batches may take
@@ -1612,7 +1628,7 @@ int launch_gemm_pruned(int prec, const void* Ah, const void* Al, const float* As
         return T2X_EINVAL;
     }
     static_assert(PRUNED_TILE == GBM && PRUNED_TILE == GBN, "tile of k_gemm_tn and k_gemm_x3");
-    if (K % (fp32 ? GBK : XK) != 0 || Mrows_pad % GBM != 0 || Nrows_pad % GBN != 0) {
+    if (K % (fp32 ? GBK : XK) != 0 || Mrows_pad % WBM != 0 || Nrows_pad % WBN != 0) {
         set_error("gemm_pruned: operands not padded to tile multiples");
         return T2X_EINVAL;
     }
@@ -1624,6 +1640,7 @@ int launch_gemm_pruned(int prec, const void* Ah, const void* Al, const float* As
     EpiParams el = ep;
     el.tile_list = list;
     el.tile_count = count;
+    el.tile_most = most;
     SplitOperand A{Ah, Al, As, lda}, B{Bh, Bl, Bs, ldb};
     if (fp32)
         k_gemm_tn<EPI_DIFF2, true><<<(unsigned)(4 * n_cu), 256, 0, st>>>((const float*)Ah, lda, (const float*)Bh, ldb, K,
@@ -1634,6 +1651,13 @@ int launch_gemm_pruned(int prec, const void* Ah, const void* Al, const float* As
         k_gemm_x3<__bf16, EPI_DIFF2, 3, true><<<(unsigned)(3 * n_cu), 256, 0, st>>>(A, B, K, tm, tn, 0, el);
     else
         k_gemm_x3<_Float16, EPI_DIFF2, 3, true><<<(unsigned)(3 * n_cu), 256, 0, st>>>(A, B, K, tm, tn, 0, el);
+    const int wm = Mrows_pad / WBM, wn = Nrows_pad / WBN;
+    if (prec == T2X_PREC_FP16X2)
+        k_gemm_x3p<_Float16, EPI_DIFF2, 2, true><<<(unsigned)n_cu, 512, 0, st>>>(A, B, K, wm, wn, 32, el, nullptr);
+    else if (prec == T2X_PREC_BF16X3)
+        k_gemm_x3p<__bf16, EPI_DIFF2, 3, true><<<(unsigned)n_cu, 512, 0, st>>>(A, B, K, wm, wn, 32, el, nullptr);
+    else if (!fp32)
+        k_gemm_x3p<_Float16, EPI_DIFF2, 3, true><<<(unsigned)n_cu, 512, 0, st>>>(A, B, K, wm, wn, 32, el, nullptr);
     T2X_HIP(hipGetLastError());
     return T2X_OK;
 }

@@ -172,9 +172,11 @@ struct EpiParams {
     // stored (the block minimum still is, so every reader skips the block). null: store all.
     unsigned int* pmin;
     // Pruned coarse pass: the tiles a list-driven (persistent) launch computes, *tile_count of
-    // them (read by the kernels of the LIST form only).
+    // them; with more than tile_most it computes none, and the launch after it all tiles (read by
+    // the kernels of these two forms only).
     const unsigned int* tile_list;
     const unsigned int* tile_count;
+    unsigned int tile_most;
 };
 
 // Rows and columns of the tiles of the pruned coarse pass's full GEMM.

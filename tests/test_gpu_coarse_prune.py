@@ -141,6 +141,25 @@ def test_later_batches_that_do_not_prune(gpu_device, monkeypatch, prec):
     same(eager, ex)
 
 
+@pytest.mark.parametrize("prec", [T.T2X_PREC_FP16X2, T.T2X_PREC_FP16X3, T.T2X_PREC_BF16X3])
+def test_long_list_runs_all_tiles(gpu_device, monkeypatch, prec):
+    """A batch behind one that pruned, with a list too long for the listed GEMM: all tiles, by the
+    256 x 256 kernel (258), with the exhaustive pass's results."""
+    lib = T.load()
+    monkeypatch.setenv("T2X_BATCH", "24")
+    wl = H.Workload("refine64", n=48, seed_offset=88, precision=prec, snr=1.0, overrides=dict(healpix_order=3))
+    later = (np.arange(48) >= 24).astype(int)
+    wl.set_groups([wl.sigma2, 30.0 * wl.sigma2], group_of=np.zeros(48, int), optics_of=later)
+    pr, cnt = run(wl, gpu_device, False)
+    st = T.Stats()
+    T.check(lib.t2x_stats_get(gpu_device, C.byref(st)))
+    ex, _ = run(wl, gpu_device, True)
+    tiles = 16 * 288
+    assert cnt[1] == 2 * tiles and 0.85 * tiles < cnt[0] < tiles
+    assert st.gemm_tile_used == 258
+    same(pr, ex)
+
+
 @pytest.mark.parametrize("tile", ["259", "258"])
 def test_pruned_other_bounds_kernels(gpu_device, monkeypatch, tile):
     """The bounds GEMM as k_gemm_x2h<true> (128x256 tiles) or as k_gemm_x3p with one K chunk per
