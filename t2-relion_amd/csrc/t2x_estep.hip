@@ -2829,19 +2829,28 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
 
     // ---- pruned coarse pass (t2x_prune.hip): global searches without the proposal or diagnostics ----
     // The low set: the (|frequency|-ordered) coarse pixels within 0.80 of the coarse radius, filled up
-    // to whole K steps of the INT8 GEMM.
-    int n_low = 0, K8 = 0;
+    // to whole K steps of the INT8 GEMM, or as many as there are. The first costs less where it prunes
+    // enough (class256 in FP16X2, the GEMM stage 7.0 ms a batch against 9.8), the second keeps fewer tiles
+    // where the references have power up to the coarse radius (586 particles of a 106 box, K = 4: 5%
+    // against 36%).
+    int n_low[2] = {0, 0}, K8[2] = {0, 0};
     const bool prune_force = getenv("T2X_PRUNE_FORCE") != nullptr;   // tests: every batch, whatever it prunes
     bool prune_call = !cfg->coarse_exhaustive && !local && !use_prop && !(dbg && dbg->n_debug > 0);
+    int prune_set = -1;   // the call's low set, once its first batch has been looked at
     if (prune_call) {
         double frac = 0.80;
         const char* env_pr = getenv("T2X_PRUNE_RADIUS");   // fraction of the coarse radius
         if (env_pr && atof(env_pr) > 0.) frac = atof(env_pr);
         const double rl = frac * (cc / 2.0);
-        while (n_low < tc.npix && tc.h_x[n_low] * tc.h_x[n_low] + tc.h_y[n_low] * tc.h_y[n_low] <= rl * rl) n_low++;
-        K8 = (int)std::min<long long>(round_up(2LL * n_low, 128), 16384);   // 16,384: the image side's LDS row
-        n_low = std::min(tc.npix, K8 / 2);
-        if (n_low < 16) prune_call = false;
+        while (n_low[0] < tc.npix && tc.h_x[n_low[0]] * tc.h_x[n_low[0]] + tc.h_y[n_low[0]] * tc.h_y[n_low[0]] <= rl * rl)
+            n_low[0]++;
+        n_low[1] = tc.npix;
+        for (int k = 0; k < 2; k++) {
+            K8[k] = (int)std::min<long long>(round_up(2LL * n_low[k], 128), 16384);   // 16,384: the image side's LDS row
+            n_low[k] = std::min(tc.npix, K8[k] / 2);
+        }
+        if (n_low[0] < 16) prune_call = false;
+        if (prune_force) prune_set = 0;
     }
 
     // ---- coarse projections, cached across calls ----
@@ -2903,22 +2912,16 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
         d->coarse_key = key;
         d->prune_key.clear();
     }
-    // The pruned coarse pass of a batch of B particles: its ten launches and the bounds GEMM pay where the
-    // exhaustive GEMM takes longer than about 0.15 ms (110 TFLOP/s in FP32, 1,150 TFLOP/s a product).
-    auto prune_pays = [&](int B) {
-        const double gemm_flop = 4. * (double)T * (double)O_all * (double)tc.npix * B;
-        const double gemm_rate = prec == T2X_PREC_FP32 ? 110e12 : (prec == T2X_PREC_FP16X2 ? 575e12 : 383e12);
-        return prune_force || gemm_flop > 1.5e-4 * gemm_rate;
+    // The pruned coarse pass pays for a call, whose first batch samples it for 0.2 to 0.3 ms (the reference
+    // side, ten small launches, two readbacks), where the exhaustive GEMM takes longer than about 0.8 ms in
+    // all, and for a batch, whose ten launches and bounds GEMM cost 0.1 ms and more, above 0.15 ms (by 110
+    // TFLOP/s in FP32, 1,150 TFLOP/s a product). 434 particles of an 82 box in FP32 (0.7 ms, 93% of the
+    // tiles kept): 6.65 ms a call, with the sample 6.96.
+    auto gemm_ms = [&](int B) {
+        const double gemm_rate = prec == T2X_PREC_FP32 ? 110e9 : (prec == T2X_PREC_FP16X2 ? 575e9 : 383e9);
+        return 4. * (double)T * (double)O_all * (double)tc.npix * B / gemm_rate;
     };
-    if (!prune_pays(n)) prune_call = false;   // no batch is larger: the reference side (30 us) is not needed either
-    if (prune_call) {
-        const std::string pkey = key + "/" + std::to_string(n_low);
-        if (pkey != d->prune_key) {
-            d->prune_key.clear();
-            T2X_TRY(prune_prepare_refs(d, O_all, O_pad, Kc, Kn, n_low, K8, st));
-            d->prune_key = pkey;
-        }
-    }
+    if (!prune_force && gemm_ms(n) < (prec == T2X_PREC_FP32 ? 1. : 0.45)) prune_call = false;
     (void)hipEventRecord(d->ev[1], st);
     {
         float ms = 0;
@@ -3056,15 +3059,20 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
 
     for (int b0 = 0; b0 < n; b0 += Bmax) {
         const int B = std::min(Bmax, n - b0);
-        const bool prune_batch = prune_call && prune_pays(B);
-        // its full GEMM's tiles, known here for graph replays too
-        const long long prune_ntiles =
-            prune_batch ? (round_up((long long)B * T, 256) / PRUNED_TILE) * (O_pad / PRUNED_TILE) : 0;
-        // Most tiles that the listed GEMM may keep: a listed tile of the split precisions costs about six
-        // times its share of the exhaustive GEMM (launch_gemm_pruned), an FP32 one the same, and the
-        // bounds come on top.
-        const unsigned prune_most = (unsigned)((prec == T2X_PREC_FP32 ? 0.6 : 0.15) * (double)prune_ntiles);
-        bool prune_listed = prune_batch;
+        // (the first batch may find that it does not pay)
+        bool prune_batch = prune_call && (prune_force || gemm_ms(B) > 0.15);
+        // the full GEMM's tiles that hold rows of B particles and orientations (for graph replays too)
+        auto tiles_of = [&](int b) {
+            const long long tile = PRUNED_TILE;
+            return ((long long)b * T + tile - 1) / tile * ((O_all + tile - 1) / tile);
+        };
+        const long long prune_ntiles = prune_batch ? tiles_of(B) : 0;
+        // Most of them that the listed GEMM may keep: a listed tile of the split precisions costs 1.6 to 1.9
+        // times its share of the exhaustive GEMM, an FP32 one the same, and the bounds cost 0.2 to 0.3 of
+        // it (split; bounds and list against the exhaustive GEMM: 36% kept 3.5 and 4.4 ms, 51% 1.6 and
+        // 2.2, 58% 9.2 and 7.3).
+        const double prune_share = prec == T2X_PREC_FP32 ? 0.6 : 0.35;
+        const unsigned prune_most = (unsigned)(prune_share * (double)prune_ntiles);
         const size_t NN = (size_t)N * N;
         int ev = 0;
         (void)hipEventRecord(d->ev[ev++], st);
@@ -3539,35 +3547,72 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
                 k_fill_f32<<<(unsigned)((M_pad * rowmin_ld + 255) / 256), 256, 0, st>>>(d_rowmin.as<float>(), 3.0e38f,
                                                                                         M_pad * rowmin_ld);
                 if (prune_batch) {
-                    // bounds, seeds and the list of the tiles to compute; a tile that is not keeps +inf minima
-                    k_const_term<<<B, 256, 0, st>>>(d->Fimg_cur.as<float2>(), Pw, tc.d_win.as<int>(),
-                                                    tc.d_minv.as<float>(), tc.npix, d_ps, 2, n_low);
-                    T2X_HIP(hipGetLastError());
                     T2X_TRY(d->prune.cnt.ensure(sizeof(unsigned) * 2));
-                    T2X_TRY(zero_async(d->prune.cnt.ptr, sizeof(unsigned) * 2, st));
-                    PruneCall pc{};
-                    pc.prec = prec;
-                    pc.B = B;
-                    pc.T = (int)T;
-                    pc.M_pad = M_pad;
-                    pc.O_all = O_all;
-                    pc.O_pad = O_pad;
-                    pc.Kn = Kn;
-                    pc.n_low = n_low;
-                    pc.K8 = K8;
-                    pc.Cb = ep.Cb;
-                    pc.force = prune_force;
-                    T2X_TRY(prune_bounds(d, pc, d_ps, tc, Pw, st));
-                    // the call's first batch looks at what the bounds left before it takes the list; the
-                    // later ones go by the batch before them, and on the device by their own list
-                    if (b0 == 0 && !capturing && !prune_force) {
-                        unsigned kept = 0;
-                        T2X_HIP(hipMemcpyAsync(&kept, d->prune.cnt.ptr, sizeof(unsigned), hipMemcpyDeviceToHost, st));
+                    // bounds, seeds and the list of the tiles to compute, for Bs particles of the batch
+                    auto call = [&](int k, int Bs) {
+                        return PruneCall{prec, Bs, (int)T, B / Bs, round_up((long long)Bs * T, 256), O_all, O_pad, Kn,
+                                         n_low[k], K8[k], ep.Cb};
+                    };
+                    auto bounds = [&](int k, int Bs) -> int {
+                        T2X_TRY(zero_async(d->prune.cnt.ptr, sizeof(unsigned) * 2, st));
+                        k_const_term<<<B, 256, 0, st>>>(d->Fimg_cur.as<float2>(), Pw, tc.d_win.as<int>(),
+                                                        tc.d_minv.as<float>(), tc.npix, d_ps, 2, n_low[k]);
+                        T2X_HIP(hipGetLastError());
+                        const std::string pkey = key + "/" + std::to_string(n_low[k]);
+                        if (pkey != d->prune_key) {
+                            d->prune_key.clear();
+                            T2X_TRY(prune_prepare_refs(d, O_all, O_pad, Kc, Kn, n_low[k], K8[k], st));
+                            d->prune_key = pkey;
+                        }
+                        T2X_TRY(prune_bounds(d, call(k, Bs), d_ps, tc, Pw, st));
+                        if (!capturing)
+                            stt.coarse_bound_flop += 4.0 * (double)T * (double)O_all * (double)n_low[k] * Bs;
+                        return T2X_OK;
+                    };
+                    unsigned h[2];
+                    auto counts = [&]() -> int {
+                        T2X_HIP(hipMemcpyAsync(h, d->prune.cnt.ptr, sizeof(h), hipMemcpyDeviceToHost, st));
                         T2X_HIP(hipStreamSynchronize(st));
-                        prune_listed = kept <= prune_most;
+                        return T2X_OK;
+                    };
+                    // The call's first batch (which is never captured) decides by a sample of its
+                    // particles: the share of tiles that the first low set keeps and, where that is over a
+                    // fifth and a quarter of the sample loses by the high set, the second set's, taken if
+                    // it halves the share. Two to five tiles a compute unit (512 to 2,048 rows) and eight
+                    // particles; where that is over a quarter of the batch, all of it. (725 particles of a 106 box
+                    // in FP32, which keep 79% by the first set: the bounds of all, for nothing, had cost
+                    // 0.9 of 24.5 ms.)
+                    bool bounded = false;   // the batch's bounds are there
+                    if (prune_set < 0) {
+                        const long long rows = std::max(512LL, std::min(2048LL, (2048LL << 14) / O_all));
+                        int Bs = (int)std::max(8LL, rows / T);
+                        if (4 * Bs > B) Bs = B;
+                        double share = 1.;
+                        for (int k = 0; k < 2; k++) {
+                            if (k == 1) {
+                                if (share <= 0.2 || n_low[1] == n_low[0]) break;
+                                T2X_TRY(prune_high(d, call(0, Bs), d_ps, tc, st));
+                                T2X_TRY(counts());
+                                if (4 * h[1] < (unsigned)Bs) break;
+                            }
+                            T2X_TRY(bounds(k, Bs));
+                            T2X_TRY(counts());
+                            const double kept = (double)h[0] / (double)tiles_of(Bs);
+                            bounded = false;
+                            if (kept <= prune_share && (prune_set < 0 || kept < 0.5 * share)) {
+                                prune_set = k;
+                                bounded = Bs == B;
+                            }
+                            share = kept;
+                        }
+                        if (prune_set < 0) {
+                            prune_call = prune_batch = false;
+                            stt.coarse_tiles_checked += (double)tiles_of(Bs);
+                        }
                     }
+                    if (prune_batch && !bounded) T2X_TRY(bounds(prune_set, B));
                 }
-                if (prune_listed) {
+                if (prune_batch) {   // a tile that is not listed keeps +inf minima
                     const bool f32 = prec == T2X_PREC_FP32;
                     T2X_TRY(launch_gemm_pruned(prec, f32 ? d->A.ptr : d->Ah.ptr, d->Al.ptr, d->As.as<float>(), Kc,
                                                f32 ? d->coarse_B.ptr : d->coarse_Bh.ptr, d->coarse_Bl.ptr,
@@ -4053,7 +4098,7 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
                 T2X_TRY(coarse_part());
                 ev_plan = ev;
                 T2X_TRY(post_part());
-                if (gmode) d->eager_B.insert({B, prune_listed});
+                if (gmode) d->eager_B.insert({B, prune_batch});
             }
         } else {
             ev = ev_plan;
@@ -4092,14 +4137,14 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
         if (bp_bricks) stt.bp_brick_items += (double)std::min(nitems, bp_item_cap);
         if (prune_batch) {
             const bool short_list = hprune <= prune_most || prune_force;
-            if (prune_listed && (short_list || prec == T2X_PREC_FP32))
+            if (short_list || prec == T2X_PREC_FP32)
                 stt.coarse_tiles_pruned += (double)prune_ntiles - (double)hprune;
-            else if (prune_listed) {   // all tiles, by k_gemm_x3p
+            else {   // all tiles, by k_gemm_x3p
                 stt.gemm_tile_used = 258;
                 stt.gemm_group_used = 32;
             }
             stt.coarse_tiles_checked += (double)prune_ntiles;
-            stt.coarse_bound_flop += 4.0 * (double)T * (double)O_all * (double)n_low * B;
+            if (graph_used) stt.coarse_bound_flop += 4.0 * (double)T * (double)O_all * (double)n_low[prune_set] * B;
             // a pass that prunes little does not pay for its bounds: off for the call's rest
             if (!short_list) prune_call = false;
         }

@@ -1613,9 +1613,9 @@ static int launch_x3_variant(int prec, int epi, const SplitOperand& A, const Spl
 // 64-column blocks: at class256 0.9% of the 128x128 tiles and 2.8% of the 256x256 ones are (0.73
 // against 1.06 ms per 800 particles with k_gemm_x3p, for all its faster K loop; 3 products at 500
 // particles 1.60 against 2.06 ms). A list of more than `most` tiles of a split precision, which the
-// launch cannot know (a listed tile costs about six times its share of the exhaustive GEMM, so a full
-// list 9.7 ms against 1.6 for 4096 particles of a 72 box), is left to a persistent k_gemm_x3p over all
-// tiles, at the exhaustive GEMM's cost; that launch otherwise ends at once.
+// launch cannot know (a listed tile costs 1.6 to 1.9 times its share of the exhaustive GEMM), is left to
+// a persistent k_gemm_x3p over all tiles, at the exhaustive GEMM's cost; that launch otherwise ends at
+// once. (200 particles of a 64 box at HEALPix 3, every tile kept: 3.2 -> 1.9 ms in FP16X2.)
 int launch_gemm_pruned(int prec, const void* Ah, const void* Al, const float* As, long long lda, const void* Bh,
                        const void* Bl, const float* Bs, long long ldb, int K, int Mrows_pad, int Nrows_pad,
                        const EpiParams& ep, const unsigned* list, const unsigned* count, unsigned most, int n_cu,

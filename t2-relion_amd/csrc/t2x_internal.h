@@ -175,9 +175,9 @@ namespace cnn { struct Net; }
 
 // Pruned coarse pass (t2x_prune.hip): the INT8 bounds GEMM's operands (reference side made with the
 // coarse projections, image side per batch), its base table, block bounds, seeds and tile list;
-// cnt[0] counts the list, cnt[1] the particles for which the bounds can pay.
+// cnt[0] counts the list.
 struct PruneBufs {
-    DevBuf w, B8, sb, nb, A8, pa, pf, base, lbs, seed, list, cnt;
+    DevBuf w, B8, sb, nb, A8, pa, base, lbs, seed, list, cnt;
 };
 
 struct Device;

@@ -182,20 +182,21 @@ struct EpiParams {
 // Rows and columns of the tiles of the pruned coarse pass's full GEMM.
 #define PRUNED_TILE 128
 
-// One batch of the pruned coarse pass (t2x_prune.hip).
+// The pruned coarse pass of a batch, or of a sample of its particles (t2x_prune.hip).
 struct PruneCall {
-    int prec, B, T;
+    int prec, B, T;            // B particles, the batch's 0, stride, 2 stride, ..
+    int stride;
     long long M_pad, O_all, O_pad;
     int Kn;                    // columns of the N1 operands (pixels, padded); the GEMM's are 2 Kn
     int n_low, K8;             // pixels of the low set; bytes of an INT8 row (a multiple of 128)
-    int force;                 // take the bounds whether or not they look to pay (tests)
-    const double* Cb;          // [B] C_b
+    const double* Cb;          // the batch's C_b
 };
-// The reference side of the bounds (once per coarse projection), and a batch's bounds, seeds and list
-// of PRUNED_TILE tiles (in prune.list, prune.cnt[0] of them; both words of prune.cnt zero on entry). prune_bounds also
-// seeds the running minima pmin where the bounds are taken.
+// The reference side of the bounds (once per coarse projection and low set); bounds, seeds and the list of
+// PRUNED_TILE tiles (prune.list, prune.cnt[0] of them), which also seed the running minima pmin; and of the
+// same particles those that lose by the high set (prune.cnt[1]). prune.cnt is zero on entry to the bounds.
 int prune_prepare_refs(Device* d, long long O_all, long long O_pad, int Kc, int Kn, int n_low, int K8, hipStream_t st);
 int prune_bounds(Device* d, const PruneCall& c, const PartScalars* d_ps, const PassTables& tc, int Pw, hipStream_t st);
+int prune_high(Device* d, const PruneCall& c, const PartScalars* d_ps, const PassTables& tc, hipStream_t st);
 
 struct SelParams {
     double fraction;

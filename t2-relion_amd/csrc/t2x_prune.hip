@@ -152,46 +152,40 @@ __global__ __launch_bounds__(1024) void k_prune_quant_b(const float* __restrict_
     }
 }
 
-// Whether the bounds can pay, and the factors of sqrt(N1h) and sqrt(N1) (pf). An orientation that
-// matches the image poorly has a diff2 of the order of N1 above the minimum, a tile's best sample less,
-// and the bounds lose c0 sqrt(N1h) + c1 sqrt(N1) + the quantisation's ~2% of 2 sqrt(N1 Cl): counted are
-// the particles for which N1 less that, over 32 orientations on average, is above 150 (the cut is 61).
-// The pass is worth its cost when a quarter of the batch's are (prune_on): refine64 (SNR 0.05, 64^2)
-// has ~80 and prunes 0.2% of its tiles, class2d64 15% at ~90, class256 99% at ~400.
-// One workgroup per particle, one wave per orientation.
-__global__ __launch_bounds__(256) void k_prune_gate(const PartScalars* __restrict__ ps, const float* __restrict__ N1,
-                                                    long long ldn, const float* __restrict__ A1, long long lda1,
-                                                    const float* __restrict__ B2, long long ldb2, long long O_all,
-                                                    int n_low, int npix, const double* __restrict__ prior_o, int force,
-                                                    float2* __restrict__ pf, unsigned* __restrict__ count)
+// What a particle's bounds lose: the factors of sqrt(N1h) (the high set) and sqrt(N1) (the margin).
+// 2^-7: the BF16 rounding of N1h's operands and, in the high set, the full pass's own; 2^-9: the margin.
+__device__ __forceinline__ float2 prune_factors(const PartScalars& s)
 {
-    __shared__ float sv[4], sn[4];
-    const int b = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    // 2^-7: the BF16 rounding of N1h's operands and, in the high set, the full pass's own; 2^-9: the margin
-    const float ch = (float)fmax(ps[b].C_coarse - ps[b].C_low, 0.) * 1.00001f;
-    const float cl = (float)fmax(ps[b].C_low - ps[b].highres_Xi2 / 2., 0.) * 1.00001f;
-    const float c0 = 2.f * (1.f + 1.f / 128.f) * sqrtf(ch), c1 = 2.f / 512.f * sqrtf(cl);
-    float sum = 0.f, cnt = 0.f;
+    const float ch = (float)fmax(s.C_coarse - s.C_low, 0.) * 1.00001f;
+    const float cl = (float)fmax(s.C_low - s.highres_Xi2 / 2., 0.) * 1.00001f;
+    return make_float2(2.f * (1.f + 1.f / 128.f) * sqrtf(ch), 2.f / 512.f * sqrtf(cl));
+}
+
+// Particles whose bounds lose more than 10 (the cut is 61) by the high set, over 32 orientations on
+// average: a larger low set helps them. One workgroup per particle, one wave per orientation.
+__global__ __launch_bounds__(256) void k_prune_high(const PartScalars* __restrict__ ps, int stride,
+                                                    const float* __restrict__ A1, long long lda1,
+                                                    const float* __restrict__ B2, long long ldb2, long long O_all,
+                                                    int n_low, int npix, const double* __restrict__ prior_o,
+                                                    unsigned* __restrict__ count)
+{
+    __shared__ float sh[4], sn[4];
+    const long long b = (long long)blockIdx.x * stride;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const float c0 = prune_factors(ps[b]).x;
+    float high = 0.f, cnt = 0.f;
     for (int q = wave; q < 32; q += 4) {
         const long long n = (long long)((q + 0.5) * (double)O_all / 32.);
         if (n >= O_all || !(prior_o[n] > 0.)) continue;
         float h = 0.f;
         for (int p = n_low + lane; p < npix; p += 64) h += A1[b * lda1 + p] * B2[n * ldb2 + p];
-        h = wave_sum(h);
-        const float n1 = N1[b * ldn + n];
-        sum += n1 - c0 * sqrtf(fmaxf(h, 0.f)) - (c1 + 0.04f * sqrtf(cl)) * sqrtf(fmaxf(n1, 0.f));
+        high += c0 * sqrtf(fmaxf(wave_sum(h), 0.f));
         cnt += 1.f;
     }
-    if (lane == 0) { sv[wave] = sum; sn[wave] = cnt; }
+    if (lane == 0) { sh[wave] = high; sn[wave] = cnt; }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        const float s = sv[0] + sv[1] + sv[2] + sv[3], c = sn[0] + sn[1] + sn[2] + sn[3];
-        pf[b] = make_float2(c0, c1);
-        if (force || s > 150.f * c) atomicAdd(count, 1u);
-    }
+    if (threadIdx.x == 0 && sh[0] + sh[1] + sh[2] + sh[3] > 10.f * (sn[0] + sn[1] + sn[2] + sn[3])) atomicAdd(count, 1u);
 }
-
-__device__ __forceinline__ bool prune_on(const unsigned* gate, int B) { return *gate * 4u >= (unsigned)B; }
 
 // The images' side: one workgroup per particle, its T rows minv ctf X_t w in whole numbers with one
 // scale; pa[b] = (scale, largest |Aq| of its rows, largest |dA|, 0). The particle's weighted image
@@ -199,19 +193,19 @@ __device__ __forceinline__ bool prune_on(const unsigned* gate, int B) { return *
 __global__ __launch_bounds__(256) void k_prune_quant_a(const float2* __restrict__ Fimg, const float* __restrict__ Fctf,
                                                        int Pw, const int* __restrict__ win,
                                                        const float* __restrict__ minv, int npix,
-                                                       const PartScalars* __restrict__ ps,
+                                                       const PartScalars* __restrict__ ps, int stride,
                                                        const float2* __restrict__ ab, int T, int n_low, int K8,
-                                                       const float* __restrict__ w, const unsigned* __restrict__ gate,
-                                                       int B, signed char* __restrict__ q8, float4* __restrict__ pa)
+                                                       const float* __restrict__ w, signed char* __restrict__ q8,
+                                                       float4* __restrict__ pa)
 {
     extern __shared__ float2 y[];   // [n_low]
     __shared__ float red[4][2];
-    if (!prune_on(gate, B)) return;
     const int b = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const float* mv = minv + (size_t)ps[b].og * npix;
+    const size_t bs = (size_t)b * stride;
+    const float* mv = minv + (size_t)ps[bs].og * npix;
     float mx = 0.f;
     for (int p = threadIdx.x; p < n_low; p += 256) {
-        const size_t q = (size_t)b * Pw + win[p];
+        const size_t q = bs * Pw + win[p];
         const float2 x = Fimg[q];
         const float s = mv[p] * Fctf[q] * w[p];
         const float2 v = make_float2(s * x.x, s * x.y);
@@ -266,21 +260,20 @@ __device__ __forceinline__ float prune_base_value(float n1, float n1h, float2 pf
 // non-negative operands rounded to BF16 as they are staged in LDS (their 2^-8 is in c0). 128x128 tiles
 // of 4 waves, K step 32; bound by the N1 read and the table's write.
 #define PB_PAD 8
-__global__ __launch_bounds__(256) void k_prune_base(const float2* __restrict__ pf, int B,
+__global__ __launch_bounds__(256) void k_prune_base(const PartScalars* __restrict__ ps, int B, int stride,
                                                     const float* __restrict__ N1, long long ldn,
                                                     const float* __restrict__ A1, long long lda1,
                                                     const float* __restrict__ B2, long long ldb2, long long O_all,
                                                     int n_low, int Kn, const float4* __restrict__ pa,
                                                     const float* __restrict__ sb, const float2* __restrict__ nb,
                                                     const double* __restrict__ prior_o, int tiles_m,
-                                                    const unsigned* __restrict__ gate, int* __restrict__ base)
+                                                    int* __restrict__ base)
 {
     typedef Vec8<__bf16>::type v8;
     __shared__ __attribute__((aligned(16))) __bf16 As[128][32 + PB_PAD];
     __shared__ __attribute__((aligned(16))) __bf16 Bs[128][32 + PB_PAD];
     __shared__ float4 spa[128];
     __shared__ float2 spf[128];
-    if (!prune_on(gate, B)) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
     const int m0 = (int)(blockIdx.x % (unsigned)tiles_m) * 128;
@@ -291,11 +284,11 @@ __global__ __launch_bounds__(256) void k_prune_base(const float2* __restrict__ p
     if (tid < 128) {
         const int b = min(m0 + tid, B - 1);
         spa[tid] = pa[b];
-        spf[tid] = pf[b];
+        spf[tid] = prune_factors(ps[(long long)b * stride]);
     }
     // loader: thread -> (row tid / 2, 16 columns), one K step ahead; rows beyond B read the last particle's
     const int lrow = tid >> 1, lc = (tid & 1) * 16;
-    const float* ap = A1 + (long long)min(m0 + lrow, B - 1) * lda1 + lc;
+    const float* ap = A1 + (long long)min(m0 + lrow, B - 1) * stride * lda1 + lc;
     const float* bp = B2 + (n0 + lrow) * ldb2 + lc;
     const int kb = n_low & ~31;
     float a[16], b[16];
@@ -352,7 +345,7 @@ __global__ __launch_bounds__(256) void k_prune_base(const float2* __restrict__ p
 #pragma unroll
         for (int r = 0; r < 4; r++)
 #pragma unroll
-            for (int j = 0; j < 4; j++) n1[r][j] = N1[(long long)min(m0 + r0 + r, B - 1) * ldn + nl + j * 16];
+            for (int j = 0; j < 4; j++) n1[r][j] = N1[(long long)min(m0 + r0 + r, B - 1) * stride * ldn + nl + j * 16];
 #pragma unroll
         for (int r = 0; r < 4; r++) {
             const int bb = m0 + r0 + r;
@@ -413,7 +406,7 @@ struct BoundsParams {
     long long ldb;
     int* lbs;               // [tiles_m * 2][S][nblk]
     int nblk, S, nb_part;   // particles
-    const unsigned* gate;
+    int stride;             // particle b is the batch's particle b stride
 };
 
 // The INT8 bounds GEMM. lbs[h][z][blk]: over rows [128 h, 128 h + 128) of the z-th particle among them
@@ -437,7 +430,6 @@ __global__ __launch_bounds__(512, 2) void k_gemm_i8_bounds(BoundsParams p)
 {
     __shared__ __attribute__((aligned(16))) signed char s0[32768], s1[32768], s2[32768], s3[32768];
     __shared__ __attribute__((aligned(16))) int sbase[(SB ? SB : 1) * 8 * 256];
-    if (!prune_on(p.gate, p.nb_part)) return;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave & 1, wn = wave >> 1;
@@ -644,8 +636,8 @@ __global__ __launch_bounds__(256) void k_prune_seed(BoundsParams p, const float4
     __shared__ float sv[256];
     __shared__ int si[256];
     __shared__ float sd[64];
-    if (!prune_on(p.gate, p.nb_part)) return;
     const int b = blockIdx.x, tid = threadIdx.x, T = p.T, lane = tid & 63;
+    const long long bs = (long long)b * p.stride;   // in the batch
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int h0 = b * T >> 7, nh = ((b * T + T - 1) >> 7) - h0 + 1;
     const int nscan = (int)((N + 63) / 64);   // blocks with a valid column
@@ -708,7 +700,7 @@ __global__ __launch_bounds__(256) void k_prune_seed(BoundsParams p, const float4
                 }
         }
         reduce();
-        const int r = max(si[0], ra);
+        const long long r = max(si[0], ra) + (bs - b) * T;   // the batch's row
         for (int c0 = wave * 16; c0 < wave * 16 + 16; c0 += 4) {   // (rows beyond N are zero, in memory)
             const long long n0 = (long long)blk * 64 + c0;
             float acc[4];
@@ -719,7 +711,7 @@ __global__ __launch_bounds__(256) void k_prune_seed(BoundsParams p, const float4
                 float d = 3.0e38f;
                 if (nc < N && prior_o[nc] > 0.) {
                     const float v = dot * (As ? As[r] : 1.f) * (Bs ? Bs[nc] : 1.f);
-                    d = (float)(Cb[b] + (double)N1[(long long)b * ldn + nc] - (double)v);
+                    d = (float)(Cb[bs] + (double)N1[bs * ldn + nc] - (double)v);
                 }
                 sd[c0 + lane] = d;
             }
@@ -731,13 +723,12 @@ __global__ __launch_bounds__(256) void k_prune_seed(BoundsParams p, const float4
     if (tid == 0) {
         const float sdv = m < 3.0e38f ? m + 1.f + 1e-4f * fabsf(m) : __builtin_inff();
         seed[b] = sdv;
-        pmin[b] = float_to_ordered(sdv);
+        pmin[bs] = float_to_ordered(sdv);
     }
 }
 
 // The tiles of the full GEMM that have to be computed: those with a (particle, block) whose bound is
-// not more than the negligible-weight cut (60, plus 1 for rounding) above the particle's seed; all of
-// them where the bounds were not worth taking. Appended to list (indices tm * tiles_n + tn) in about
+// not more than the negligible-weight cut (60, plus 1 for rounding) above the particle's seed. Appended to list (indices tm * tiles_n + tn) in about
 // the order of the GEMM's tile walk (groups of 64 tile rows). One thread per tile.
 __global__ __launch_bounds__(256) void k_prune_plan(BoundsParams p, const float4* __restrict__ pa,
                                                     const float* __restrict__ sb, const double* __restrict__ Cb,
@@ -754,18 +745,16 @@ __global__ __launch_bounds__(256) void k_prune_plan(BoundsParams p, const float4
         const unsigned gs = min((unsigned)tiles_m - g * 64u, 64u);
         const int tm = (int)(g * 64u + r % gs), tn = (int)(r / gs);
         tile = (unsigned)tm * (unsigned)tiles_n + (unsigned)tn;
-        if (prune_on(p.gate, p.nb_part)) {
-            keep = false;
-            const int r0 = tm * 128, r1 = min(r0 + 128, p.M);
-            const int z0 = r0 / p.T, z1 = r0 < r1 ? (r1 - 1) / p.T : z0 - 1;
-            for (int z = z0; z <= z1 && !keep; z++) {
-                const double lim = (double)seed[z] + 61. - Cb[z];
-                const float sa = pa[z].x;
-                const int* v = p.lbs + ((long long)tm * p.S + (z - z0)) * p.nblk + tn * 2;
+        keep = false;
+        const int r0 = tm * 128, r1 = min(r0 + 128, p.M);
+        const int z0 = r0 / p.T, z1 = r0 < r1 ? (r1 - 1) / p.T : z0 - 1;
+        for (int z = z0; z <= z1 && !keep; z++) {
+            const double lim = (double)seed[z] + 61. - Cb[(long long)z * p.stride];
+            const float sa = pa[z].x;
+            const int* v = p.lbs + ((long long)tm * p.S + (z - z0)) * p.nblk + tn * 2;
 #pragma unroll
-                for (int k = 0; k < 2; k++)
-                    if (v[k] <= PB_LOW || !((double)v[k] * (double)prune_unit(sa, sb[tn * 2 + k]) > lim)) keep = true;
-            }
+            for (int k = 0; k < 2; k++)
+                if (v[k] <= PB_LOW || !((double)v[k] * (double)prune_unit(sa, sb[tn * 2 + k]) > lim)) keep = true;
         }
     }
     const unsigned long long mask = __ballot(keep);
@@ -799,6 +788,15 @@ int prune_prepare_refs(Device* d, long long O_all, long long O_pad, int Kc, int 
     return T2X_OK;
 }
 
+int prune_high(Device* d, const PruneCall& c, const PartScalars* d_ps, const PassTables& tc, hipStream_t st)
+{
+    k_prune_high<<<(unsigned)c.B, 256, 0, st>>>(d_ps, c.stride, d->A1.as<float>(), c.Kn, d->coarse_B2.as<float>(), c.Kn,
+                                               c.O_all, c.n_low, tc.npix, d->prior_o.as<double>(),
+                                               d->prune.cnt.as<unsigned>() + 1);
+    T2X_HIP(hipGetLastError());
+    return T2X_OK;
+}
+
 int prune_bounds(Device* d, const PruneCall& c, const PartScalars* d_ps, const PassTables& tc, int Pw, hipStream_t st)
 {
     PruneBufs& q = d->prune;
@@ -812,22 +810,17 @@ int prune_bounds(Device* d, const PruneCall& c, const PartScalars* d_ps, const P
     if ((long long)tm * tn > 0x3fffffffLL || c.M_pad > 0x7fffffffLL) { set_error("prune: grid too large"); return T2X_EINVAL; }
     T2X_TRY(q.A8.ensure((size_t)c.M_pad * c.K8));
     T2X_TRY(q.pa.ensure(sizeof(float4) * c.B));
-    T2X_TRY(q.pf.ensure(sizeof(float2) * c.B));
     T2X_TRY(q.base.ensure(sizeof(int) * c.B * c.O_pad));
     T2X_TRY(q.lbs.ensure(sizeof(int) * (c.M_pad / 128) * S * nblk));
     T2X_TRY(q.seed.ensure(sizeof(float) * c.B));
     float* w = q.w.as<float>();
-    unsigned* gate = q.cnt.as<unsigned>() + 1;
-    k_prune_gate<<<(unsigned)c.B, 256, 0, st>>>(d_ps, d->N1.as<float>(), c.O_pad, d->A1.as<float>(), c.Kn,
-                                               d->coarse_B2.as<float>(), c.Kn, c.O_all, c.n_low, tc.npix,
-                                               d->prior_o.as<double>(), c.force, q.pf.as<float2>(), gate);
     k_prune_quant_a<<<(unsigned)c.B, 256, sizeof(float2) * c.n_low, st>>>(
         d->Fimg_cur.as<float2>(), d->Fctf_cur.as<float>(), Pw, tc.d_win.as<int>(), tc.d_minv.as<float>(), tc.npix, d_ps,
-        d->ab_coarse.as<float2>(), c.T, c.n_low, c.K8, w, gate, c.B, q.A8.as<signed char>(), q.pa.as<float4>());
+        c.stride, d->ab_coarse.as<float2>(), c.T, c.n_low, c.K8, w, q.A8.as<signed char>(), q.pa.as<float4>());
     const int bm = (c.B + 127) / 128;
     k_prune_base<<<(unsigned)(bm * (c.O_pad / 128)), 256, 0, st>>>(
-        q.pf.as<float2>(), c.B, d->N1.as<float>(), c.O_pad, d->A1.as<float>(), c.Kn, d->coarse_B2.as<float>(), c.Kn, c.O_all,
-        c.n_low, c.Kn, q.pa.as<float4>(), q.sb.as<float>(), q.nb.as<float2>(), d->prior_o.as<double>(), bm, gate, q.base.as<int>());
+        d_ps, c.B, c.stride, d->N1.as<float>(), c.O_pad, d->A1.as<float>(), c.Kn, d->coarse_B2.as<float>(), c.Kn, c.O_all,
+        c.n_low, c.Kn, q.pa.as<float4>(), q.sb.as<float>(), q.nb.as<float2>(), d->prior_o.as<double>(), bm, q.base.as<int>());
     BoundsParams p{};
     p.A = q.A8.as<signed char>();
     p.B = q.B8.as<signed char>();
@@ -842,7 +835,7 @@ int prune_bounds(Device* d, const PruneCall& c, const PartScalars* d_ps, const P
     p.nblk = nblk;
     p.S = S;
     p.nb_part = c.B;
-    p.gate = gate;
+    p.stride = c.stride;
     const unsigned grid = (unsigned)std::min<long long>(d->n_cu, (long long)tm * tn);
     // particles a 256-row tile can hold: ceil(255 / T) + 1
     const int slots = (254 + c.T) / c.T + 1;

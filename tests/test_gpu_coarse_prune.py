@@ -64,22 +64,30 @@ def test_pruned_equals_exhaustive_class256(gpu_device, monkeypatch, prec):
     same(pr, ex)
 
 
-def test_pruned_equals_exhaustive_when_little_prunes(gpu_device, monkeypatch):
-    monkeypatch.setenv("T2X_BATCH", "8")
-    wl = H.Workload("refine64", n=24, K=2, seed_offset=82, precision=T.T2X_PREC_FP16X2)
-    ex, _ = run(wl, gpu_device, True)
+def test_call_that_does_not_prune_pays_for_a_sample(gpu_device):
+    """Thirty times the noise: nothing prunes, and the bounds are those of a sample of the batch alone."""
+    lib = T.load()
+    wl = H.Workload("refine64", n=160, seed_offset=82, precision=T.T2X_PREC_FP16X2, overrides=dict(healpix_order=3))
+    wl.sigma2 *= 30.0   # (the model points at it)
     pr, cnt = run(wl, gpu_device, False)
-    print(f"\n[prune] refine64: {cnt[0]:.0f} of {cnt[1]:.0f} tiles pruned")
+    st = T.Stats()
+    T.check(lib.t2x_stats_get(gpu_device, C.byref(st)))
+    ex, _ = run(wl, gpu_device, True)
+    print(f"\n[prune] refine64: {cnt[0]:.0f} of {cnt[1]:.0f} tiles pruned, {st.coarse_bound_flop:.3g} bound flops")
+    assert cnt[0] == 0 and 0 < cnt[1] <= 102 * 288 / 4   # a batch: 12,960 rows, 36,864 orientations
+    assert 0 < st.coarse_bound_flop <= st.coarse_diff2_flop / 4
     same(pr, ex)
 
 
 def test_pruned_small_prefix(gpu_device, monkeypatch):
+    """A first low set of a quarter of the pixels keeps too many tiles: the call takes every pixel."""
     monkeypatch.setenv("T2X_BATCH", "6")
-    monkeypatch.setenv("T2X_PRUNE_RADIUS", "0.5")   # a quarter of the pixels: weak bounds
+    monkeypatch.setenv("T2X_PRUNE_RADIUS", "0.5")
     wl = H.Workload("class256", n=12, seed_offset=83, precision=T.T2X_PREC_FP16X2)
     ex, _ = run(wl, gpu_device, True)
     pr, cnt = run(wl, gpu_device, False)
     print(f"\n[prune] class256, prefix radius 0.5: {cnt[0]:.0f} of {cnt[1]:.0f} tiles pruned")
+    assert cnt[0] > 0.9 * cnt[1] > 0
     same(pr, ex)
 
 
@@ -146,16 +154,16 @@ def test_long_list_runs_all_tiles(gpu_device, monkeypatch, prec):
     """A batch behind one that pruned, with a list too long for the listed GEMM: all tiles, by the
     256 x 256 kernel (258), with the exhaustive pass's results."""
     lib = T.load()
-    monkeypatch.setenv("T2X_BATCH", "24")
-    wl = H.Workload("refine64", n=48, seed_offset=88, precision=prec, snr=1.0, overrides=dict(healpix_order=3))
-    later = (np.arange(48) >= 24).astype(int)
-    wl.set_groups([wl.sigma2, 30.0 * wl.sigma2], group_of=np.zeros(48, int), optics_of=later)
+    monkeypatch.setenv("T2X_BATCH", "64")
+    wl = H.Workload("refine64", n=128, seed_offset=88, precision=prec, snr=1.0, overrides=dict(healpix_order=3))
+    later = (np.arange(128) >= 64).astype(int)
+    wl.set_groups([wl.sigma2, 30.0 * wl.sigma2], group_of=np.zeros(128, int), optics_of=later)
     pr, cnt = run(wl, gpu_device, False)
     st = T.Stats()
     T.check(lib.t2x_stats_get(gpu_device, C.byref(st)))
     ex, _ = run(wl, gpu_device, True)
-    tiles = 16 * 288
-    assert cnt[1] == 2 * tiles and 0.85 * tiles < cnt[0] < tiles
+    tiles = 41 * 288   # of a batch: 64 x 81 rows
+    assert cnt[1] == 2 * tiles and 0.65 * tiles < cnt[0] < tiles
     assert st.gemm_tile_used == 258
     same(pr, ex)
 
