@@ -3059,8 +3059,10 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
 
     for (int b0 = 0; b0 < n; b0 += Bmax) {
         const int B = std::min(Bmax, n - b0);
-        // (the first batch may find that it does not pay)
-        bool prune_batch = prune_call && (prune_force || gemm_ms(B) > 0.15);
+        // (the first batch may find that it does not pay; operands that the exhaustive FP16X2 GEMM refuses
+        // go to it)
+        const bool x2_wide = prec == T2X_PREC_FP16X2 && 2 * Kc * std::max(O_pad, round_up((long long)B * T, 256)) >= 1LL << 32;
+        bool prune_batch = prune_call && !x2_wide && (prune_force || gemm_ms(B) > 0.15);
         // the full GEMM's tiles that hold rows of B particles and orientations (for graph replays too)
         auto tiles_of = [&](int b) {
             const long long tile = PRUNED_TILE;

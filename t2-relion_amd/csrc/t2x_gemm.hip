@@ -1622,11 +1622,9 @@ int launch_gemm_pruned(int prec, const void* Ah, const void* Al, const float* As
                        hipStream_t st)
 {
     const bool fp32 = prec == T2X_PREC_FP32;
-    const long long lim = 1LL << 32;   // as the exhaustive FP16X2 GEMM, which the call's other batches may take
-    if (!fp32 && ((long long)Mrows_pad * lda * 2 >= lim || (long long)Nrows_pad * ldb * 2 >= lim)) {
-        set_error("gemm_pruned: operands beyond 4 GiB (32-bit offsets)");
-        return T2X_EINVAL;
-    }
+    // k_gemm_x3p addresses operands with 32-bit byte offsets: beyond them a list of any length is walked
+    const long long lim = 1LL << 32;
+    const bool off32 = (long long)Mrows_pad * lda * 2 < lim && (long long)Nrows_pad * ldb * 2 < lim;
     static_assert(PRUNED_TILE == GBM && PRUNED_TILE == GBN, "tile of k_gemm_tn and k_gemm_x3");
     if (K % (fp32 ? GBK : XK) != 0 || Mrows_pad % WBM != 0 || Nrows_pad % WBN != 0) {
         set_error("gemm_pruned: operands not padded to tile multiples");
@@ -1640,7 +1638,7 @@ int launch_gemm_pruned(int prec, const void* Ah, const void* Al, const float* As
     EpiParams el = ep;
     el.tile_list = list;
     el.tile_count = count;
-    el.tile_most = most;
+    el.tile_most = fp32 || !off32 ? 0xffffffffu : most;
     SplitOperand A{Ah, Al, As, lda}, B{Bh, Bl, Bs, ldb};
     if (fp32)
         k_gemm_tn<EPI_DIFF2, true><<<(unsigned)(4 * n_cu), 256, 0, st>>>((const float*)Ah, lda, (const float*)Bh, ldb, K,
@@ -1652,11 +1650,15 @@ int launch_gemm_pruned(int prec, const void* Ah, const void* Al, const float* As
     else
         k_gemm_x3<_Float16, EPI_DIFF2, 3, true><<<(unsigned)(3 * n_cu), 256, 0, st>>>(A, B, K, tm, tn, 0, el);
     const int wm = Mrows_pad / WBM, wn = Nrows_pad / WBN;
+    if (el.tile_most == 0xffffffffu) {
+        T2X_HIP(hipGetLastError());
+        return T2X_OK;
+    }
     if (prec == T2X_PREC_FP16X2)
         k_gemm_x3p<_Float16, EPI_DIFF2, 2, true><<<(unsigned)n_cu, 512, 0, st>>>(A, B, K, wm, wn, 32, el, nullptr);
     else if (prec == T2X_PREC_BF16X3)
         k_gemm_x3p<__bf16, EPI_DIFF2, 3, true><<<(unsigned)n_cu, 512, 0, st>>>(A, B, K, wm, wn, 32, el, nullptr);
-    else if (!fp32)
+    else
         k_gemm_x3p<_Float16, EPI_DIFF2, 3, true><<<(unsigned)n_cu, 512, 0, st>>>(A, B, K, wm, wn, 32, el, nullptr);
     T2X_HIP(hipGetLastError());
     return T2X_OK;

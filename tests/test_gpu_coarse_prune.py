@@ -168,6 +168,28 @@ def test_long_list_runs_all_tiles(gpu_device, monkeypatch, prec):
     same(pr, ex)
 
 
+@pytest.mark.parametrize("prec", [T.T2X_PREC_FP16X3, T.T2X_PREC_BF16X3, T.T2X_PREC_FP16X2])
+def test_operands_beyond_4_gib(gpu_device, prec):
+    """320 particles, 421 translations and 10,000 pixels: 5.4 GB of rows in each half. The three-product
+    precisions prune as they run exhaustively; FP16X2 refuses them either way."""
+    lib = T.load()
+    wl = H.Workload("class2d64", n=320, seed_offset=89, precision=prec, snr=1.0, current_size=160,
+                    overrides=dict(ori_size=160, particle_diameter=250.0, blob_radius=50.0, offset_range_px=11.5))
+    wl.cfg.adaptive_oversampling = 0
+    if prec == T.T2X_PREC_FP16X2:
+        for exhaustive in (True, False):
+            with pytest.raises(RuntimeError, match="4 GiB"):
+                run(wl, gpu_device, exhaustive)
+        return
+    pr, cnt = run(wl, gpu_device, False)
+    st = T.Stats()
+    T.check(lib.t2x_stats_get(gpu_device, C.byref(st)))
+    print(f"\n[prune] {st.P_coarse} pixels: {cnt[0]:.0f} of {cnt[1]:.0f} tiles pruned")
+    assert 320 * wl.info.nr_trans * 2 * st.P_coarse * 2 > 1 << 32 and cnt[0] > 0
+    ex, _ = run(wl, gpu_device, True)
+    same(pr, ex)
+
+
 @pytest.mark.parametrize("tile", ["259", "258"])
 def test_pruned_other_bounds_kernels(gpu_device, monkeypatch, tile):
     """The bounds GEMM as k_gemm_x2h<true> (128x256 tiles) or as k_gemm_x3p with one K chunk per
