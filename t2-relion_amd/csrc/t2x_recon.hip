@@ -281,9 +281,16 @@ struct Arena {
     size_t take(size_t n) { const size_t o = bytes; bytes += (n + 255) / 256 * 256; return o; }
 };
 
+// The end of a call, on every way out: its copies are over (a caller's page-locked arrays are read and
+// written by the device directly), and an arena that is too large to keep is given back.
 struct ArenaRelease {
     ReconWork& w;
-    ~ArenaRelease() { if (w.arena.bytes > kReconKeep) w.arena.release(); }
+    hipStream_t st;
+    ~ArenaRelease()
+    {
+        (void)hipStreamSynchronize(st);
+        if (w.arena.bytes > kReconKeep) w.arena.release();
+    }
 };
 
 // A piece of a transfer between the caller's pageable memory and the device.
@@ -446,6 +453,11 @@ static int reconstruct_run(Device* d, const t2x_recon_params* p, const double* d
     const size_t nr = (size_t)P * P * P;
     const size_t no = (size_t)g.ori * g.ori * g.ori;
     const int nshell_tau = g.ori / 2 + 1;
+    // the MAP shell index ROUND(|k|/pf) for |k|^2 < max_r2 stays below r_max + 1 <= ori/2 + 1
+    if (p->do_map && (long long)p->r_max + 1 > nshell_tau) {
+        set_error("t2x_reconstruct: r_max exceeds the tau2 spectrum (ori_size/2+1 shells)");
+        return T2X_EINVAL;
+    }
     ReconWork& rw = d->recon;
     if (recon_plan(rw, 0, (int)P, st) != T2X_OK) {
         set_error("t2x_reconstruct: hipFFT Z2D plan failed");
@@ -458,7 +470,7 @@ static int reconstruct_run(Device* d, const t2x_recon_params* p, const double* d
                  o_err = ar.take(sizeof(int)), o_W = ar.take(nw * 16), o_R = ar.take(nr * 8),
                  o_vol = ar.take(no * 8), o_bg = ar.take(kShellBlocks * 8), o_bw = ar.take(kShellBlocks * 8),
                  o_fft = ar.take(rw.plan_work[0]);
-    ArenaRelease release{rw};
+    ArenaRelease release{rw, st};
     T2X_TRY(rw.arena.ensure(ar.bytes));
     char* base = rw.arena.as<char>();
     auto at = [&](size_t o) { return reinterpret_cast<double*>(base + o); };
@@ -477,11 +489,6 @@ static int reconstruct_run(Device* d, const t2x_recon_params* p, const double* d
     if (p->do_map) T2X_HIP(hipMemcpyAsync(b_tau, tau2, (size_t)nshell_tau * 8, hipMemcpyHostToDevice, st));
     else T2X_HIP(hipMemsetAsync(b_tau, 0, (size_t)nshell_tau * 8, st));
     T2X_HIP(hipMemsetAsync(b_err, 0, sizeof(int), st));
-    // the MAP shell index ROUND(|k|/pf) for |k|^2 < max_r2 stays below r_max + 1 <= ori/2 + 1
-    if (p->do_map && (long long)p->r_max + 1 > nshell_tau) {
-        set_error("t2x_reconstruct: r_max exceeds the tau2 spectrum (ori_size/2+1 shells)");
-        return T2X_EINVAL;
-    }
 
     k_recon_weights<<<kShellBlocks, 256, 2 * sizeof(double) * g.r_max, st>>>(
         g, b_w, b_tau, b_Fw, b_ps, b_pc,
@@ -555,7 +562,7 @@ extern "C" int t2x_fsc(t2x_device* hdev, int n, const double* map1, const double
     const size_t o_r1 = ar.take(nr * 8), o_r2 = ar.take(nr * 8), o_c1 = ar.take(nc * 16), o_c2 = ar.take(nc * 16),
                  o_part = ar.take((size_t)kShellBlocks * 3 * xh * 8), o_out = ar.take((size_t)xh * 8),
                  o_fft = ar.take(rw.plan_work[1]);
-    ArenaRelease release{rw};
+    ArenaRelease release{rw, st};
     T2X_TRY(rw.arena.ensure(ar.bytes));
     char* base = rw.arena.as<char>();
     double *r1 = reinterpret_cast<double*>(base + o_r1), *r2 = reinterpret_cast<double*>(base + o_r2),
