@@ -81,6 +81,18 @@ def test_2d_and_one_pass(gpu_device, monkeypatch, prec):
     check(wl, gpu_device, monkeypatch)
 
 
+@pytest.mark.parametrize("prec", [FP32, FP16X3])
+def test_largest_low_set(gpu_device, monkeypatch, prec):
+    """One pass at current size 190: 14,000 pixels, of which the low set takes the most that its LDS row
+    holds (8,192), at 0.80 of the radius (9,000 pixels) as with every pixel asked for."""
+    wl = H.Workload("class2d64", n=6, K=3, seed_offset=98, precision=prec, snr=1.0, current_size=190,
+                    overrides=dict(ori_size=200, particle_diameter=300.0, blob_radius=60.0))
+    wl.cfg.adaptive_oversampling = 0
+    for radius in ("0.8", "1.5"):
+        monkeypatch.setenv("T2X_PRUNE_RADIUS", radius)
+        assert check(wl, gpu_device, monkeypatch)[0] > 0
+
+
 def test_zero_references(gpu_device, monkeypatch):
     """References of zeros: every bound is its particle's constant, nothing is dropped."""
     wl = H.Workload("refine64", n=4, seed_offset=96, precision=FP32)
