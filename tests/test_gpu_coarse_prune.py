@@ -1,20 +1,22 @@
 """The pruned coarse pass (t2x_estep_config.coarse_exhaustive 0) against the exhaustive one.
 
-The coarse diff2 of a sample is a sum of non-negative pixel terms (1/2 minv |ctf F - X_t|^2,
-plus a constant). A first GEMM over a prefix of the |frequency|-ordered coarse pixels (the low
-frequencies), with the rest bounded by Cauchy-Schwarz and a margin for the FP16 product it
-drops, gives each 64-column block's lower bound; per particle the full diff2 of its most promising block gives an upper bound of its
-minimum (the seed); the full GEMM then skips the tiles whose blocks all lie more than the
-negligible-weight cut (60, plus one for rounding) above the seed. Every skipped block is one the
-selection already treats as negligible (its minimum beyond the cut), so poses, dLL, the
-significant sets, the weighted sums and the backprojections are those of the exhaustive pass:
-identical, up to the run-to-run order of the store's atomic sums (weighted sums 1e-9,
+The coarse diff2 of a sample is a sum of non-negative pixel terms (1/2 minv |ctf F - X_t|^2, plus a
+constant). An INT8 GEMM over a low set of the |frequency|-ordered coarse pixels, with its quantisation
+errors and the rest of the pixels bounded by Cauchy-Schwarz, gives each 64-column block's lower bound; per
+particle the full diff2 of one row of its most promising block gives an upper bound of its minimum (the
+seed); the full GEMM then computes the tiles with a block not more than the negligible-weight cut (60,
+plus one for rounding) above the seed. Every skipped block is one the selection already treats as
+negligible, so poses, dLL, the significant sets, the weighted sums and the backprojections are those of
+the exhaustive pass: identical, up to the run-to-run order of the store's atomic sums (weighted sums 1e-9,
 backprojections 1e-6).
 
-Covered: the three split precisions at class256 shapes (where most tiles are pruned), a
-workload where few are (refine64: the pass turns itself off after a batch that prunes under
-40% of its tiles), a prefix radius forced small (T2X_PRUNE_RADIUS), ragged batches, the bounds
-GEMM in the full split precision and as each of its kernels, and graph replays.
+A call's first batch decides by a sample of its particles whether the pass is taken, and with which low
+set; a batch whose list is too long (35% of the tiles; 60% in FP32) runs all its tiles and turns the pass
+off for the rest of the call.
+
+Covered: the three split precisions at class256 shapes (where most tiles are pruned; FP32 in
+test_gpu_prune_bounds.py), a call that prunes nothing, a first low set that is too small, ragged batches,
+batches that stop pruning, graph replays, operands of 4 GiB and more.
 """
 import ctypes as C
 
@@ -88,19 +90,6 @@ def test_pruned_small_prefix(gpu_device, monkeypatch):
     pr, cnt = run(wl, gpu_device, False)
     print(f"\n[prune] class256, prefix radius 0.5: {cnt[0]:.0f} of {cnt[1]:.0f} tiles pruned")
     assert cnt[0] > 0.9 * cnt[1] > 0
-    same(pr, ex)
-
-
-def test_pruned_full_split_bounds(gpu_device, monkeypatch):
-    """The bounds pass in the full split precision (T2X_PRUNE_FULL_BOUNDS; the default under FP16
-    takes one product per element and allows for the dropped term)."""
-    monkeypatch.setenv("T2X_BATCH", "6")
-    monkeypatch.setenv("T2X_PRUNE_FULL_BOUNDS", "1")
-    wl = H.Workload("class256", n=12, seed_offset=84, precision=T.T2X_PREC_FP16X2)
-    ex, _ = run(wl, gpu_device, True)
-    pr, cnt = run(wl, gpu_device, False)
-    print(f"\n[prune] class256, full-split bounds: {cnt[0]:.0f} of {cnt[1]:.0f} tiles pruned")
-    assert cnt[0] > 0.5 * cnt[1]
     same(pr, ex)
 
 
@@ -187,18 +176,4 @@ def test_operands_beyond_4_gib(gpu_device, prec):
     print(f"\n[prune] {st.P_coarse} pixels: {cnt[0]:.0f} of {cnt[1]:.0f} tiles pruned")
     assert 320 * wl.info.nr_trans * 2 * st.P_coarse * 2 > 1 << 32 and cnt[0] > 0
     ex, _ = run(wl, gpu_device, True)
-    same(pr, ex)
-
-
-@pytest.mark.parametrize("tile", ["259", "258"])
-def test_pruned_other_bounds_kernels(gpu_device, monkeypatch, tile):
-    """The bounds GEMM as k_gemm_x2h<true> (128x256 tiles) or as k_gemm_x3p with one K chunk per
-    stage (the default takes two)."""
-    monkeypatch.setenv("T2X_BATCH", "6")
-    monkeypatch.setenv("T2X_BOUNDS_TILE", tile)
-    wl = H.Workload("class256", n=12, seed_offset=86, precision=T.T2X_PREC_FP16X2)
-    ex, _ = run(wl, gpu_device, True)
-    pr, cnt = run(wl, gpu_device, False)
-    print(f"\n[prune] class256, bounds tile {tile}: {cnt[0]:.0f} of {cnt[1]:.0f} tiles pruned")
-    assert cnt[0] > 0.5 * cnt[1]
     same(pr, ex)

@@ -4,7 +4,7 @@ pay, so that wrong bounds would drop tiles that matter).
 
 Edges: numbers of translations from 1 to 441 (the 8- and 24-particle base stages, the unstaged form,
 particles that end inside 16-row blocks, span row tiles, or fill one row each), ragged particle and
-orientation counts, prefixes of 16 pixels up to every pixel, references of very different power,
+orientation counts, low sets of 64 pixels up to every pixel, references of very different power,
 classes and directions that are not scored, one pass at the current size, 2D references, optics and
 image groups, each precision. Poses, dLL, significance and fine-sample counts are identical, weighted
 sums and backprojections within the order of the store's atomic sums (1e-9, 1e-6).
@@ -33,14 +33,25 @@ def check(wl, dev, monkeypatch):
     return cnt
 
 
+def three_poses(truth):
+    """Particles in three poses in turn: a tile of many particles is needed for three blocks at most, and
+    bounds that go to a neighbour drop it."""
+    n = len(truth["rot"])
+    for k in ("rot", "tilt", "psi"):
+        truth[k][:] = truth[k][np.arange(n) % 3].copy()
+    truth["x"][:] = 0
+    truth["y"][:] = 0
+
+
 @pytest.mark.parametrize("offsets,n", [((0.5, 1.0), 300), ((1.0, 1.0), 61), ((2.0, 1.0), 40), ((2.5, 1.0), 33),
                                        ((3.3, 1.0), 27), ((4.0, 1.0), 9), ((11.5, 1.0), 3)],
                          ids=lambda v: str(v))
 @pytest.mark.parametrize("prec", [FP32, FP16X2])
 def test_translations(gpu_device, monkeypatch, offsets, n, prec):
-    wl = H.Workload("refine64", n=n, seed_offset=91, precision=prec, snr=0.3,
+    wl = H.Workload("refine64", n=n, seed_offset=91, precision=prec, snr=3.0, truth_hook=three_poses,
                     overrides=dict(offset_range_px=offsets[0], offset_step_px=offsets[1]))
-    check(wl, gpu_device, monkeypatch)
+    cnt = check(wl, gpu_device, monkeypatch)
+    assert cnt[0] > 0.7 * cnt[1]
 
 
 @pytest.mark.parametrize("prec", [FP32, BF16X3, FP16X3, FP16X2])
@@ -48,14 +59,13 @@ def test_translations(gpu_device, monkeypatch, offsets, n, prec):
 def test_prefixes(gpu_device, monkeypatch, prec, radius):
     monkeypatch.setenv("T2X_PRUNE_RADIUS", radius)
     monkeypatch.setenv("T2X_BATCH", "7")
-    wl = H.Workload("refine64", n=17, K=3, seed_offset=92, precision=prec, snr=1.0)
+    wl = H.Workload("refine64", n=17, K=3, seed_offset=92, precision=prec, snr=1.0, overrides=dict(resolution=9.0))
     wl.ref_re[1] *= np.float32(1e-3)      # a class of hardly any power, and one with far too much
     wl.ref_im[1] *= np.float32(1e-3)
     wl.ref_re[2] *= np.float32(30)
     wl.ref_im[2] *= np.float32(30)
     cnt = check(wl, gpu_device, monkeypatch)
-    if radius == "1.5" and prec == FP16X3:
-        assert cnt[0] > 0
+    assert cnt[0] > 0.5 * cnt[1]   # two of the classes without any doubt
 
 
 @pytest.mark.parametrize("prec", [FP32, FP16X3])
@@ -68,17 +78,18 @@ def test_unscored_and_groups(gpu_device, monkeypatch, prec):
     s2 = wl.sigma2
     wl.set_groups([s2, 1.7 * s2], group_of=np.arange(12) % 3, optics_of=np.arange(12) % 2, scale=[0.8, 1.0, 1.3],
                   dvp=np.full((2, wl.N // 2 + 1), 10.0))
-    check(wl, gpu_device, monkeypatch)
+    assert check(wl, gpu_device, monkeypatch)[0] > 0
     wl.pdf_class[:] = [0.0, 1.0]
-    check(wl, gpu_device, monkeypatch)
+    assert check(wl, gpu_device, monkeypatch)[0] > 0
 
 
 @pytest.mark.parametrize("prec", [FP32, BF16X3])
 def test_2d_and_one_pass(gpu_device, monkeypatch, prec):
-    check(H.Workload("class2d64", n=37, K=5, seed_offset=94, precision=prec, snr=0.5), gpu_device, monkeypatch)
+    wl = H.Workload("class2d64", n=37, K=5, seed_offset=94, precision=prec, snr=0.5)
+    assert check(wl, gpu_device, monkeypatch)[0] > 0
     wl = H.Workload("refine64", n=5, seed_offset=95, precision=prec, snr=0.5)
     wl.cfg.adaptive_oversampling = 0
-    check(wl, gpu_device, monkeypatch)
+    assert check(wl, gpu_device, monkeypatch)[0] > 0
 
 
 @pytest.mark.parametrize("prec", [FP32, FP16X3])
@@ -94,11 +105,18 @@ def test_largest_low_set(gpu_device, monkeypatch, prec):
 
 
 def test_zero_references(gpu_device, monkeypatch):
-    """References of zeros: every bound is its particle's constant, nothing is dropped."""
+    """References of zeros: every bound is its particle's constant, nothing is dropped. (The weighted sums
+    run over every sample of the search in FP32 in no fixed order: two exhaustive runs differ by up to
+    1.5e-9, so the poses and counts alone are compared.)"""
+    monkeypatch.setenv("T2X_PRUNE_FORCE", "1")
     wl = H.Workload("refine64", n=4, seed_offset=96, precision=FP32)
     wl.ref_re[0][:] = 0
     wl.ref_im[0][:] = 0
-    check(wl, gpu_device, monkeypatch)
+    ex, _ = run(wl, gpu_device, True)
+    pr, cnt = run(wl, gpu_device, False)
+    assert cnt[0] == 0 < cnt[1]
+    for k in ("best_hidden", "dLL", "nr_significant_coarse", "nr_fine_samples"):
+        assert np.array_equal(pr["out"][k], ex["out"][k]), k
 
 
 def test_fp32_class256(gpu_device, monkeypatch):
