@@ -34,9 +34,8 @@ The headline value is the fastest path, per-iteration costs included, that keeps
 agreement with exhaustive search and the plain path's FSC-0.143 within 0.1 A (--headline pins
 one). The dominant kernel of the headline path is timed with HIP events on the library's stream;
 its roofline fraction counts the algorithmic 4*T*O*P_c flops (the MFMA-product utilisation of the
-split forms is reported beside it); for the pruned pass, the exhaustive pass's count over the
-pruned stage's time (an effective rate), with the work actually executed and its MFMA
-utilisation beside it. A quality phase reconstructs half-maps (first and second half
+split forms is reported beside it); for the pruned pass, the work that the pass executes, with the
+exhaustive pass's count over the pruned stage's time (an effective rate) beside it. A quality phase reconstructs half-maps (first and second half
 of all particles) of every class for each path on the GPU and reports the FSC-0.143 resolution
 per path; the pose agreement of each path with exhaustive search is reported per variant.
 
@@ -700,9 +699,9 @@ def main():
             "mfma_products_per_pair": nprod,
             "mfma_product_utilisation": nprod * achieved / peak}
     if pruned:
-        # the pruned pass computes part of the exhaustive pass's products for identical outputs:
-        # `achieved` stays the counting convention's (effective) rate; the work the MFMA units
-        # actually did is reported beside it
+        # the pruned pass computes part of the exhaustive pass's products for identical outputs: the
+        # roofline figures are those of the work it did, and the exhaustive pass's algorithmic flops
+        # over its time stand beside them as an effective rate
         f_kept = 1.0 - st.coarse_tiles_pruned / st.coarse_tiles_checked
         exec_pairs = (st.coarse_bound_flop + flop_total * f_kept) / launches
         # matrix-core time of the executed work at the dense peaks (INT8 bounds: 5 POP/s)
@@ -712,11 +711,15 @@ def main():
                        "over the low-frequency coarse pixels, block minima only) + k_prune_seed + k_prune_plan + "
                        + ("k_gemm_tn<LIST> (FP32" if hb == "fp32" else f"k_gemm_x3<LIST> ({nprod} products") +
                        ", persistent over the 128x128 tiles not beyond the negligible-weight cut)"),
-            "achieved_convention": ("effective: the exhaustive pass's algorithmic flops per batch over the pruned "
-                                    "stage's time per batch (same outputs)"),
+            "achieved": exec_pairs / (avg_ms * 1e-3) / 1e12 if avg_ms > 0 else 0.0,
+            "frac": exec_ms / avg_ms if avg_ms > 0 else 0.0,
+            "frac_convention": ("matrix-core time of the executed work (INT8 bounds at 5 POP/s, kept tiles at `peak`) over "
+                                "the stage's time"),
+            "effective_tflops": achieved,
+            "effective_convention": ("the exhaustive pass's algorithmic flops per batch over the pruned stage's time per "
+                                     "batch (same outputs; no fraction of a roofline)"),
             "tiles_pruned_fraction": 1.0 - f_kept,
             "executed_flop_per_launch": exec_pairs,
-            "executed_mfma_utilisation": exec_ms / avg_ms if avg_ms > 0 else 0.0,
         })
         del roof["mfma_product_utilisation"]
     configure(cfg, head)

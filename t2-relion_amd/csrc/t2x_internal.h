@@ -360,7 +360,7 @@ __host__ __device__ inline void inv3(const double* A, double* R)
 // line of 128 bytes each, cells x fastest. In x they overlap by one value (cell c holds x = 3c .. 3c + 3),
 // so that x and x + 1 always lie in one cell, 16 bytes to load. A trilinear sample then touches 2.25
 // lines on average and needs four loads, whatever the slice orientation; disjoint bricks of 4 x 4 x 4
-// (a third less memory) had it touch 3.1 in eight loads.
+// (a quarter less memory) had it touch 3.1 in eight loads.
 // Element (x, y, z) as the lower one of its pair; the copy in slot 3 of the cell before it, for x a
 // positive multiple of 3, is at vol_cell_index(x - 1, y, z) + 1.
 __host__ __device__ __forceinline__ size_t vol_cell_index(int x, int y, int z, int ncx, int ncy)

@@ -56,7 +56,7 @@ __device__ __forceinline__ float wave_max(float v)
     return v;
 }
 
-// Row weights of the low pixels: w = (mean |F|^2 over up to 4,096 orientations)^(1/4), at least
+// Row weights of the low pixels: w = (mean |F|^2 over 4,096 to 8,191 orientations, or all)^(1/4), at least
 // 1e-3 of the largest (any positive weights give valid bounds; these level the rows). The sums of
 // one of PP_PARTS parts of the orientations for 64 pixels a workgroup; k_prune_weights adds the parts
 // and turns them into w and 1 / w.
@@ -364,8 +364,10 @@ __global__ __launch_bounds__(256) void k_prune_base(const PartScalars* __restric
 }
 
 // Walk of the bounds GEMM's tiles: groups of 32 tile rows, inside them blocks of 32 x 8 tiles, of which
-// the 8 XCDs (workgroup index & 7) take an 8 x 4 part each (2.4 MB + 1.2 MB of operands at 1,152 bytes a
-// row: one L2), the next block of the group keeping the rows. Partial blocks are walked rows first.
+// the 8 XCDs (workgroup index & 7) take an 8 x 4 part each, the next block of the group keeping the rows.
+// A part's 8 + 4 operand tiles are 3 KB a byte of row: up to 1,300 bytes of row they fit one L2 (4 MB)
+// whole; longer rows are walked in step, 64 bytes at a time, so that what the parts' tiles share is in
+// the L2 together too. Measured at rows of 1,152 bytes only. Partial blocks are walked rows first.
 #define PW_ROWS 32
 #define PW_COLS 8
 __device__ __forceinline__ void bounds_tile(int t, int tiles_m, int tiles_n, int& tm, int& tn)
