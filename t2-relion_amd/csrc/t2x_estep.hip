@@ -3738,7 +3738,10 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
         long long cap = local_pairs ? std::max<long long>(npairs_c, 1) : (long long)B * kCandCap;
         const char* cap_env = getenv("T2X_PLAN_CAP");   // tests: a small capacity forces a second plan
         if (cap_env && atoll(cap_env) > 0) cap = atoll(cap_env);
-        else cap = std::max(cap, d->plan_cap);
+        else   // what the lists of earlier batches hold anyway
+            cap = std::max<long long>(cap, (long long)std::min({d->sig_pairs.bytes / sizeof(int2), d->sig_orient.bytes / sizeof(int),
+                                                                d->orient_pairs_off.bytes / sizeof(long long),
+                                                                d->fine_diff2.bytes / (sizeof(float) * nover)}));
         BatchPlan hplan{};
         std::vector<long long> pair_off(B + 1, 0);
         long long npairs = 0, nitems = 0;
@@ -4132,7 +4135,6 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
         // run the batch's fine pass and store again (the first run did no work)
         if (attempt > 0) { set_error("batch plan: work lists exceeded twice"); return T2X_EDEVICE; }
         cap = std::max(hplan.npairs, hplan.norients);
-        d->plan_cap = std::max(d->plan_cap, cap);
         }   // attempt
         npairs = hplan.npairs;
         nitems = hplan.nitems;

@@ -69,7 +69,8 @@ def test_pruned_equals_exhaustive_class256(gpu_device, monkeypatch, prec):
 def test_call_that_does_not_prune_pays_for_a_sample(gpu_device):
     """Thirty times the noise: nothing prunes, and the bounds are those of a sample of the batch alone."""
     lib = T.load()
-    wl = H.Workload("refine64", n=160, seed_offset=82, precision=T.T2X_PREC_FP16X2, overrides=dict(healpix_order=3))
+    wl = H.Workload("refine64", n=160, seed_offset=82, precision=T.T2X_PREC_FP16X2,
+                    maximum_significants=200, overrides=dict(healpix_order=3))
     wl.sigma2 *= 30.0   # (the model points at it)
     pr, cnt = run(wl, gpu_device, False)
     st = T.Stats()
@@ -118,7 +119,8 @@ def test_later_batches_that_do_not_prune(gpu_device, monkeypatch, prec):
     the last two, whose shape has not been tuned in the process, runs eagerly before it is captured."""
     lib = T.load()
     monkeypatch.setenv("T2X_BATCH", "24")
-    wl = H.Workload("refine64", n=120, seed_offset=87, precision=prec, snr=1.0, overrides=dict(healpix_order=3))
+    wl = H.Workload("refine64", n=120, seed_offset=87, precision=prec, snr=1.0,
+                    maximum_significants=200, overrides=dict(healpix_order=3))
     later = (np.arange(120) >= 48).astype(int)
     wl.set_groups([wl.sigma2, 30.0 * wl.sigma2], group_of=np.zeros(120, int), optics_of=later)
     tiles = 16 * 288   # of a batch: 24 x 81 rows and 36,864 orientations, 128 x 128
@@ -144,7 +146,8 @@ def test_long_list_runs_all_tiles(gpu_device, monkeypatch, prec):
     256 x 256 kernel (258), with the exhaustive pass's results."""
     lib = T.load()
     monkeypatch.setenv("T2X_BATCH", "64")
-    wl = H.Workload("refine64", n=128, seed_offset=88, precision=prec, snr=1.0, overrides=dict(healpix_order=3))
+    wl = H.Workload("refine64", n=128, seed_offset=88, precision=prec, snr=1.0,
+                    maximum_significants=200, overrides=dict(healpix_order=3))
     later = (np.arange(128) >= 64).astype(int)
     wl.set_groups([wl.sigma2, 30.0 * wl.sigma2], group_of=np.zeros(128, int), optics_of=later)
     pr, cnt = run(wl, gpu_device, False)

@@ -78,3 +78,18 @@ def test_local360_current_size_206(local360_cs206, gpu_device, prec):
     wl.cfg.precision = 0
     e_fine, e_dll = compare(wl, o, g, prec)
     print(f"local360 cs 206 precision {prec}: fine diff2 max rel {e_fine:.2e}, dLL {e_dll:.2e}")
+
+
+def test_after_a_call_with_long_lists(gpu_device):
+    """A call of 64 x 16 fine samples per significant pair after one with 120 million significant pairs (one
+    pass, noise alone) on the same handle: its lists are sized by its own batch."""
+    wl = H.Workload("refine64", n=40, seed_offset=5, overrides=dict(healpix_order=3))
+    wl.sigma2 *= 30.0
+    wl.cfg.adaptive_oversampling = 0
+    g = wl.run_gpu(dev=gpu_device)
+    assert g["out"]["nr_significant_coarse"].sum() > 100e6
+    wl = H.Workload("refine64", n=2, seed_offset=6, snr=0.5)
+    wl.cfg.adaptive_oversampling = 2
+    o = wl.run_oracle()
+    g = wl.run_gpu(dev=gpu_device)
+    compare(wl, o, g, 0, fine=False)
