@@ -3061,8 +3061,8 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
         const int B = std::min(Bmax, n - b0);
         // (the first batch may find that it does not pay; operands that the exhaustive FP16X2 GEMM refuses
         // go to it)
-        const bool x2_wide = prec == T2X_PREC_FP16X2 && 2 * Kc * std::max(O_pad, round_up((long long)B * T, 256)) >= 1LL << 32;
-        bool prune_batch = prune_call && !x2_wide && (prune_force || gemm_ms(B) > 0.15);
+        const bool wide = prec != T2X_PREC_FP32 && 2 * Kc * std::max(O_pad, round_up((long long)B * T, 256)) >= 1LL << 32;
+        bool prune_batch = prune_call && !(wide && prec == T2X_PREC_FP16X2) && (prune_force || gemm_ms(B) > 0.15);
         // the full GEMM's tiles that hold rows of B particles and orientations (for graph replays too)
         auto tiles_of = [&](int b) {
             const long long tile = PRUNED_TILE;
@@ -4141,7 +4141,7 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
         if (bp_bricks) stt.bp_brick_items += (double)std::min(nitems, bp_item_cap);
         if (prune_batch) {
             const bool short_list = hprune <= prune_most || prune_force;
-            if (short_list || prec == T2X_PREC_FP32)
+            if (short_list || prec == T2X_PREC_FP32 || wide)   // the list (launch_gemm_pruned)
                 stt.coarse_tiles_pruned += (double)prune_ntiles - (double)hprune;
             else {   // all tiles, by k_gemm_x3p
                 stt.gemm_tile_used = 258;
