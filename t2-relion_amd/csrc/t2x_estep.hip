@@ -3546,8 +3546,13 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
                 k_fill_u32<<<(unsigned)((B + 255) / 256), 256, 0, st>>>(d->pmin.as<unsigned>(), 0xFF800000u, B);  // +inf
                 ep.pmin = (dbg && dbg->n_debug > 0) ? nullptr : d->pmin.as<unsigned>();
                 // rows beyond the valid columns of the last tile keep +inf
-                k_fill_f32<<<(unsigned)((M_pad * rowmin_ld + 255) / 256), 256, 0, st>>>(d_rowmin.as<float>(), 3.0e38f,
-                                                                                        M_pad * rowmin_ld);
+                bool filled = false;
+                auto fill_minima = [&]() {
+                    if (!filled)
+                        k_fill_f32<<<(unsigned)((M_pad * rowmin_ld + 255) / 256), 256, 0, st>>>(d_rowmin.as<float>(), 3.0e38f,
+                                                                                                M_pad * rowmin_ld);
+                    filled = true;
+                };
                 if (prune_batch) {
                     T2X_TRY(d->prune.cnt.ensure(sizeof(unsigned) * 2));
                     // bounds, seeds and the list of the tiles to compute, for Bs particles of the batch
@@ -3571,10 +3576,14 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
                             stt.coarse_bound_flop += 4.0 * (double)T * (double)O_all * (double)n_low[k] * Bs;
                         return T2X_OK;
                     };
-                    unsigned h[2];
+                    // (the fill runs while the host waits for the counters)
+                    T2X_TRY(d->rb_host.ensure(sizeof(unsigned) * 2));
+                    const unsigned* h = d->rb_host.as<unsigned>();
                     auto counts = [&]() -> int {
-                        T2X_HIP(hipMemcpyAsync(h, d->prune.cnt.ptr, sizeof(h), hipMemcpyDeviceToHost, st));
-                        T2X_HIP(hipStreamSynchronize(st));
+                        T2X_HIP(hipMemcpyAsync(d->rb_host.ptr, d->prune.cnt.ptr, sizeof(unsigned) * 2, hipMemcpyDeviceToHost, st));
+                        T2X_HIP(hipEventRecord(d->ev[13], st));
+                        fill_minima();
+                        T2X_HIP(hipEventSynchronize(d->ev[13]));
                         return T2X_OK;
                     };
                     // The call's first batch (which is never captured) decides by a sample of its
@@ -3614,6 +3623,7 @@ extern "C" int t2x_estep(t2x_device* h, const t2x_estep_config* cfg, const t2x_m
                     }
                     if (prune_batch && !bounded) T2X_TRY(bounds(prune_set, B));
                 }
+                fill_minima();
                 if (prune_batch) {   // a tile that is not listed keeps +inf minima
                     const bool f32 = prec == T2X_PREC_FP32;
                     T2X_TRY(launch_gemm_pruned(prec, f32 ? d->A.ptr : d->Ah.ptr, d->Al.ptr, d->As.as<float>(), Kc,
